@@ -58,26 +58,31 @@ std::map<std::vector<long long>, BankEntry> g_banks;
 unsigned long long g_bank_clock = 0;
 long long g_bank_budget = 64LL << 30;
 
-std::vector<long long> bank_key(const Plan &p)
+// The whole rows' bank, or (width) the row sets'.
+std::vector<long long> bank_key(const Plan &p, bool width)
 {
-    std::vector<long long> k{p.device};
-    for (auto &H : p.harms) {
+    std::vector<long long> k{p.device, width};
+    for (auto &H : width ? p.sets : p.harms) {
         k.push_back(H.numharm);
         k.push_back(H.harmnum);
         k.push_back(H.zmax);
         k.push_back(H.wmax);
         k.push_back(H.fftlen);
+        k.push_back(H.nrows);
     }
     return k;
 }
 
-void release_bank(Plan *p)
+void release_banks(Plan *p)
 {
-    if (!p->d_bank) return;
     std::lock_guard<std::mutex> lk(g_bank_mu);
-    auto it = g_banks.find(bank_key(*p));
-    if (it != g_banks.end() && it->second.ptr == p->d_bank) it->second.refs--;
-    p->d_bank = nullptr;
+    for (bool width : {false, true}) {
+        float2 *&bank = width ? p->d_wbank : p->d_bank;
+        if (!bank) continue;
+        auto it = g_banks.find(bank_key(*p, width));
+        if (it != g_banks.end() && it->second.ptr == bank) it->second.refs--;
+        bank = nullptr;
+    }
 }
 
 void evict_banks_locked(long long incoming)
@@ -97,25 +102,26 @@ void evict_banks_locked(long long incoming)
     }
 }
 
-// The bank of this plan's shape: from the cache, or built on the GPU now.
-int acquire_bank(Plan *p, bool *built)
+// A bank of this plan's shape: from the cache, or built on the GPU now.
+int acquire_bank(Plan *p, bool width, bool *built)
 {
     std::lock_guard<std::mutex> lk(g_bank_mu);
-    const auto key = bank_key(*p);
+    const auto key = bank_key(*p, width);
     auto it = g_banks.find(key);
+    float2 *&bank = width ? p->d_wbank : p->d_bank;
     *built = false;
     if (it != g_banks.end()) {
         it->second.refs++;
         it->second.last_use = ++g_bank_clock;
-        p->d_bank = it->second.ptr;
+        bank = it->second.ptr;
         return 0;
     }
-    evict_banks_locked(p->g.bank_bytes);
     BankEntry e;
-    e.bytes = p->g.bank_bytes;
+    e.bytes = width ? p->wbank_bytes : p->bank_bytes;
+    evict_banks_locked(e.bytes);
     PZL_HIPCHK(hipMalloc(&e.ptr, e.bytes));
-    hipError_t err = pzl_launch_bank_build(p->d_harms, (int)p->harms.size(), p->g.numharm_kernels, p->max_fftlen,
-                                           e.ptr, p->st);
+    hipError_t err = pzl_launch_bank_build(width ? p->d_sets : p->d_harms, (int)(width ? p->sets : p->harms).size(),
+                                           p->g.numharm_kernels, p->max_fftlen, e.ptr, p->st);
     if (err == hipSuccess) err = hipStreamSynchronize(p->st);
     if (err != hipSuccess) {
         (void)hipFree(e.ptr);
@@ -124,9 +130,19 @@ int acquire_bank(Plan *p, bool *built)
     e.refs = 1;
     e.last_use = ++g_bank_clock;
     g_banks[key] = e;
-    p->d_bank = e.ptr;
+    bank = e.ptr;
     *built = true;
     return 0;
+}
+
+// The whole rows' bank of a plan whose default form reads the row sets' only.
+int need_whole_bank(Plan *p)
+{
+    if (p->d_bank) return 0;
+    bool built = false;
+    const int rc = acquire_bank(p, false, &built);
+    if (rc == 0) p->g.device_bytes += p->bank_bytes;
+    return rc;
 }
 
 // Batch size, hit-slot capacity and slot count of a plan (pzl_plan_create
@@ -135,8 +151,16 @@ struct PlanSizes {
     int B;
     long long hitcap;
     int nslots;
-    long long seg_stride;
+    long long seg_stride;      // whole rows' segments of one rstep ...
+    long long set_seg_stride;  // ... and the row sets'
+    long long wbank_bytes;
+    std::vector<PzlHarm> sets;  // rows by width (empty: the form does not hold this shape)
+    std::vector<int> set_rows;
 };
+
+// The group of rows by width: the last one.
+int width_group() { return pzl_corr_num_groups() - 1; }
+int width_has(int n) { return pzl_corr_group_has(width_group(), n); }
 
 PlanSizes plan_sizes(const PzlConfig &cfg, const PzlGeometry &g, const std::vector<PzlHarm> &harms)
 {
@@ -154,6 +178,15 @@ PlanSizes plan_sizes(const PzlConfig &cfg, const PzlGeometry &g, const std::vect
     z.nslots = (int)std::max<long long>(1, std::min<long long>(Plan::kSlots, nbatches));
     z.seg_stride = 0;
     for (auto &H : harms) z.seg_stride += H.fftlen / 2;
+    z.set_seg_stride = z.wbank_bytes = 0;
+    if (!compute_row_sets(harms, g.corr_uselen, width_has, &z.sets, &z.set_rows)) {
+        z.sets.clear();
+        z.set_rows.clear();
+    }
+    for (auto &S : z.sets) {
+        z.set_seg_stride += S.fftlen / 2;
+        z.wbank_bytes += (long long)sizeof(float2) * S.nrows * S.fftlen;
+    }
     return z;
 }
 
@@ -178,9 +211,12 @@ std::vector<long long> plan_arena_items(const PzlGeometry &g, const PlanSizes &z
     std::vector<long long> v{(long long)sizeof(PzlHarm) * nh, (long long)sizeof(int) * nh,
                              (long long)sizeof(double) * (g.nrsteps + 1), (long long)sizeof(uint16_t) * nh * F.numz,
                              (long long)sizeof(int) * nh * F.numw,
-                             (long long)sizeof(int) * F.numw * F.numz * std::max<long long>(nh - 1, 1)};
+                             (long long)sizeof(int) * F.numw * F.numz * std::max<long long>(nh - 1, 1),
+                             (long long)sizeof(PzlHarm) * (long long)z.sets.size(),
+                             (long long)sizeof(int) * (long long)z.sets.size(),
+                             (long long)sizeof(int) * (long long)z.set_rows.size()};
     for (int k = 0; k < Plan::kSets; k++) {
-        v.push_back((long long)sizeof(float2) * z.seg_stride * z.B);
+        v.push_back((long long)sizeof(float2) * std::max(z.seg_stride, z.set_seg_stride) * z.B);
         v.push_back((long long)sizeof(uint16_t) * z.B * nh * g.corr_uselen);
         v.push_back((long long)sizeof(PzlHrTab) * z.B * nh);
         v.push_back((long long)sizeof(float) * (g.plane_bytes_per_rstep / 4 * z.B + PZL_PLANE_SLACK));
@@ -204,12 +240,12 @@ long long arena_bytes(const std::vector<long long> &items)
     return t;
 }
 
-// HBM held by a plan whose spectrum was set from the host: kernel bank,
-// spectrum and arena.
+// HBM held by a plan whose spectrum was set from the host: the default form's
+// kernel bank, spectrum and arena.
 long long plan_device_bytes(const PzlGeometry &g, const PlanSizes &z, const std::vector<PzlHarm> &harms,
                             long long sort_temp)
 {
-    return g.bank_bytes + (long long)sizeof(float2) * g.numbins + arena_bytes(plan_arena_items(g, z, harms, sort_temp));
+    return (z.sets.empty() ? g.bank_bytes : z.wbank_bytes) + (long long)sizeof(float2) * g.numbins + arena_bytes(plan_arena_items(g, z, harms, sort_temp));
 }
 
 // hipMalloc of a plan-owned buffer, counted in p->dev_bytes
@@ -220,52 +256,13 @@ template <typename T> hipError_t plan_malloc(Plan *p, T **ptr, size_t bytes)
     return e;
 }
 
-// Correlation variants chosen by pzl_autotune, per (device, FFT length,
-// batch size, row counts of the class): later plans of the same shape use them.
-std::mutex g_tune_mu;
-std::map<std::vector<long long>, int> g_tuned;
-
-std::vector<long long> tune_key(const Plan &p, const SizeClass &c)
-{
-    std::vector<long long> k{p.device, c.fftlen, p.B};
-    for (int n : c.nrows) k.push_back(n);
-    return k;
-}
-
-int tuned_variant(const Plan &p, const SizeClass &c)
-{
-    std::lock_guard<std::mutex> lk(g_tune_mu);
-    auto it = g_tuned.find(tune_key(p, c));
-    return it == g_tuned.end() ? 0 : it->second;
-}
-
-// ... and the grouped launch (-1: one launch per length; g: the shorter
-// lengths in group g; g + ngroups: every length in group g), per (device,
-// batch size, every class's length and row counts).
-std::map<std::vector<long long>, int> g_tuned_group;
-
-std::vector<long long> group_key(const Plan &p)
-{
-    std::vector<long long> k{p.device, p.B};
-    for (auto &c : p.classes) {
-        k.push_back(-c.fftlen);
-        for (int n : c.nrows) k.push_back(n);
-    }
-    return k;
-}
-
-int tuned_group(const Plan &p)
-{
-    std::lock_guard<std::mutex> lk(g_tune_mu);
-    auto it = g_tuned_group.find(group_key(p));
-    return it == g_tuned_group.end() ? -1 : it->second;
-}
-
 // Whether group g holds every FFT length of the plan but the longest (all:
 // the longest too).
 bool group_covers(const Plan &p, int g, bool all)
 {
-    if (g < 0 || g >= pzl_corr_num_groups() || p.classes.size() < 2) return false;
+    if (g < 0 || g >= pzl_corr_num_groups()) return false;
+    if (g == width_group()) return all && !p.sets.empty();
+    if (p.classes.size() < 2) return false;
     int longest = 0;
     for (auto &c : p.classes) longest = std::max(longest, c.fftlen);
     for (auto &c : p.classes)
@@ -367,7 +364,7 @@ void free_plan(Plan *p)
     streams.erase(std::unique(streams.begin(), streams.end()), streams.end());
     for (hipStream_t s : streams)
         if (s) (void)hipStreamSynchronize(s);
-    release_bank(p);
+    release_banks(p);
     (void)hipFree(p->d_arena);
     (void)hipFree(p->d_fft_own);
     for (int k = 0; k < Plan::kSets; k++) {
@@ -444,17 +441,21 @@ struct Scope {
     }
 };
 
+// Rows by width is the launch form in use.
+bool by_width(const Plan &p) { return !p.sets.empty() && p.group_all && p.side_group == width_group(); }
+
 PzlCorrArgs corr_args(const Plan &p, const SizeClass &c, int nb, int set)
 {
+    const bool width = by_width(p);
     PzlCorrArgs ca{};
-    ca.harms = p.d_harms;
+    ca.harms = width ? p.d_sets : p.d_harms;
     ca.nh = (int)p.harms.size();
     ca.nb = nb;
     ca.class_harms = c.d_harms;
     ca.nclass = (int)c.harms.size();
     ca.segs = p.d_segs[set];
-    ca.seg_stride = p.seg_stride;
-    ca.bank = p.d_bank;
+    ca.seg_stride = width ? p.set_seg_stride : p.seg_stride;
+    ca.bank = width ? p.d_wbank : p.d_bank;
     ca.planes = p.d_planes[set];
     ca.plane_stride = p.plane_stride;
     ca.hr_tab = p.d_hr[set];
@@ -483,7 +484,10 @@ int launch_corr_part(Plan &p, long long r0, int nb, int set, Timers *tm, const l
     ba.file_lobin = p.g.lobin;
     ba.nph = p.cfg.nph;
     ba.segs = p.d_segs[set];
-    ba.seg_stride = p.seg_stride;
+    const bool width = by_width(p);
+    ba.seg_stride = width ? p.set_seg_stride : p.seg_stride;
+    ba.segs_of = width ? p.d_sets : p.d_harms;
+    ba.nseg = (int)(width ? p.sets : p.harms).size();
     ba.rinds = p.d_rinds[set];
     ba.hr_tab = p.d_hr[set];
     // the segments of a batch can run ahead on their own stream, beside the
@@ -509,23 +513,27 @@ int launch_corrs(Plan &p, int nb, int set, Timers *tm, bool seg_stream)
     // With the segments on their own stream, the shorter FFT lengths (small
     // grids that alone leave most of the chip idle) can follow them there and
     // run beside the longest length's correlation on the main stream.
-    const bool side = seg_stream && p.side_classes && p.classes.size() > 1;
+    const bool width = by_width(p);
+    const std::vector<SizeClass> &classes = width ? p.set_classes : p.classes;
+    const bool grouped = width || (p.side_group >= 0 && classes.size() > 1);
+    const bool all = grouped && p.group_all;
+    const bool side = seg_stream && p.side_classes && classes.size() > 1 && !all;
     size_t main_k = 0;
-    for (size_t k = 1; k < p.classes.size(); k++)
-        if (p.classes[k].fftlen > p.classes[main_k].fftlen) main_k = k;
-    const bool grouped = p.side_group >= 0 && p.classes.size() > 1;
+    for (size_t k = 1; k < classes.size(); k++)
+        if (classes[k].fftlen > classes[main_k].fftlen) main_k = k;
+    if (!width && !p.d_bank) return fail(PZL_ERR_ARG, "the kernel rows of this launch form are not built");
     if (grouped) {
         // the shorter lengths (with group_all: every length, on the main
         // stream) in one grouped launch, longest first
-        hipStream_t cs = side && !p.group_all ? ss : p.st;
+        hipStream_t cs = side ? ss : p.st;
         std::vector<PzlCorrArgs> args;
         std::vector<const PzlCorrArgs *> argp;
         std::vector<int> lens;
         std::vector<const int *> rows;
-        args.reserve(p.classes.size());
-        for (size_t k = 0; k < p.classes.size(); k++) {
-            if (k == main_k && !p.group_all) continue;
-            const SizeClass &c = p.classes[k];
+        args.reserve(classes.size());
+        for (size_t k = 0; k < classes.size(); k++) {
+            if (k == main_k && !all) continue;
+            const SizeClass &c = classes[k];
             args.push_back(corr_args(p, c, nb, set));
             lens.push_back(c.fftlen);
             rows.push_back(c.nrows.data());
@@ -534,9 +542,9 @@ int launch_corrs(Plan &p, int nb, int set, Timers *tm, bool seg_stream)
         Scope s(tm, 1, 0, cs);
         PZL_HIPCHK(pzl_launch_corr_group(p.side_group, (int)args.size(), lens.data(), argp.data(), rows.data(), cs));
     }
-    for (size_t k = 0; k < p.classes.size(); k++) {
-        if (grouped && (k != main_k || p.group_all)) continue;
-        const SizeClass &c = p.classes[k];
+    for (size_t k = 0; k < classes.size(); k++) {
+        if (grouped && (k != main_k || all)) continue;
+        const SizeClass &c = classes[k];
         hipStream_t cs = (side && k != main_k) ? ss : p.st;
         const PzlCorrArgs ca = corr_args(p, c, nb, set);
         Scope s(tm, 1, c.fftlen, cs);
@@ -1015,7 +1023,9 @@ int pzl_geometry_from_config(const PzlConfig *cfg, PzlGeometry *g)
     std::vector<PzlHarm> harms;
     int rc = compute_geometry(*cfg, *g, &harms, nullptr);
     if (rc) return rc;
-    g->device_bytes = plan_device_bytes(*g, plan_sizes(*cfg, *g, harms), harms, -1);
+    const PlanSizes z = plan_sizes(*cfg, *g, harms);
+    g->device_bytes = plan_device_bytes(*g, z, harms, -1);
+    if (!z.sets.empty()) g->bank_bytes = z.wbank_bytes;
     return 0;
 }
 
@@ -1113,13 +1123,26 @@ int pzl_plan_create(const PzlConfig *cfg, int device, void **plan_out)
         c.fftlen = it->first;
         c.harms = it->second;
         for (int h : c.harms) c.nrows.push_back(p->harms[h].nrows);
-        c.variant = tuned_variant(*p, c);
         p->classes.push_back(c);
     }
-    {
-        const int t = tuned_group(*p), ng = pzl_corr_num_groups();
-        p->side_group = t < 0 ? -1 : t % ng;
-        p->group_all = t >= ng;
+    // rows by width by default, one launch per length where it does not hold the shape
+    p->sets = sizes.sets;
+    p->set_rows = sizes.set_rows;
+    p->set_seg_stride = sizes.set_seg_stride;
+    p->bank_bytes = p->g.bank_bytes;
+    p->wbank_bytes = sizes.wbank_bytes;
+    if (!p->sets.empty()) {
+        p->side_group = width_group();
+        p->group_all = true;
+        cls.clear();
+        for (int k = 0; k < (int)p->sets.size(); k++) cls[p->sets[k].fftlen].push_back(k);
+        for (auto it = cls.rbegin(); it != cls.rend(); ++it) {
+            SizeClass c;
+            c.fftlen = it->first;
+            c.harms = it->second;
+            for (int k : c.harms) c.nrows.push_back(p->sets[k].nrows);
+            p->set_classes.push_back(c);
+        }
     }
     p->hitcap = sizes.hitcap;
     const long long maxkey = std::max<long long>(p->g.nrsteps, 1) * p->g.numharmstages * F.numw * F.numz *
@@ -1178,6 +1201,9 @@ int pzl_plan_create(const PzlConfig *cfg, int device, void **plan_out)
     p->d_zinds = (uint16_t *)carve();
     p->d_winds = (int *)carve();
     p->d_zoff = (int *)carve();
+    p->d_sets = (PzlHarm *)carve();
+    int *set_cls_idx = (int *)carve();
+    p->d_set_rows = (int *)carve();
     for (int k = 0; k < Plan::kSets; k++) {
         p->d_segs[k] = (float2 *)carve();
         p->d_rinds[k] = (uint16_t *)carve();
@@ -1199,6 +1225,20 @@ int pzl_plan_create(const PzlConfig *cfg, int device, void **plan_out)
         c.d_harms = cls_idx;
         PCHK(hipMemcpy(c.d_harms, c.harms.data(), sizeof(int) * c.harms.size(), hipMemcpyHostToDevice));
         cls_idx += c.harms.size();
+    }
+    if (!p->sets.empty()) {
+        const int *list = p->d_set_rows;
+        for (auto &S : p->sets) {
+            S.rowlist = list;
+            list += S.nrows;
+        }
+        PCHK(hipMemcpy(p->d_sets, p->sets.data(), sizeof(PzlHarm) * p->sets.size(), hipMemcpyHostToDevice));
+        PCHK(hipMemcpy(p->d_set_rows, p->set_rows.data(), sizeof(int) * p->set_rows.size(), hipMemcpyHostToDevice));
+        for (auto &c : p->set_classes) {
+            c.d_harms = set_cls_idx;
+            PCHK(hipMemcpy(c.d_harms, c.harms.data(), sizeof(int) * c.harms.size(), hipMemcpyHostToDevice));
+            set_cls_idx += c.harms.size();
+        }
     }
     if (!p->startr.empty())
         PCHK(hipMemcpy(p->d_startr, p->startr.data(), sizeof(double) * p->startr.size(), hipMemcpyHostToDevice));
@@ -1240,11 +1280,12 @@ int pzl_plan_create(const PzlConfig *cfg, int device, void **plan_out)
     // The kernel bank: built once per shape and kept resident.
     {
         bool built = false;
-        int brc = acquire_bank(p, &built);
+        int brc = acquire_bank(p, !p->sets.empty(), &built);
         if (brc) return cleanup(brc);
         p->bank_built = built;
     }
     p->g.device_bytes = plan_device_bytes(p->g, sizes, p->harms, (long long)p->sort_temp_bytes);
+    if (!p->sets.empty()) p->g.bank_bytes = p->wbank_bytes;
 #undef PCHK
     *plan_out = p;
     return 0;
@@ -1256,7 +1297,7 @@ int pzl_plan_device_bytes(void *plan, long long *held)
 {
     Plan *p = (Plan *)plan;
     if (!p || !held) return fail(PZL_ERR_ARG, "null argument");
-    *held = p->dev_bytes + (p->d_bank ? p->g.bank_bytes : 0);
+    *held = p->dev_bytes + (p->d_bank ? p->bank_bytes : 0) + (p->d_wbank ? p->wbank_bytes : 0);
     return 0;
 }
 
@@ -1443,7 +1484,8 @@ int pzl_search(void *plan, long long rstep_lo, long long rstep_hi, PzlCand *cand
         stats->nrsteps = rstep_hi - rstep_lo;
         stats->cells = (double)stats->nrsteps * p->g.corr_uselen * p->g.numz * std::max(p->g.numw, 1);
         double seg_bytes = 0;
-        for (auto &H : p->harms) seg_bytes += H.fftlen / 2 * 8.0;
+        const bool width = by_width(*p);
+        for (auto &H : width ? p->sets : p->harms) seg_bytes += H.fftlen / 2 * 8.0;
         const double planes = plane_alg_bytes(*p);
         stats->bytes_alg = stats->nrsteps * (planes + seg_bytes) + (double)p->g.bank_bytes;
         stats->bytes_alg_corr = stats->nrsteps * (planes / 2 + seg_bytes) + (double)p->g.bank_bytes;
@@ -1456,7 +1498,7 @@ int pzl_search(void *plan, long long rstep_lo, long long rstep_hi, PzlCand *cand
         stats->ms_corr_group *= scale;
         for (auto &kv : per_class) kv.second *= scale;
         for (auto &kv : per_class_n) kv.second = i;
-        const bool grouped = p->side_group >= 0 && p->classes.size() > 1;
+        const bool grouped = width || (p->side_group >= 0 && p->classes.size() > 1);
         stats->group_launches = grouped ? i : 0;
         stats->corr_launches = (long long)i * (grouped ? (p->group_all ? 1LL : 2LL) : (long long)p->classes.size());
         stats->graph_launches = (long long)std::llround(stats->graph_launches * scale);
@@ -1472,8 +1514,9 @@ int pzl_search(void *plan, long long rstep_lo, long long rstep_hi, PzlCand *cand
             // per rstep: its plane rows written + segments read; the kernel rows
             // once per search (they are re-read by every launch: class_bank_bytes)
             double per_rstep = 0, bank = 0, flops = 0;
-            for (int h : c.harms) {
-                const PzlHarm &H = p->harms[h];
+            // (by width: of the row sets of the class's harmonics)
+            for (const PzlHarm &H : width ? p->sets : p->harms) {
+                if (H.ref_fftlen != c.fftlen) continue;
                 const double n = H.fftlen;
                 per_rstep += (double)H.nrows * H.max_numrs * 4.0 + H.fftlen / 2 * 8.0;
                 bank += (double)H.nrows * H.fftlen * 8.0;
@@ -1517,42 +1560,6 @@ int pzl_autotune(void *plan, int reps, char *report, int report_len)
     PZL_HIPCHK(hipEventCreate(&e1));
     std::string rep;
     char line[256];
-    std::vector<std::pair<float, int>> lead_times;  // (ms, variant) of the longest FFT length
-    for (auto &c : p->classes) {
-        const PzlCorrArgs ca = corr_args(*p, c, nb, 0);
-        const int nv = pzl_corr_num_variants(c.fftlen);
-        int best = c.variant;
-        float best_ms = 1e30f;
-        for (int v = 0; v < nv; v++) {
-            hipError_t e = pzl_launch_corr(c.fftlen, v, &ca, c.nrows.data(), p->st);
-            if (e == hipSuccess) e = hipEventRecord(e0, p->st);
-            for (int k = 0; k < reps && e == hipSuccess; k++)
-                e = pzl_launch_corr(c.fftlen, v, &ca, c.nrows.data(), p->st);
-            if (e == hipSuccess) e = hipEventRecord(e1, p->st);
-            if (e == hipSuccess) e = hipEventSynchronize(e1);
-            float ms = 0;
-            if (e == hipSuccess) e = hipEventElapsedTime(&ms, e0, e1);
-            if (e != hipSuccess) {
-                (void)hipGetLastError();
-                snprintf(line, sizeof line, "fftlen %d variant %d (%s): failed: %s\n", c.fftlen, v,
-                         pzl_corr_variant_name(c.fftlen, v), hipGetErrorString(e));
-                rep += line;
-                continue;
-            }
-            ms /= reps;
-            snprintf(line, sizeof line, "fftlen %d variant %d (%s): %.4f ms\n", c.fftlen, v,
-                     pzl_corr_variant_name(c.fftlen, v), ms);
-            rep += line;
-            if (&c == &p->classes[0]) lead_times.emplace_back(ms, v);
-            if (ms < best_ms) {
-                best_ms = ms;
-                best = v;
-            }
-        }
-        c.variant = best;
-        std::lock_guard<std::mutex> lk(g_tune_mu);
-        g_tuned[tune_key(*p, c)] = best;
-    }
     // harmonic-sum workgroup order, on the planes the correlations just wrote
     std::vector<std::pair<float, int>> sum_times;  // (ms, form = order | rpt log2 << 1)
     {
@@ -1600,46 +1607,10 @@ int pzl_autotune(void *plan, int reps, char *report, int report_len)
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    // In the search the longest length's correlation shares the CUs with the
-    // harmonic sum and the shorter lengths: the variants of it within 8% of
-    // the fastest alone are timed on a band of the real pipeline (best of two
-    // searches of 8 batches), and the fastest there is kept.
-    std::sort(lead_times.begin(), lead_times.end());
+    // The harmonic-sum forms within 8% of the fastest alone are timed on a band
+    // of the real pipeline (best of two searches of 8 batches), where they share
+    // the CUs with the correlations, and the fastest there is kept
     const long long band = 8LL * p->B;
-    if (lead_times.size() >= 2 && nr >= band) {
-        SizeClass &c = p->classes[0];
-        const long long lo = (nr - band) / 2;
-        float best_ms = 1e30f;
-        int best = c.variant;
-        for (size_t i = 0; i < lead_times.size() && i < 5; i++) {
-            if (lead_times[i].first > 1.08f * lead_times[0].first) break;
-            c.variant = lead_times[i].second;
-            rc = drop_graphs(*p);  // captured graphs hold the variants of their capture
-            if (rc) return rc;
-            float ms = 1e30f;
-            for (int k = 0; k < 2; k++) {
-                long long n = 0;
-                const auto t0 = std::chrono::steady_clock::now();
-                rc = pzl_search(plan, lo, lo + band, nullptr, 0, &n, nullptr);
-                if (rc) return rc;
-                ms = std::min(ms, (float)std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() -
-                                                                                  t0).count());
-            }
-            snprintf(line, sizeof line, "fftlen %d variant %d in a search band of %lld rsteps: %.3f ms\n", c.fftlen,
-                     c.variant, band, ms);
-            rep += line;
-            if (ms < best_ms) {
-                best_ms = ms;
-                best = c.variant;
-            }
-        }
-        c.variant = best;
-        rc = drop_graphs(*p);
-        if (rc) return rc;
-        std::lock_guard<std::mutex> lk(g_tune_mu);
-        g_tuned[tune_key(*p, c)] = best;
-    }
-    // likewise the harmonic-sum forms within 8% of the fastest alone
     std::sort(sum_times.begin(), sum_times.end());
     if (sum_times.size() >= 2 && nr >= band && sum_times[1].first <= 1.08f * sum_times[0].first) {
         const long long lo = (nr - band) / 2;
@@ -1669,59 +1640,6 @@ int pzl_autotune(void *plan, int reps, char *report, int report_len)
         }
         p->sum_order = best_order;
         p->sum_rpt = best_rpt;
-    }
-    // every length in one grouped launch, the shorter lengths in one, or one
-    // launch per length: each form a group allows is timed on the same band
-    // (best of three searches), in that order (the last group first: the
-    // leanest), and a form replaces the one kept so far only when it is faster
-    // by more than 2% (the forms differ by about that much, and the choice
-    // should not follow the timing noise)
-    if (p->classes.size() >= 2 && nr >= band) {
-        const long long lo = (nr - band) / 2;
-        const int ng = pzl_corr_num_groups();
-        std::vector<int> forms;  // as g_tuned_group
-        for (int all = 1; all >= 0; all--)
-            for (int g = ng - 1; g >= 0; g--)
-                if (group_covers(*p, g, all != 0)) forms.push_back(g + all * ng);
-        forms.push_back(-1);
-        if (forms.size() > 1) {
-            float best_ms = 1e30f;
-            int best = forms[0];
-            for (int f : forms) {
-                p->side_group = f < 0 ? -1 : f % ng;
-                p->group_all = f >= ng;
-                rc = drop_graphs(*p);
-                if (rc) return rc;
-                float ms = 1e30f;
-                for (int k = 0; k < 3; k++) {
-                    long long n = 0;
-                    const auto t0 = std::chrono::steady_clock::now();
-                    rc = pzl_search(plan, lo, lo + band, nullptr, 0, &n, nullptr);
-                    if (rc) {
-                        p->side_group = -1;
-                        p->group_all = false;
-                        return rc;
-                    }
-                    ms = std::min(ms, (float)std::chrono::duration<double, std::milli>(
-                                          std::chrono::steady_clock::now() - t0)
-                                          .count());
-                }
-                snprintf(line, sizeof line, "%s%s in a search band of %lld rsteps: %.3f ms\n",
-                         f < 0 ? "one launch per FFT length" : (f >= ng ? "every length in " : "shorter lengths in "),
-                         f < 0 ? "" : pzl_corr_group_name(f % ng), band, ms);
-                rep += line;
-                if (ms < 0.98f * best_ms) {
-                    best_ms = ms;
-                    best = f;
-                }
-            }
-            p->side_group = best < 0 ? -1 : best % ng;
-            p->group_all = best >= ng;
-            rc = drop_graphs(*p);
-            if (rc) return rc;
-            std::lock_guard<std::mutex> lk(g_tune_mu);
-            g_tuned_group[group_key(*p)] = best;
-        }
     }
     // CU split (pzl_plan_set_cu_split): the harmonic sums on 3 or 2 CUs per
     // shader engine, the segments and correlations on every CU (keeping CUs
@@ -1969,6 +1887,7 @@ int pzl_plan_set_corr_group(void *plan, int group, int all)
     }
     if (group != p->side_group || (all != 0) != p->group_all) {
         int rc = drop_graphs(*p);
+        if (rc == 0 && !(all && group == width_group())) rc = need_whole_bank(p);
         if (rc) return rc;
     }
     p->side_group = group;
@@ -2018,11 +1937,16 @@ int pzl_plan_set_variant(void *plan, int fftlen, int variant)
         return fail(PZL_ERR_ARG, "FFT length %d has no variant %d", fftlen, variant);
     for (auto &c : p->classes)
         if (c.fftlen == fftlen) {
-            if (c.variant != variant) {
+            if (c.variant != variant || by_width(*p)) {
                 int rc = drop_graphs(*p);
+                if (rc == 0) rc = need_whole_bank(p);
                 if (rc) return rc;
             }
             c.variant = variant;
+            if (by_width(*p)) {
+                p->side_group = -1;
+                p->group_all = false;
+            }
             return 0;
         }
     return fail(PZL_ERR_ARG, "no FFT length %d in this plan", fftlen);
@@ -2078,11 +2002,12 @@ int pzl_get_kernel(void *plan, int idx, int row, float *out)
         return fail(PZL_ERR_ARG, "bad kernel index");
     const PzlHarm &H = p->harms[idx];
     PZL_HIPCHK(hipSetDevice(p->device));
+    const int brc = need_whole_bank(p);
+    if (brc) return brc;
     PZL_HIPCHK(hipMemcpy(out, p->d_bank + H.bank_off + (long long)row * H.fftlen, sizeof(float2) * H.fftlen,
                          hipMemcpyDeviceToHost));
-    // power-of-two rows are held as K / fftlen (an exact scale): undo it
-    if ((H.fftlen & (H.fftlen - 1)) == 0)
-        for (int k = 0; k < 2 * H.fftlen; k++) out[k] *= (float)H.fftlen;
+    // rows are held as K / fftlen: undo it
+    for (int k = 0; k < 2 * H.fftlen; k++) out[k] *= (float)H.fftlen;
     return 0;
 }
 

@@ -273,6 +273,7 @@ template <int R, int SIGN, typename C> PZL_FFT_HD void dftR(C *v)
     else if constexpr (R == 4) dft4<SIGN>(v);
     else if constexpr (R == 5) dft5<SIGN>(v);
     else if constexpr (R == 6) dft6<SIGN>(v);
+    else if constexpr (R == 7) dft_odd<7, SIGN>(v);
     else if constexpr (R == 8) dft8<SIGN>(v);
     else if constexpr (R == 10) dft_comp<2, 5, SIGN>(v);
     else if constexpr (R == 12) dft_comp<4, 3, SIGN>(v);
@@ -317,7 +318,8 @@ __device__ __forceinline__ void lds_fft_pass_f64(double2 *buf, int n, int Ns, in
             if constexpr (R == 2) dft2<SIGN>(v[b][0], v[b][1]);
             else if constexpr (R == 3) dft3<SIGN>(v[b]);
             else if constexpr (R == 4) dft4<SIGN>(v[b]);
-            else dft5<SIGN>(v[b]);
+            else if constexpr (R == 5) dft5<SIGN>(v[b]);
+            else dft_odd<7, SIGN>(v[b]);
             const int jm = j % Ns;
             const int idxD = (j / Ns) * Ns * R + jm;
 #pragma unroll
@@ -328,8 +330,8 @@ __device__ __forceinline__ void lds_fft_pass_f64(double2 *buf, int n, int Ns, in
 }
 
 // Block-cooperative double-precision Stockham FFT of n points held in LDS
-// (buf, n <= NMAX <= 4096), any n = 2^a 3^b 5^c, by NT threads: passes of
-// radix 4 while 4 divides what is left, then 2, 3, 5.  Used by the
+// (buf, n <= NMAX <= 4096), any n = 2^a 3^b 5^c 7^d, by NT threads: passes of
+// radix 4 while 4 divides what is left, then 2, 3, 5, 7.  Used by the
 // kernel-bank build and the segment transforms; a smaller NMAX holds fewer
 // butterflies per thread in registers.
 template <int SIGN, int NT, int NMAX = 4096>
@@ -348,9 +350,12 @@ __device__ __forceinline__ void lds_fft_f64(double2 *buf, int n, int tid)
         } else if (rem % 3 == 0) {
             lds_fft_pass_f64<SIGN, 3, NT, NMAX>(buf, n, Ns, tid);
             Ns *= 3;
-        } else {
+        } else if (rem % 5 == 0) {
             lds_fft_pass_f64<SIGN, 5, NT, NMAX>(buf, n, Ns, tid);
             Ns *= 5;
+        } else {
+            lds_fft_pass_f64<SIGN, 7, NT, NMAX>(buf, n, Ns, tid);
+            Ns *= 7;
         }
     }
 }

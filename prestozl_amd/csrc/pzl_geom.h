@@ -75,4 +75,10 @@ struct PzlHarm {
     long long bank_off;           // complex offset of this harmonic's kernels in the bank
     long long plane_off;          // float offset of this plane inside one rstep's planes
     long long seg_off;            // complex offset of this harmonic's segment inside one rstep
+    // A row set: the kernel rows of one harmonic that a shorter correlation
+    // length holds (compute_row_sets).  fftlen, halfwidth, nrows, bank_off and seg_off
+    // are then the set's own, the rest is the harmonic's.
+    int parent;                   // the harmonic's index (its own index where this is no row set)
+    int ref_fftlen, ref_halfwidth;  // the harmonic's fftlen and halfwidth: its median window
+    const int *rowlist;           // device: row of the harmonic of each row of the set; null: all, in order
 };

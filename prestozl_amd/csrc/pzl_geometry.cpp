@@ -152,6 +152,9 @@ int compute_geometry(const PzlConfig &c, PzlGeometry &g, std::vector<PzlHarm> *h
             H.bank_off = bank_off;
             H.plane_off = plane_off;
             H.seg_off = seg_off;
+            H.parent = (int)harms.size();
+            H.ref_fftlen = H.fftlen;
+            H.ref_halfwidth = H.halfwidth;
             bank_off += (long long)H.nrows * H.fftlen;
             plane_off += (long long)H.nrows * H.rs_stride;
             seg_off += H.fftlen / 2;
@@ -165,6 +168,57 @@ int compute_geometry(const PzlConfig &c, PzlGeometry &g, std::vector<PzlHarm> *h
     if (harms_out) *harms_out = harms;
     if (startr_out) *startr_out = startr;
     return 0;
+}
+
+// A row's correlation length.  The reference gives every row of a harmonic the
+// length of its widest kernel (calc_fftlen, accel_utils.c:137-149), but a
+// kernel of half-width khw (z, w near 0: a third of the widest) only reaches
+// 2 khw bins beyond each end of the wanted window, so a transform of numrs +
+// 4 khw points gives the same outputs without wrap-around.  At zmax 200, wmax
+// 300, 16 harmonics the points per rstep fall to 0.81 of the reference's
+// lengths (with the lengths of the last correlation group).
+bool compute_row_sets(const std::vector<PzlHarm> &harms, int corr_uselen, int (*has)(int n), std::vector<PzlHarm> *sets,
+                      std::vector<int> *rows)
+{
+    sets->clear();
+    rows->clear();
+    long long bank_off = 0, seg_off = 0;
+    for (const PzlHarm &H : harms) {
+        if (!has(H.fftlen)) return false;
+        std::vector<int> lens;  // held lengths up to the harmonic's own
+        for (int n = 2; n <= H.fftlen; n += 2)
+            if (has(n)) lens.push_back(n);
+        // the widest window any start gives this harmonic (pzl_harm_r): its ends
+        // round to half bins and then outwards to whole ones
+        const double span = (corr_uselen / 2 - PZL_DR) * H.hf + 0.5;
+        const int window = H.stage == 0 ? corr_uselen : std::max(H.max_numrs, 2 * ((int)floor(span + 1.0) + 1));
+        std::vector<std::vector<int>> by_len(lens.size());  // rows of each length
+        std::vector<int> widest(lens.size(), 0);
+        for (int row = 0; row < H.nrows; row++) {
+            const double z = -H.zmax + (row % H.numz) * PZL_DZ, w = -H.wmax + (row / H.numz) * PZL_DW;
+            const int khw = pzl_w_resp_halfwidth(z, w);
+            size_t k = lens.size() - 1;
+            if (khw <= H.halfwidth)
+                k = std::min<size_t>(k, std::lower_bound(lens.begin(), lens.end(), window + 4 * khw) - lens.begin());
+            by_len[k].push_back(row);
+            widest[k] = std::max(widest[k], khw);
+        }
+        for (size_t k = lens.size(); k-- > 0;) {
+            if (by_len[k].empty()) continue;
+            PzlHarm S = H;
+            S.fftlen = lens[k];
+            // the full length keeps the harmonic's own segment, whatever its rows reach
+            S.halfwidth = lens[k] == H.fftlen ? H.halfwidth : widest[k];
+            S.nrows = (int)by_len[k].size();
+            S.bank_off = bank_off;
+            S.seg_off = seg_off;
+            bank_off += (long long)S.nrows * S.fftlen;
+            seg_off += S.fftlen / 2;
+            rows->insert(rows->end(), by_len[k].begin(), by_len[k].end());
+            sets->push_back(S);
+        }
+    }
+    return true;
 }
 
 }  // namespace pzl

@@ -42,10 +42,13 @@ struct PzlBatchArgs {
     long long seg_stride;
     uint16_t *rinds;       // [nb][nh][corr_uselen]
     PzlHrTab *hr_tab;      // [nb][nh]
+    const PzlHarm *segs_of;  // the segments of one rstep: the harmonics, or their row sets in
+                             // the harmonics' order (each with a segment of its own) ...
+    int nseg;                // ... and how many
 };
 
 struct PzlCorrArgs {
-    const PzlHarm *harms;
+    const PzlHarm *harms;    // harmonics or row sets (class_harms counts in these)
     int nh, nb;
     const int *class_harms;  // harmonics of one FFT length
     int nclass;
@@ -106,7 +109,7 @@ const char *pzl_corr_variant_name(int n, int v);
 // Correlation of several FFT-length classes in one launch of group 'group':
 // class c has length fftlens[c], arguments *args[c] and host row counts
 // class_nrows[c]; a length the group does not hold, or one given twice, is an
-// error.
+// error.  The last group holds closely spaced lengths, for classes of row sets.
 hipError_t pzl_launch_corr_group(int group, int ncls, const int *fftlens, const PzlCorrArgs *const *args,
                                  const int *const *class_nrows, hipStream_t st);
 int pzl_corr_num_groups(void);

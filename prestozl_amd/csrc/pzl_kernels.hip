@@ -17,7 +17,7 @@
 
 #include <algorithm>
 #include <mutex>
-
+#include <vector>
 
 #include "pzl_fft.h"
 #include "pzl_kernels.h"
@@ -57,7 +57,8 @@ __global__ __launch_bounds__(BANK_NT) void k_bank_build(const PzlHarm *__restric
     const int h = find_harm(harms, nh, blockIdx.x, &row);
     if (h < 0) return;
     const PzlHarm H = harms[h];
-    const int wi = row / H.numz, zi = row % H.numz;
+    const int hrow = H.rowlist ? H.rowlist[row] : row;
+    const int wi = hrow / H.numz, zi = hrow % H.numz;
     const double z = (double)(-H.zmax + zi * PZL_DZ);
     const double w = (double)(-H.wmax + wi * PZL_DW);
     const int khw = pzl_w_resp_halfwidth(z, w);
@@ -79,10 +80,10 @@ __global__ __launch_bounds__(BANK_NT) void k_bank_build(const PzlHarm *__restric
     }
     __syncthreads();
     lds_fft_f64<-1, BANK_NT>(sbuf, fftlen, tid);
-    // For power-of-two lengths the bank holds K / fftlen: the correlation's
-    // 1 / fftlen^2 power normalisation then comes out of the product, exactly
-    // (a power-of-two scale commutes with every rounding on the way).
-    const double bscale = (fftlen & (fftlen - 1)) == 0 ? 1.0 / fftlen : 1.0;
+    // The bank holds K / fftlen (scaled in double, rounded once): the
+    // correlation's 1 / fftlen^2 power normalisation then comes out of the
+    // product.
+    const double bscale = 1.0 / fftlen;
     float2 *out = bank + H.bank_off + (long long)row * fftlen;
     for (int k = tid; k < fftlen; k += BANK_NT)
         out[k] = float2{(float)(sbuf[k].x * bscale), (float)(sbuf[k].y * bscale)};
@@ -146,19 +147,22 @@ __global__ __launch_bounds__(SEG_NT) void k_segments(PzlBatchArgs a)
 {
     extern __shared__ double2 sbuf[];  // fftlen/2 complex doubles, then keys
     const int tid = threadIdx.x;
-    const int b = blockIdx.x / a.nh, h = blockIdx.x % a.nh;
-    const PzlHarm H = a.harms[h];
+    const int b = blockIdx.x / a.nseg, sg = blockIdx.x % a.nseg;
+    const PzlHarm H = a.segs_of[sg];
+    const int h = H.parent;
+    const bool first = sg == 0 || a.segs_of[sg - 1].parent != h;  // writes the harmonic's r tables
     const long long rstep = (a.rstep0_dev ? *a.rstep0_dev : a.rstep0) + b;
     const double fullrlo = a.startr[rstep];
     const double fullrhi = fullrlo + a.rstep_bins - PZL_DR;
     const PzlHarmR hr = pzl_harm_r(H.hf, h == 0, fullrlo, fullrhi, a.corr_uselen);
-    const long long lobin = hr.rlo - H.halfwidth;
-    const int numdata = H.fftlen / PZL_NUMBETWEEN;
+    // the harmonic's own segment: what the median is taken over
+    const long long lobin = hr.rlo - H.ref_halfwidth;
+    const int numdata = H.ref_fftlen / PZL_NUMBETWEEN;
     int n2 = 1;
     while (n2 < numdata) n2 <<= 1;
     float *keys = (float *)(sbuf + numdata);
 
-    if (tid == 0) {
+    if (tid == 0 && first) {
         a.hr_tab[b * a.nh + h].rlo = hr.rlo;
         a.hr_tab[b * a.nh + h].numrs = hr.numrs;
     }
@@ -182,18 +186,40 @@ __global__ __launch_bounds__(SEG_NT) void k_segments(PzlBatchArgs a)
         // the lower median: element (n-1)/2 of the powers in ascending order
         norm = 1.0 / sqrt((double)seg_select(keys, n2, (unsigned)(numdata - 1) / 2, tid) / log(2.0));
     }
+    // A row set's segment is the part of the harmonic's from 'skip' on that its
+    // rows reach.  A value that is not finite anywhere in the harmonic's segment
+    // makes every power of the harmonic NaN, whichever part the row set reads.
+    __shared__ float wild;
+    if (tid == 0) wild = 0.0f;
+    const int ndata = H.fftlen / PZL_NUMBETWEEN, skip = H.ref_halfwidth - H.halfwidth;
+    constexpr int PER = (SEG_MAXDATA + SEG_NT - 1) / SEG_NT;
+    float2 xs[PER];
     __syncthreads();
-    for (int i = tid; i < numdata; i += SEG_NT) {
-        const double2 x = sbuf[i];
-        sbuf[i] = double2{(double)(float)(x.x * norm), (double)(float)(x.y * norm)};
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+        const int i = tid + q * SEG_NT;
+        if (i < numdata) {
+            const double2 x = sbuf[i];
+            xs[q] = float2{(float)(x.x * norm), (float)(x.y * norm)};
+            const float d = (xs[q].x - xs[q].x) + (xs[q].y - xs[q].y);  // 0, or NaN
+            if (d != 0.0f) wild = d;
+        }
     }
     __syncthreads();
-    // FFT of the fftlen-point spread array == numdata-point FFT, repeated
-    // (numdata = fftlen / 2 <= 2048)
-    lds_fft_f64<-1, SEG_NT, SEG_MAXDATA>(sbuf, numdata, tid);
+    const double nan0 = wild;
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+        const int i = tid + q * SEG_NT, k = i - skip;
+        if (i < numdata && k >= 0 && k < ndata) sbuf[k] = double2{(double)xs[q].x + nan0, (double)xs[q].y + nan0};
+        if (i < ndata && i + skip >= numdata) sbuf[i] = double2{nan0, nan0};  // beyond what the rows reach
+    }
+    __syncthreads();
+    // FFT of the fftlen-point spread array == ndata-point FFT, repeated
+    // (ndata = fftlen / 2 <= 2048)
+    lds_fft_f64<-1, SEG_NT, SEG_MAXDATA>(sbuf, ndata, tid);
     float2 *seg = a.segs + (long long)b * a.seg_stride + H.seg_off;
-    for (int k = tid; k < numdata; k += SEG_NT) seg[k] = float2{(float)sbuf[k].x, (float)sbuf[k].y};
-    if (h > 0) {
+    for (int k = tid; k < ndata; k += SEG_NT) seg[k] = float2{(float)sbuf[k].x, (float)sbuf[k].y};
+    if (h > 0 && first) {
         uint16_t *rinds = a.rinds + ((long long)b * a.nh + h) * a.corr_uselen;
         for (int ii = tid; ii < a.corr_uselen; ii += SEG_NT)
             rinds[ii] = (uint16_t)pzl_rind(H.hf, fullrlo, hr.rlo, ii);
@@ -271,7 +297,7 @@ template <int N, int NT, int G, bool PING, int SH, int PADSH, int... Rs> struct 
     template <int P> static __device__ __forceinline__ void where(int bf, int &g, int &j)
     {
         constexpr int NBP = N / CP::RAD[P];
-        g = bf / NBP;
+        g = G == 1 ? 0 : bf / NBP;
         j = bf - g * NBP;
     }
 
@@ -295,10 +321,12 @@ template <int N, int NT, int G, bool PING, int SH, int PADSH, int... Rs> struct 
         }
     }
 
-    // passes 1 .. NP-1 of one FFT set; 'src' holds the output of pass P-1
-    template <int P>
-    static __device__ __forceinline__ void pass(float2 *b0, float2 *b1, const float2 *tw, int tid, float *pbase,
-                                                long long rs_stride, int gvalid, int numrs, int offset, float norm)
+    // passes 1 .. NP-1 of one FFT set; 'src' holds the output of pass P-1.
+    // rows(i) is the plane row of this thread's i-th butterfly of the last
+    // pass, null where there is none.
+    template <int P, typename D>
+    static __device__ __forceinline__ void pass(float2 *b0, float2 *b1, const float2 *tw, int tid, const D &rows,
+                                                int numrs, int offset)
     {
         constexpr int R = CP::RAD[P], Ns = CP::ns(P), NBP = N / R;
         constexpr bool last = (P == NP - 1);
@@ -339,32 +367,31 @@ template <int N, int NT, int G, bool PING, int SH, int PADSH, int... Rs> struct 
                         if constexpr (Ns % (1 << PADSH) == 0) wp[r * lds_pad<PADSH>(Ns)] = v[i][r];
                         else dst[lds_pad<PADSH>(g * N + idxD + r * Ns)] = v[i][r];
                     }
-                } else if constexpr (NBP % 64 == 0) {
+                } else if constexpr (G == 1 || NBP % 64 == 0) {
                     // g is uniform in a wave: a buffer store whose range is the
                     // row's numrs powers drops the outputs outside the r window
                     // (negative offsets wrap to out of range) without branches
                     const int gu = __builtin_amdgcn_readfirstlane(g);
-                    const int row = gu >> SH, par = gu & ((1 << SH) - 1);
-                    const __amdgpu_buffer_rsrc_t rs =
-                        uniform_rsrc(pbase + row * rs_stride, row < gvalid ? numrs * 4 : 0);
+                    const int par = gu & ((1 << SH) - 1);
+                    float *const pl = rows(i);
+                    const __amdgpu_buffer_rsrc_t rs = uniform_rsrc(pl, pl ? numrs * 4 : 0);
 #pragma unroll
                     for (int r = 0; r < R; r++) {
                         // natural-order output index (of the row) minus offset
                         const int ro = ((j + r * NBP) << SH) + par - offset;
                         const float2 y = v[i][r];
-                        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint((y.x * y.x + y.y * y.y) * norm), rs,
+                        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y.x * y.x + y.y * y.y), rs,
                                                               ro * 4, 0, 0);
                     }
                 } else {
-                    const int row = g >> SH, par = g & ((1 << SH) - 1);
-                    if (row < gvalid) {
-                        float *pl = pbase + row * rs_stride;
+                    const int par = g & ((1 << SH) - 1);
+                    if (float *const pl = rows(i)) {
 #pragma unroll
                         for (int r = 0; r < R; r++) {
                             const int ro = ((j + r * NBP) << SH) + par - offset;
                             if (ro >= 0 && ro < numrs) {
                                 const float2 y = v[i][r];
-                                pl[ro] = (y.x * y.x + y.y * y.y) * norm;
+                                pl[ro] = y.x * y.x + y.y * y.y;
                             }
                         }
                     }
@@ -373,7 +400,7 @@ template <int N, int NT, int G, bool PING, int SH, int PADSH, int... Rs> struct 
         }
         if constexpr (!last) {
             __syncthreads();
-            pass<P + 1>(b0, b1, tw, tid, pbase, rs_stride, gvalid, numrs, offset, norm);
+            pass<P + 1>(b0, b1, tw, tid, rows, numrs, offset);
         }
     }
 };
@@ -423,10 +450,8 @@ __device__ __forceinline__ void corr_units(const PzlCorrArgs &a, long long u0, l
     constexpr int R0 = CP::RAD[0], NB0 = NF / R0;
     float2 *b0 = smem, *b1 = PING ? smem + CP::BUF : smem;
     const int tid = threadIdx.x;
-    // power normalisation 1 / N^2 (accel_utils.c:1234, 1278-1282); for power-of-two N
-    // the bank rows carry 1 / N each, so the powers need no further scaling
-    constexpr bool POW2 = (N & (N - 1)) == 0;
-    const float norm = POW2 ? 1.0f : (float)(1.0 / ((double)N * (double)N));
+    // (the power normalisation 1 / N^2, accel_utils.c:1234, 1278-1282, is in the
+    // bank's rows, which carry 1 / N each)
 
     // twiddles of this thread, from the variant's table ([TWN][NT], see k_corr_twiddles)
     float2 tw[CP::TWN > 0 ? CP::TWN : 1];
@@ -476,8 +501,9 @@ __device__ __forceinline__ void corr_units(const PzlCorrArgs &a, long long u0, l
             const int bf = tid + i * NT;
             int g, j;
             F::template where<0>(bf, g, j);
-            if constexpr (NB0 % 64 == 0 && CP::full(0)) {
-                // g is uniform in a wave: rows past the harmonic read as zeros
+            if constexpr (GF == 1 || (NB0 % 64 == 0 && CP::full(0))) {
+                // g is uniform in a wave: rows past the harmonic (and what a thread
+                // without a butterfly would read past the last row) read as zeros
                 const int gu = __builtin_amdgcn_readfirstlane(g);
                 const int row = gu >> SH;
                 const __amdgpu_buffer_rsrc_t rs =
@@ -530,7 +556,20 @@ __device__ __forceinline__ void corr_units(const PzlCorrArgs &a, long long u0, l
                     kv[i][r + HR] = cmul(csub(k1, k2), float2{et.c[r], et.s[r]});
                 }
         }
-        const int offset = 2 * H.halfwidth;
+        // the plane row of each of this thread's last-pass butterflies, -1: none
+        constexpr int PL = CP::NP - 1;
+        int prow[CP::per(PL)];
+#pragma unroll
+        for (int i = 0; i < CP::per(PL); i++) {
+            int g, j;
+            F::template where<PL>(tid + i * NT, g, j);
+            if constexpr (GF == 1 || NF / CP::RAD[PL] % 64 == 0) g = __builtin_amdgcn_readfirstlane(g);
+            const int row = row0 + (g >> SH);
+            prow[i] = -1;
+            if (row < nrows) prow[i] = H.rowlist ? H.rowlist[row] : row;
+            if constexpr (GF == 1 || NF / CP::RAD[PL] % 64 == 0) prow[i] = __builtin_amdgcn_readfirstlane(prow[i]);
+        }
+        const int offset = 2 * H.halfwidth, parent = __builtin_amdgcn_readfirstlane(H.parent);
         // segment values of the next rstep are loaded while this one is transformed;
         // without the split, the spread segment's period N/2 lets an even radix
         // read each value once
@@ -555,8 +594,8 @@ __device__ __forceinline__ void corr_units(const PzlCorrArgs &a, long long u0, l
         };
         load_seg(b_lo);
         for (int b = b_lo; b < b_hi; b++) {
-            const int numrs = __builtin_amdgcn_readfirstlane(a.hr_tab[b * a.nh + h].numrs);
-            float *pbase = a.planes + (long long)b * a.plane_stride + H.plane_off + (long long)row0 * H.rs_stride;
+            const int numrs = __builtin_amdgcn_readfirstlane(a.hr_tab[b * a.nh + parent].numrs);
+            float *pbase = a.planes + (long long)b * a.plane_stride + H.plane_off;
             float2 cur[CP::per(0)][NSV];
 #pragma unroll
             for (int i = 0; i < CP::per(0); i++)
@@ -606,7 +645,10 @@ __device__ __forceinline__ void corr_units(const PzlCorrArgs &a, long long u0, l
                 }
             }
             __syncthreads();
-            F::template pass<1>(b0, b1, tw, tid, pbase, H.rs_stride, nrows - row0, numrs, offset, norm);
+            const auto rows = [&](int i) {
+                return prow[i] >= 0 ? pbase + (long long)prow[i] * H.rs_stride : nullptr;
+            };
+            F::template pass<1>(b0, b1, tw, tid, rows, numrs, offset);
             // the next pass 0 overwrites b0: wait for this FFT's readers of b0
             if constexpr (!PING || (CP::NP % 2 == 0)) __syncthreads();
         }
@@ -664,20 +706,26 @@ template <int N_, int NT_, int G_, bool PING, int SH, int PADSH, int... Rs> stru
 // Waves a correlation launch aims for at least (two rounds of 4 waves per SIMD).
 constexpr long long kCorrWaves = 2 * 4 * 1024;
 
-// Work units of one class for a variant of NT threads and G rows per
-// workgroup: a class with few row groups (the short FFT lengths) splits the
-// batch's rsteps over several units, so that the launch still has about
-// kCorrWaves waves; its rows are then read once per block of rsteps instead
-// of once per batch.  Returns false when the units exceed 2^31 - 1.
-static bool corr_units_of(const PzlCorrArgs &a, const int *class_nrows, int NT, int G, PzlCorrArgs &out)
+// Row groups of a class for a variant of G rows per workgroup.
+static long long corr_rowunits(const PzlCorrArgs &a, const int *class_nrows, int G)
 {
-    long long rowunits = 0;
-    for (int c = 0; c < a.nclass; c++) rowunits += (class_nrows[c] + G - 1) / G;
+    long long n = 0;
+    for (int c = 0; c < a.nclass; c++) n += (class_nrows[c] + G - 1) / G;
+    return n;
+}
+
+// Work units of one class for a variant of G rows per workgroup, in a launch
+// whose row groups make 'waves' waves: a launch with few of them splits the
+// batch's rsteps over several units, so that it still has about kCorrWaves
+// waves; its rows are then read once per block of rsteps instead of once per
+// batch.  Returns false when the units exceed 2^31 - 1.
+static bool corr_units_of(const PzlCorrArgs &a, const int *class_nrows, long long waves, int G, PzlCorrArgs &out)
+{
+    const long long rowunits = corr_rowunits(a, class_nrows, G);
     out = a;
     out.total_items = 0;
     out.rb = out.nblk = 1;
     if (rowunits < 1 || a.nb < 1) return true;
-    const long long waves = rowunits * (NT / 64);
     const int nblk = (int)std::min<long long>(a.nb, std::max<long long>(1, (kCorrWaves + waves - 1) / waves));
     out.rb = (a.nb + nblk - 1) / nblk;
     out.nblk = (a.nb + out.rb - 1) / out.rb;
@@ -1143,7 +1191,7 @@ extern "C" hipError_t pzl_launch_segments(const PzlBatchArgs *a, int max_fftlen,
     int n2 = 1;
     while (n2 < numdata) n2 <<= 1;
     const size_t smem = (size_t)numdata * sizeof(double2) + (size_t)n2 * sizeof(float);
-    return pzl_launch((const void *)k_segments, dim3(a->nb * a->nh), dim3(SEG_NT), smem, st, *a);
+    return pzl_launch((const void *)k_segments, dim3(a->nb * a->nseg), dim3(SEG_NT), smem, st, *a);
 }
 
 // One correlation variant: kernel-row length N, NT threads, G rows per
@@ -1155,7 +1203,8 @@ static hipError_t launch_corr_t(const PzlCorrArgs *a, const int *class_nrows, hi
 {
     using V = CorrV<N, NT, G, PING, SH, PADSH, Rs...>;
     PzlCorrArgs a2;
-    if (!corr_units_of(*a, class_nrows, NT, G, a2)) return hipErrorInvalidValue;
+    if (!corr_units_of(*a, class_nrows, corr_rowunits(*a, class_nrows, G) * (NT / 64), G, a2))
+        return hipErrorInvalidValue;
     if (a2.total_items < 1) return hipSuccess;
     hipError_t e = V::table(st, &a2.twtab);
     if (e != hipSuccess) return e;
@@ -1174,21 +1223,22 @@ static hipError_t launch_corr_t(const PzlCorrArgs *a, const int *class_nrows, hi
 // code) and runs that unit.  The short lengths, which alone fill a small part
 // of the chip, then share one launch and its tail with the longer ones.
 
-#define PZL_CORR_GROUP_MAX 10
+#define PZL_CORR_GROUP_MAX 15
 
 struct PzlCorrGroupArgs {
     PzlCorrArgs c[PZL_CORR_GROUP_MAX];    // per member: its class (total_items 0: absent)
     long long begin[PZL_CORR_GROUP_MAX + 1];  // first workgroup of each member
 };
 
-template <int K, typename V, typename... Vs>
+template <int NT, int K, typename V, typename... Vs>
 __device__ __forceinline__ void group_unit(const PzlCorrGroupArgs &g, long long wg, float2 *sm)
 {
     if (wg < g.begin[K + 1]) {
-        V::unit(g.c[K], wg - g.begin[K], sm);
+        // a member of fewer threads ends its other waves (they then count for no barrier)
+        if (V::NT == NT || threadIdx.x < V::NT) V::unit(g.c[K], wg - g.begin[K], sm);
         return;
     }
-    if constexpr (sizeof...(Vs) > 0) group_unit<K + 1, Vs...>(g, wg, sm);
+    if constexpr (sizeof...(Vs) > 0) group_unit<NT, K + 1, Vs...>(g, wg, sm);
 }
 
 // WMIN: waves per SIMD the registers must allow (1: the compiler's choice)
@@ -1196,13 +1246,13 @@ template <int NT, int WMIN, typename... Vs>
 __global__ __launch_bounds__(NT, WMIN) void k_corr_group(PzlCorrGroupArgs g)
 {
     extern __shared__ float2 smem[];
-    group_unit<0, Vs...>(g, blockIdx.x, smem);
+    group_unit<NT, 0, Vs...>(g, blockIdx.x, smem);
 }
 
 template <int NT, int WMIN, typename... Vs> struct CorrGroup {
     static constexpr int M = sizeof...(Vs);
     static_assert(M <= PZL_CORR_GROUP_MAX, "too many members");
-    static_assert(((Vs::NT == NT) && ...), "members share the thread count");
+    static_assert(((Vs::NT <= NT && Vs::NT % 64 == 0) && ...), "a member takes whole waves of the group's threads");
     static constexpr int lens[M] = {Vs::N...};
     static int member(int n)
     {
@@ -1210,22 +1260,31 @@ template <int NT, int WMIN, typename... Vs> struct CorrGroup {
             if (lens[k] == n) return k;
         return -1;
     }
+    // waves of the row groups of members K..
+    template <int K, typename V, typename... Rest>
+    static long long waves_of(const int *cls, const PzlCorrArgs *const *args, const int *const *class_nrows)
+    {
+        long long w = 0;
+        if (cls[K] >= 0) w = corr_rowunits(*args[cls[K]], class_nrows[cls[K]], V::G) * (V::NT / 64);
+        if constexpr (sizeof...(Rest) > 0) w += waves_of<K + 1, Rest...>(cls, args, class_nrows);
+        return w;
+    }
     // members K..: their classes' units (cls[k] < 0: absent), in order
     template <int K, typename V, typename... Rest>
-    static hipError_t fill(PzlCorrGroupArgs &g, long long &acc, const int *cls, const PzlCorrArgs *const *args,
-                           const int *const *class_nrows, hipStream_t st)
+    static hipError_t fill(PzlCorrGroupArgs &g, long long &acc, long long waves, const int *cls,
+                           const PzlCorrArgs *const *args, const int *const *class_nrows, hipStream_t st)
     {
         g.begin[K] = acc;
         g.c[K] = PzlCorrArgs{};
         if (cls[K] >= 0) {
-            if (!corr_units_of(*args[cls[K]], class_nrows[cls[K]], NT, V::G, g.c[K])) return hipErrorInvalidValue;
+            if (!corr_units_of(*args[cls[K]], class_nrows[cls[K]], waves, V::G, g.c[K])) return hipErrorInvalidValue;
             if (g.c[K].total_items > 0) {
                 hipError_t e = V::table(st, &g.c[K].twtab);
                 if (e != hipSuccess) return e;
             }
             acc += g.c[K].total_items;
         }
-        if constexpr (sizeof...(Rest) > 0) return fill<K + 1, Rest...>(g, acc, cls, args, class_nrows, st);
+        if constexpr (sizeof...(Rest) > 0) return fill<K + 1, Rest...>(g, acc, waves, cls, args, class_nrows, st);
         return hipSuccess;
     }
     static hipError_t launch(int ncls, const int *fftlens, const PzlCorrArgs *const *args,
@@ -1240,7 +1299,8 @@ template <int NT, int WMIN, typename... Vs> struct CorrGroup {
         }
         PzlCorrGroupArgs g{};
         long long acc = 0;
-        hipError_t e = fill<0, Vs...>(g, acc, cls, args, class_nrows, st);
+        const long long waves = std::max<long long>(1, waves_of<0, Vs...>(cls, args, class_nrows));
+        hipError_t e = fill<0, Vs...>(g, acc, waves, cls, args, class_nrows, st);
         if (e != hipSuccess) return e;
         for (int k = M; k <= PZL_CORR_GROUP_MAX; k++) g.begin[k] = acc;
         if (acc < 1) return hipSuccess;
@@ -1270,6 +1330,55 @@ using CorrGroup256Lean =
               CorrV<256, 256, 8, true, 0, 4, 8, 8, 4>, CorrV<192, 256, 8, true, 0, 4, 8, 4, 6>,
               CorrV<128, 256, 16, true, 0, 4, 8, 4, 4>>;
 
+// The groups for rows sorted by width (pzl_launch_corr_group's last group):
+// every row takes the shortest of these lengths that holds its window and its
+// own kernel's width, so the lengths are closely spaced.  What bounds each is
+// FP32 issue (VALU 62-66% busy, LDS exchanges and barriers the rest), at about
+// the same time per point: measured alone on MI355X, 6144 rows x 8 rsteps, ns
+// per row and rstep, 2048: 3.9, 1792: 3.6, 1536: 3.0, 1280: 2.65, 1152: 2.2,
+// 1024: 1.9, 896: 1.7, 768: 1.3, 640: 1.05, 512: 0.83, 4096: 7.7, 3584: 7.0,
+// 3072: 6.5, 2560: 5.8.  Lengths between them (1920, 1728, 1680, 1600, 1440,
+// 1344, 3840, 2304) measured no faster than the next one here: their radices
+// need two butterflies per thread in most passes, which spill at 128 VGPRs.
+// One launch per group: the members of more than 2048 points want 512 threads
+// and twice the LDS, which would halve the others' workgroups per CU.
+using CorrGroupWidth =
+    CorrGroup<256, 4, CorrV<2048, 256, 1, true, 0, 5, 8, 8, 4, 8>, CorrV<1792, 256, 1, true, 0, 5, 8, 8, 4, 7>,
+              CorrV<1536, 192, 1, true, 0, 5, 8, 8, 3, 8>, CorrV<1280, 256, 1, true, 0, 5, 8, 4, 5, 8>,
+              CorrV<1152, 192, 1, true, 0, 5, 8, 4, 6, 6>, CorrV<1024, 256, 2, true, 0, 5, 8, 4, 4, 8>,
+              CorrV<896, 256, 2, true, 0, 5, 8, 4, 4, 7>, CorrV<768, 192, 2, true, 0, 5, 8, 8, 12>,
+              CorrV<640, 256, 3, true, 0, 5, 8, 8, 10>, CorrV<512, 256, 4, true, 0, 4, 8, 8, 8>,
+              CorrV<384, 256, 4, true, 0, 4, 8, 8, 6>, CorrV<320, 256, 4, true, 0, 5, 8, 8, 5>,
+              CorrV<256, 256, 8, true, 0, 4, 8, 8, 4>, CorrV<192, 256, 8, true, 0, 4, 8, 4, 6>,
+              CorrV<128, 256, 16, true, 0, 4, 8, 4, 4>>;
+using CorrGroupWidthLong =
+    CorrGroup<512, 4, CorrV<4096, 512, 1, true, 0, 5, 8, 8, 8, 8>, CorrV<3584, 512, 1, true, 0, 5, 8, 8, 8, 7>,
+              CorrV<3072, 512, 1, true, 0, 5, 8, 8, 6, 8>, CorrV<2560, 512, 1, true, 0, 5, 8, 8, 5, 8>>;
+
+static int width_group_has(int n) { return CorrGroupWidth::has(n) || CorrGroupWidthLong::has(n); }
+
+static hipError_t width_group_launch(int ncls, const int *fftlens, const PzlCorrArgs *const *args,
+                                     const int *const *class_nrows, hipStream_t st)
+{
+    for (int pass = 0; pass < 2; pass++) {  // the long lengths first
+        std::vector<int> lens;
+        std::vector<const PzlCorrArgs *> a;
+        std::vector<const int *> rows;
+        for (int c = 0; c < ncls; c++)
+            if ((CorrGroupWidthLong::has(fftlens[c]) != 0) == (pass == 0)) {
+                lens.push_back(fftlens[c]);
+                a.push_back(args[c]);
+                rows.push_back(class_nrows[c]);
+            }
+        if (lens.empty()) continue;
+        const int n = (int)lens.size();
+        const hipError_t e = pass == 0 ? CorrGroupWidthLong::launch(n, lens.data(), a.data(), rows.data(), st)
+                                       : CorrGroupWidth::launch(n, lens.data(), a.data(), rows.data(), st);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
 struct CorrGroupEntry {
     const char *name;
     hipError_t (*launch)(int, const int *, const PzlCorrArgs *const *, const int *const *, hipStream_t);
@@ -1281,6 +1390,8 @@ static const CorrGroupEntry g_corr_groups[] = {
      CorrGroup256::has},
     {"256t lean: 2048:1r 1280:1r 1024:2r 768:1r 512:4r 384:4r 256:8r 192:8r 128:16r", CorrGroup256Lean::launch,
      CorrGroup256Lean::has},
+    {"rows by width: 128 192 256 320 384 512 640 768 896 1024 1152 1280 1536 1792 2048 2560 3072 3584 4096",
+     width_group_launch, width_group_has},
 };
 static const int g_ncorr_groups = (int)(sizeof(g_corr_groups) / sizeof(g_corr_groups[0]));
 

@@ -36,12 +36,30 @@ struct SizeClass {
 int compute_geometry(const PzlConfig &c, PzlGeometry &g, std::vector<PzlHarm> *harms_out,
                      std::vector<double> *startr_out);
 
+// The harmonics' rows as sets by width: for every row the shortest length 'has'
+// holds that takes the window and the row's own kernel width, at most the
+// harmonic's own length.  Sets in the harmonics' order, longest first;
+// rows[] is the row lists, set after set (PzlHarm.rowlist is left null).
+// Returns false when a harmonic's own length is not held.
+bool compute_row_sets(const std::vector<PzlHarm> &harms, int corr_uselen, int (*has)(int n), std::vector<PzlHarm> *sets,
+                      std::vector<int> *rows);
+
 struct Plan {
     PzlConfig cfg{};
     PzlGeometry g{};
     std::vector<PzlHarm> harms;
     std::vector<double> startr;
     std::vector<SizeClass> classes;
+    // Rows by width (the last correlation group): each harmonic's kernel rows
+    // split into row sets by the shortest length that holds their own width.
+    // This form, its bank and its segments are the default; the whole rows'
+    // bank is built when another form is first asked for.
+    std::vector<PzlHarm> sets;         // in the harmonics' order
+    std::vector<int> set_rows;         // the sets' rows (PzlHarm.rowlist), set after set
+    std::vector<SizeClass> set_classes;
+    PzlHarm *d_sets = nullptr;
+    int *d_set_rows = nullptr;
+    long long set_seg_stride = 0;
     std::vector<uint16_t> zinds;  // [nh][numz]
     std::vector<int> winds;       // [nh][numw]
     int fnumw = 1, fnumz = 1, fzlo = 0, fwlo = 0;
@@ -72,7 +90,10 @@ struct Plan {
     std::vector<MaskedStream> masked;
     // resident
     PzlHarm *d_harms = nullptr;
-    float2 *d_bank = nullptr;  // shared, owned by the bank cache
+    // kernel banks, shared, owned by the bank cache
+    float2 *d_bank = nullptr;   // whole rows (null until a form that reads them is chosen)
+    float2 *d_wbank = nullptr;  // the row sets'
+    long long bank_bytes = 0, wbank_bytes = 0;
     bool bank_built = false;   // this plan's creation built the bank
     double *d_startr = nullptr;
     double numindep_d[6] = {0, 0, 0, 0, 0, 0};
