@@ -430,6 +430,15 @@ template <int R> struct ExpTab {
     }
 };
 
+// The tables that no kernel of a batch writes, and the r table that the
+// batch's segments wrote before: read through the constant address space, so
+// that uniform reads are scalar loads.  As vector loads they cost the rstep
+// loop three dependent memory latencies and, the loop's stores counting with
+// the loads, a wait for the previous rstep's stores.
+typedef const __attribute__((address_space(4))) PzlHarm pzl_const_harm;
+typedef const __attribute__((address_space(4))) int pzl_const_int;
+typedef const __attribute__((address_space(4))) PzlHrTab pzl_const_hr;
+
 // N: kernel-row (correlation) length, G: kernel rows per workgroup, SH: 1 to
 // transform each row as two N/2-point FFTs.  Because the segment spectrum
 // repeats with period N/2, y[2m + e] = sum_{k<N/2} P_e[k] exp(2 pi i k m/(N/2))
@@ -474,12 +483,14 @@ __device__ __forceinline__ void corr_units(const PzlCorrArgs &a, long long u0, l
         // the unit's rows (per harmonic of the class, ceil(nrows / G) row groups) and
         // its block of rsteps: the blocks of one row group are adjacent units
         const int ru = (int)(unit / a.nblk), blk = (int)(unit - (long long)ru * a.nblk);
+        const pzl_const_harm *const harms = (const pzl_const_harm *)a.harms;
         int h = -1, row0 = 0;
         {
+            const pzl_const_int *const class_harms = (const pzl_const_int *)a.class_harms;
             int acc = 0;
             for (int c = 0; c < a.nclass; c++) {
-                const int hh = a.class_harms[c];
-                const int cnt = (a.harms[hh].nrows + G - 1) / G;
+                const int hh = class_harms[c];
+                const int cnt = (harms[hh].nrows + G - 1) / G;
                 if (ru < acc + cnt) {
                     h = hh;
                     row0 = (ru - acc) * G;
@@ -492,8 +503,8 @@ __device__ __forceinline__ void corr_units(const PzlCorrArgs &a, long long u0, l
         const int b_hi = __builtin_amdgcn_readfirstlane(min(a.nb, b_lo + a.rb));
         h = __builtin_amdgcn_readfirstlane(h);
         row0 = __builtin_amdgcn_readfirstlane(row0);
-        const PzlHarm &H = a.harms[h];
-        const int nrows = __builtin_amdgcn_readfirstlane(H.nrows);
+        const pzl_const_harm &H = harms[h];
+        const int nrows = H.nrows;
         // the kernel rows (conjugated in the product below), at the positions pass 0 reads them
         float2 kv[CP::per(0)][R0];
 #pragma unroll
@@ -509,8 +520,8 @@ __device__ __forceinline__ void corr_units(const PzlCorrArgs &a, long long u0, l
                 const __amdgpu_buffer_rsrc_t rs =
                     uniform_rsrc(a.bank + H.bank_off + (long long)(row0 + row) * N, row0 + row < nrows ? N * 8 : 0);
                 auto ld = [&](int k) {
-                    return float2{__uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, k * 8, 0, 0)),
-                                  __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, k * 8 + 4, 0, 0))};
+                    const auto v = __builtin_amdgcn_raw_buffer_load_b64(rs, k * 8, 0, 0);
+                    return float2{__uint_as_float(v[0]), __uint_as_float(v[1])};
                 };
                 if constexpr (SH == 0) {
 #pragma unroll
@@ -566,10 +577,14 @@ __device__ __forceinline__ void corr_units(const PzlCorrArgs &a, long long u0, l
             if constexpr (GF == 1 || NF / CP::RAD[PL] % 64 == 0) g = __builtin_amdgcn_readfirstlane(g);
             const int row = row0 + (g >> SH);
             prow[i] = -1;
-            if (row < nrows) prow[i] = H.rowlist ? H.rowlist[row] : row;
+            if (row < nrows) prow[i] = H.rowlist ? ((const pzl_const_int *)H.rowlist)[row] : row;
             if constexpr (GF == 1 || NF / CP::RAD[PL] % 64 == 0) prow[i] = __builtin_amdgcn_readfirstlane(prow[i]);
         }
-        const int offset = 2 * H.halfwidth, parent = __builtin_amdgcn_readfirstlane(H.parent);
+        const int offset = 2 * H.halfwidth;
+        const long long rs_stride = H.rs_stride;
+        const pzl_const_hr *const hr_tab = (const pzl_const_hr *)a.hr_tab + H.parent;
+        float *pbase = a.planes + (long long)b_lo * a.plane_stride + H.plane_off;
+        const float2 *seg0 = a.segs + H.seg_off;
         // segment values of the next rstep are loaded while this one is transformed;
         // without the split, the spread segment's period N/2 lets an even radix
         // read each value once
@@ -577,7 +592,8 @@ __device__ __forceinline__ void corr_units(const PzlCorrArgs &a, long long u0, l
         constexpr int NSV = HALFPER ? R0 / 2 : R0;
         float2 sv[CP::per(0)][NSV];
         auto load_seg = [&](int b) {
-            const float2 *seg = a.segs + (long long)b * a.seg_stride + H.seg_off;
+            const float2 *seg = seg0 + (long long)b * a.seg_stride;
+            const __amdgpu_buffer_rsrc_t rs = uniform_rsrc(seg, N / 2 * 8);
 #pragma unroll
             for (int i = 0; i < CP::per(0); i++) {
                 const int bf = tid + i * NT;
@@ -586,16 +602,27 @@ __device__ __forceinline__ void corr_units(const PzlCorrArgs &a, long long u0, l
                 if (CP::full(0) || bf < CP::nbf(0)) {
 #pragma unroll
                     for (int r = 0; r < NSV; r++) {
-                        const int k = j + r * NB0;
-                        sv[i][r] = seg[k < N / 2 ? k : k - N / 2];
+                        if constexpr (HALFPER) {  // k < N / 2
+                            const auto v = __builtin_amdgcn_raw_buffer_load_b64(rs, j * 8, r * NB0 * 8, 0);
+                            sv[i][r] = float2{__uint_as_float(v[0]), __uint_as_float(v[1])};
+                        } else {
+                            const int k = j + r * NB0;
+                            sv[i][r] = seg[k < N / 2 ? k : k - N / 2];
+                        }
                     }
                 }
             }
         };
         load_seg(b_lo);
+        // the first values are waited for here: waited for inside the loop (whose
+        // later rounds have theirs already), the wait would also cover the
+        // previous rstep's stores
+#pragma unroll
+        for (int i = 0; i < CP::per(0); i++)
+#pragma unroll
+            for (int r = 0; r < NSV; r++) asm volatile("" : "+v"(sv[i][r].x), "+v"(sv[i][r].y));
         for (int b = b_lo; b < b_hi; b++) {
-            const int numrs = __builtin_amdgcn_readfirstlane(a.hr_tab[b * a.nh + parent].numrs);
-            float *pbase = a.planes + (long long)b * a.plane_stride + H.plane_off;
+            const int numrs = hr_tab[(long long)b * a.nh].numrs;
             float2 cur[CP::per(0)][NSV];
 #pragma unroll
             for (int i = 0; i < CP::per(0); i++)
@@ -646,11 +673,12 @@ __device__ __forceinline__ void corr_units(const PzlCorrArgs &a, long long u0, l
             }
             __syncthreads();
             const auto rows = [&](int i) {
-                return prow[i] >= 0 ? pbase + (long long)prow[i] * H.rs_stride : nullptr;
+                return prow[i] >= 0 ? pbase + (long long)prow[i] * rs_stride : nullptr;
             };
             F::template pass<1>(b0, b1, tw, tid, rows, numrs, offset);
             // the next pass 0 overwrites b0: wait for this FFT's readers of b0
             if constexpr (!PING || (CP::NP % 2 == 0)) __syncthreads();
+            pbase += a.plane_stride;
         }
     }
 }
@@ -852,10 +880,6 @@ template <int POS> __device__ __forceinline__ unsigned pick_bit_t(unsigned u, fl
         : "v"(bits), "n"(POS), "v"(__float_as_uint(x)), "v"(u));
     return m;
 }
-
-// The row-offset table is written once per plan, before any search: reading
-// it through the constant address space lets the compiler use scalar loads.
-typedef const __attribute__((address_space(4))) int pzl_const_int;
 
 template <int NSTAGES, int RPT>
 __global__ __launch_bounds__(SumShape<RPT>::NT) void k_harmsum(PzlSumArgs a)
