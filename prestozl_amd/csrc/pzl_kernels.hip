@@ -273,10 +273,14 @@ template <int N, int NT, int G, bool PING, int PADSH, int... Rs> struct CorrPlan
     static constexpr int nbf(int p) { return G * N / RAD[p]; }     // butterflies of pass p
     static constexpr int per(int p) { return (nbf(p) + NT - 1) / NT; }  // ... per thread
     static constexpr bool full(int p) { return nbf(p) % NT == 0; }
+    // butterflies NT apart share their twiddles (which depend on the butterfly
+    // modulo ns(p)) where ns(p) divides NT
+    static constexpr int twper(int p) { return NT % ns(p) == 0 ? 1 : per(p); }
+    static constexpr int twidx(int p, int i) { return twper(p) == 1 ? 0 : i; }
     static constexpr int twoff(int p)
     {
         int o = 0;
-        for (int i = 1; i < p; i++) o += per(i) * (RAD[i] - 1);
+        for (int i = 1; i < p; i++) o += twper(i) * (RAD[i] - 1);
         return o;
     }
     static constexpr int TWN = twoff(NP);
@@ -306,7 +310,7 @@ template <int N, int NT, int G, bool PING, int SH, int PADSH, int... Rs> struct 
         if constexpr (P < NP) {
             constexpr int R = CP::RAD[P], Ns = CP::ns(P);
 #pragma unroll
-            for (int i = 0; i < CP::per(P); i++) {
+            for (int i = 0; i < CP::twper(P); i++) {
                 int g, j;
                 where<P>(tid + i * NT, g, j);
                 const int m = j % Ns;
@@ -323,10 +327,11 @@ template <int N, int NT, int G, bool PING, int SH, int PADSH, int... Rs> struct 
 
     // passes 1 .. NP-1 of one FFT set; 'src' holds the output of pass P-1.
     // rows(i) is the plane row of this thread's i-th butterfly of the last
-    // pass, null where there is none.
-    template <int P, typename D>
+    // pass, null where there is none; at[i][r] the byte offset of its output r
+    // in the row.
+    template <int P, typename D, typename A>
     static __device__ __forceinline__ void pass(float2 *b0, float2 *b1, const float2 *tw, int tid, const D &rows,
-                                                int numrs, int offset)
+                                                const A &at, int numrs, int offset)
     {
         constexpr int R = CP::RAD[P], Ns = CP::ns(P), NBP = N / R;
         constexpr bool last = (P == NP - 1);
@@ -346,7 +351,7 @@ template <int N, int NT, int G, bool PING, int SH, int PADSH, int... Rs> struct 
                 for (int r = 0; r < R; r++) {
                     float2 x = (NBP % PM == 0) ? rp[r * lds_pad<PADSH>(NBP)]
                                                : src[lds_pad<PADSH>(g * N + j + r * NBP)];
-                    if (r > 0) x = cmul(x, tw[CP::twoff(P) + i * (R - 1) + (r - 1)]);
+                    if (r > 0) x = cmul(x, tw[CP::twoff(P) + CP::twidx(P, i) * (R - 1) + (r - 1)]);
                     v[i][r] = x;
                 }
             }
@@ -364,24 +369,23 @@ template <int N, int NT, int G, bool PING, int SH, int PADSH, int... Rs> struct 
                     float2 *wp = dst + lds_pad<PADSH>(g * N + idxD);
 #pragma unroll
                     for (int r = 0; r < R; r++) {
-                        if constexpr (Ns % (1 << PADSH) == 0) wp[r * lds_pad<PADSH>(Ns)] = v[i][r];
+                        // the padded distance from r = 0 is a constant where the padding's
+                        // period is a multiple of Ns or divides it
+                        if constexpr (Ns % (1 << PADSH) == 0 || ((1 << PADSH) % Ns == 0 && Ns * R % (1 << PADSH) == 0))
+                            wp[lds_pad<PADSH>(r * Ns)] = v[i][r];
                         else dst[lds_pad<PADSH>(g * N + idxD + r * Ns)] = v[i][r];
                     }
                 } else if constexpr (G == 1 || NBP % 64 == 0) {
                     // g is uniform in a wave: a buffer store whose range is the
                     // row's numrs powers drops the outputs outside the r window
                     // (negative offsets wrap to out of range) without branches
-                    const int gu = __builtin_amdgcn_readfirstlane(g);
-                    const int par = gu & ((1 << SH) - 1);
                     float *const pl = rows(i);
                     const __amdgpu_buffer_rsrc_t rs = uniform_rsrc(pl, pl ? numrs * 4 : 0);
 #pragma unroll
                     for (int r = 0; r < R; r++) {
-                        // natural-order output index (of the row) minus offset
-                        const int ro = ((j + r * NBP) << SH) + par - offset;
                         const float2 y = v[i][r];
                         __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y.x * y.x + y.y * y.y), rs,
-                                                              ro * 4, 0, 0);
+                                                              at[i][r], 0, 0);
                     }
                 } else {
                     const int par = g & ((1 << SH) - 1);
@@ -400,7 +404,7 @@ template <int N, int NT, int G, bool PING, int SH, int PADSH, int... Rs> struct 
         }
         if constexpr (!last) {
             __syncthreads();
-            pass<P + 1>(b0, b1, tw, tid, rows, numrs, offset);
+            pass<P + 1>(b0, b1, tw, tid, rows, at, numrs, offset);
         }
     }
 };
@@ -581,11 +585,28 @@ __device__ __forceinline__ void corr_units(const PzlCorrArgs &a, long long u0, l
             if constexpr (GF == 1 || NF / CP::RAD[PL] % 64 == 0) prow[i] = __builtin_amdgcn_readfirstlane(prow[i]);
         }
         const int offset = 2 * H.halfwidth;
+        // Byte offsets of the last pass's outputs in their row: natural-order output
+        // index (of the row) minus offset.  Each sum is made opaque in a register
+        // of its own: a constant part moved into a store's immediate would leave a
+        // negative rest, which the range check drops even where the sum is in range.
+        int at[CP::per(PL)][CP::RAD[PL]];
+#pragma unroll
+        for (int i = 0; i < CP::per(PL); i++) {
+            int g, j;
+            F::template where<PL>(tid + i * NT, g, j);
+            const int par = g & ((1 << SH) - 1);
+#pragma unroll
+            for (int r = 0; r < CP::RAD[PL]; r++) {
+                at[i][r] = 4 * (((j + r * (NF / CP::RAD[PL])) << SH) + par - offset);
+                if constexpr (GF == 1 || NF / CP::RAD[PL] % 64 == 0) asm("" : "+v"(at[i][r]));
+            }
+        }
         const long long rs_stride = H.rs_stride;
         const pzl_const_hr *const hr_tab = (const pzl_const_hr *)a.hr_tab + H.parent;
         float *pbase = a.planes + (long long)b_lo * a.plane_stride + H.plane_off;
         const float2 *seg0 = a.segs + H.seg_off;
-        // segment values of the next rstep are loaded while this one is transformed;
+        // segment values of the next rstep are loaded while this one is transformed,
+        // into the registers its pass 0 has read;
         // without the split, the spread segment's period N/2 lets an even radix
         // read each value once
         constexpr bool HALFPER = SH == 0 && R0 % 2 == 0;
@@ -623,12 +644,6 @@ __device__ __forceinline__ void corr_units(const PzlCorrArgs &a, long long u0, l
             for (int r = 0; r < NSV; r++) asm volatile("" : "+v"(sv[i][r].x), "+v"(sv[i][r].y));
         for (int b = b_lo; b < b_hi; b++) {
             const int numrs = hr_tab[(long long)b * a.nh].numrs;
-            float2 cur[CP::per(0)][NSV];
-#pragma unroll
-            for (int i = 0; i < CP::per(0); i++)
-#pragma unroll
-                for (int r = 0; r < NSV; r++) cur[i][r] = sv[i][r];
-            if (b + 1 < b_hi) load_seg(b + 1);
             // pass 0: P[k] = seg[k mod N/2] * conj(kern[k])
 #pragma unroll
             for (int i = 0; i < CP::per(0); i++) {
@@ -644,7 +659,7 @@ __device__ __forceinline__ void corr_units(const PzlCorrArgs &a, long long u0, l
                         float2 ev[HR], od[HR];
 #pragma unroll
                         for (int r = 0; r < HR; r++) {
-                            const float2 pd = cur[i][r];
+                            const float2 pd = sv[i][r];
                             const float2 ka = kv[i][r], kb = kv[i][r + HR];
                             // re = dr*kr + di*ki, im = di*kr - dr*ki (accel_utils.c:1262-1265)
                             ev[r] = float2{pd.x * ka.x + pd.y * ka.y, pd.y * ka.x - pd.x * ka.y};
@@ -660,7 +675,7 @@ __device__ __forceinline__ void corr_units(const PzlCorrArgs &a, long long u0, l
                     } else {
 #pragma unroll
                         for (int r = 0; r < R0; r++) {
-                            const float2 pd = cur[i][r];
+                            const float2 pd = sv[i][r];
                             const float2 kk = kv[i][r];
                             // re = dr*kr + di*ki, im = di*kr - dr*ki (accel_utils.c:1262-1265)
                             v[r] = float2{pd.x * kk.x + pd.y * kk.y, pd.y * kk.x - pd.x * kk.y};
@@ -671,11 +686,12 @@ __device__ __forceinline__ void corr_units(const PzlCorrArgs &a, long long u0, l
                     for (int r = 0; r < R0; r++) b0[lds_pad<PADSH>(g * NF + j * R0 + r)] = v[r];
                 }
             }
+            if (b + 1 < b_hi) load_seg(b + 1);
             __syncthreads();
             const auto rows = [&](int i) {
                 return prow[i] >= 0 ? pbase + (long long)prow[i] * rs_stride : nullptr;
             };
-            F::template pass<1>(b0, b1, tw, tid, rows, numrs, offset);
+            F::template pass<1>(b0, b1, tw, tid, rows, at, numrs, offset);
             // the next pass 0 overwrites b0: wait for this FFT's readers of b0
             if constexpr (!PING || (CP::NP % 2 == 0)) __syncthreads();
             pbase += a.plane_stride;
@@ -1247,7 +1263,7 @@ static hipError_t launch_corr_t(const PzlCorrArgs *a, const int *class_nrows, hi
 // code) and runs that unit.  The short lengths, which alone fill a small part
 // of the chip, then share one launch and its tail with the longer ones.
 
-#define PZL_CORR_GROUP_MAX 15
+#define PZL_CORR_GROUP_MAX 14
 
 struct PzlCorrGroupArgs {
     PzlCorrArgs c[PZL_CORR_GROUP_MAX];    // per member: its class (total_items 0: absent)
@@ -1354,27 +1370,26 @@ using CorrGroup256Lean =
               CorrV<256, 256, 8, true, 0, 4, 8, 8, 4>, CorrV<192, 256, 8, true, 0, 4, 8, 4, 6>,
               CorrV<128, 256, 16, true, 0, 4, 8, 4, 4>>;
 
-// The groups for rows sorted by width (pzl_launch_corr_group's last group):
-// every row takes the shortest of these lengths that holds its window and its
-// own kernel's width, so the lengths are closely spaced.  What bounds each is
-// FP32 issue (VALU 62-66% busy, LDS exchanges and barriers the rest), at about
-// the same time per point: measured alone on MI355X, 6144 rows x 8 rsteps, ns
-// per row and rstep, 2048: 3.9, 1792: 3.6, 1536: 3.0, 1280: 2.65, 1152: 2.2,
-// 1024: 1.9, 896: 1.7, 768: 1.3, 640: 1.05, 512: 0.83, 4096: 7.7, 3584: 7.0,
-// 3072: 6.5, 2560: 5.8.  Lengths between them (1920, 1728, 1680, 1600, 1440,
-// 1344, 3840, 2304) measured no faster than the next one here: their radices
-// need two butterflies per thread in most passes, which spill at 128 VGPRs.
-// One launch per group: the members of more than 2048 points want 512 threads
-// and twice the LDS, which would halve the others' workgroups per CU.
+// The groups for rows by width (pzl_launch_corr_group's last group): every row
+// takes the shortest of these lengths that holds its window and its own
+// kernel's width, so the lengths are closely spaced where that pays.  What
+// bounds them is FP32 issue: about 300 VALU instructions per thread (8 points)
+// and rstep at 2048, the VALU 90% busy.  Measured alone on MI355X, 6144 rows x
+// 8 rsteps, ns per row and rstep (radices as below, the fastest of those
+// tried): 4096: 6.2, 3584: 5.8, 3072: 5.35, 2560: 4.8, 2048: 3.07, 1792: 2.93,
+// 1536: 2.32, 1280: 2.1, 1152: 1.71, 1024: 1.28, 768: 1.04, 640: 0.81, 512:
+// 0.63, 384: 0.55.  Left out, as (nearly) no faster than the next one here: 3840
+// (6.5), 1920 (3.3), 1344 (2.2), 896 (1.28), 448 (0.63).  One launch per group:
+// the members of more than 2048 points want 512 threads and twice the LDS,
+// which would halve the others' workgroups per CU.
 using CorrGroupWidth =
     CorrGroup<256, 4, CorrV<2048, 256, 1, true, 0, 5, 8, 8, 4, 8>, CorrV<1792, 256, 1, true, 0, 5, 8, 8, 4, 7>,
-              CorrV<1536, 192, 1, true, 0, 5, 8, 8, 3, 8>, CorrV<1280, 256, 1, true, 0, 5, 8, 4, 5, 8>,
+              CorrV<1536, 256, 1, true, 0, 5, 8, 8, 4, 6>, CorrV<1280, 256, 1, true, 0, 5, 8, 4, 5, 8>,
               CorrV<1152, 192, 1, true, 0, 5, 8, 4, 6, 6>, CorrV<1024, 256, 2, true, 0, 5, 8, 4, 4, 8>,
-              CorrV<896, 256, 2, true, 0, 5, 8, 4, 4, 7>, CorrV<768, 192, 2, true, 0, 5, 8, 8, 12>,
-              CorrV<640, 256, 3, true, 0, 5, 8, 8, 10>, CorrV<512, 256, 4, true, 0, 4, 8, 8, 8>,
-              CorrV<384, 256, 4, true, 0, 4, 8, 8, 6>, CorrV<320, 256, 4, true, 0, 5, 8, 8, 5>,
-              CorrV<256, 256, 8, true, 0, 4, 8, 8, 4>, CorrV<192, 256, 8, true, 0, 4, 8, 4, 6>,
-              CorrV<128, 256, 16, true, 0, 4, 8, 4, 4>>;
+              CorrV<768, 192, 2, true, 0, 5, 8, 8, 12>, CorrV<640, 256, 3, true, 0, 5, 8, 8, 10>,
+              CorrV<512, 256, 4, true, 0, 4, 8, 8, 8>, CorrV<384, 256, 4, true, 0, 4, 8, 8, 6>,
+              CorrV<320, 256, 4, true, 0, 3, 8, 8, 5>, CorrV<256, 256, 8, true, 0, 4, 8, 8, 4>,
+              CorrV<192, 192, 4, true, 0, 4, 4, 4, 4, 3>, CorrV<128, 256, 16, true, 0, 4, 8, 4, 4>>;
 using CorrGroupWidthLong =
     CorrGroup<512, 4, CorrV<4096, 512, 1, true, 0, 5, 8, 8, 8, 8>, CorrV<3584, 512, 1, true, 0, 5, 8, 8, 8, 7>,
               CorrV<3072, 512, 1, true, 0, 5, 8, 8, 6, 8>, CorrV<2560, 512, 1, true, 0, 5, 8, 8, 5, 8>>;
@@ -1414,7 +1429,7 @@ static const CorrGroupEntry g_corr_groups[] = {
      CorrGroup256::has},
     {"256t lean: 2048:1r 1280:1r 1024:2r 768:1r 512:4r 384:4r 256:8r 192:8r 128:16r", CorrGroup256Lean::launch,
      CorrGroup256Lean::has},
-    {"rows by width: 128 192 256 320 384 512 640 768 896 1024 1152 1280 1536 1792 2048 2560 3072 3584 4096",
+    {"rows by width: 128 192 256 320 384 512 640 768 1024 1152 1280 1536 1792 2048 2560 3072 3584 4096",
      width_group_launch, width_group_has},
 };
 static const int g_ncorr_groups = (int)(sizeof(g_corr_groups) / sizeof(g_corr_groups[0]));
