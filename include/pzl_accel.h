@@ -45,7 +45,8 @@ typedef struct PzlConfig {
     int floP, fhiP, rloP, rhiP;
     double flo, fhi, rlo, rhi;
     double nph;          /* > 0: photon normalisation (-photon) */
-    int batchsize;       /* rsteps per launch group (-batchsize), >= 1 */
+    int batchsize;       /* rsteps per launch group (-batchsize), >= 1; above 1 a plan whose planes are
+                            small takes more (results do not depend on it) */
     long long maxhits;   /* hit-buffer capacity, 0 = default */
 } PzlConfig;
 

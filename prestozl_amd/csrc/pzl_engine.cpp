@@ -145,10 +145,15 @@ int need_whole_bank(Plan *p)
     return rc;
 }
 
+constexpr int kMaxBatch = 512;  // rsteps per launch the rule below goes up to
+// bytes of planes per batch it aims for; up to 32 rsteps
+constexpr long long kBatchPlanes = 512LL << 20, kBatchPlanesMost = 2LL << 30;
+
 // Batch size, hit-slot capacity and slot count of a plan (pzl_plan_create
 // uses them; the request loop uses them to size a request before admission).
 struct PlanSizes {
-    int B;
+    int B;     // rsteps per launch ...
+    int sub;   // ... and what a batch that overflows its slot is searched again by
     long long hitcap;
     int nslots;
     long long seg_stride;      // whole rows' segments of one rstep ...
@@ -165,14 +170,25 @@ int width_has(int n) { return pzl_corr_group_has(width_group(), n); }
 PlanSizes plan_sizes(const PzlConfig &cfg, const PzlGeometry &g, const std::vector<PzlHarm> &harms)
 {
     PlanSizes z;
-    z.B = cfg.batchsize > 0 ? cfg.batchsize : 8;
-    if (g.nrsteps > 0 && z.B > g.nrsteps) z.B = (int)g.nrsteps;
-    if (z.B < 1) z.B = 1;
+    z.sub = cfg.batchsize > 0 ? cfg.batchsize : 8;
+    if (g.nrsteps > 0 && z.sub > g.nrsteps) z.sub = (int)g.nrsteps;
+    if (z.sub < 1) z.sub = 1;
+    // More rsteps per launch than asked for while a batch's planes are small:
+    // a short search then fills the chip and does not pay per batch for its
+    // launches, its count's way to the host and its sort.  (One rstep per launch
+    // stays one.)  Up to 32 rsteps also while the planes are large, as each kernel
+    // row is read once per batch.  Measured on MI355X, per search, at 8 and at the
+    // rule's count: 540 rsteps of 0.3 MB 4.3 -> 0.42 ms (512), 1117 of 1.3 MB 7.9 ->
+    // 1.5 ms (512), 182 of 92 MB 12.9 -> 11.5 ms (32).
+    z.B = z.sub;
+    while (z.sub > 1 && z.B < kMaxBatch && z.B < g.nrsteps &&
+           (long long)z.B * g.plane_bytes_per_rstep < (z.B < 32 ? kBatchPlanesMost : kBatchPlanes))
+        z.B = (int)std::min<long long>({2LL * z.B, kMaxBatch, g.nrsteps});
     const PzlHarm &F = harms[0];
     // one rstep can never overflow a slot
     const long long per_rstep = (long long)g.corr_uselen * F.numz * F.numw * g.numharmstages;
     long long cap = cfg.maxhits > 0 ? cfg.maxhits : kDefaultHitCap;
-    cap = std::min<long long>(cap, per_rstep * z.B);
+    cap = std::min<long long>(cap, per_rstep * z.sub);
     z.hitcap = std::max<long long>(cap, per_rstep);
     const long long nbatches = (g.nrsteps + z.B - 1) / z.B;
     z.nslots = (int)std::max<long long>(1, std::min<long long>(Plan::kSlots, nbatches));
@@ -351,6 +367,29 @@ void pin_put(PzlHostHit *ptr, long long cap)
     pinned_free(ptr);
 }
 
+}  // namespace
+
+// At least 'count' whole chunks of hit records in the process-wide cache, as far
+// as its limit allows: the searches of a request loop then find theirs instead of
+// pinning 32 MiB (5 to 10 ms) while others run.
+int pzl::reserve_pinned_chunks(int count)
+{
+    constexpr long long chunk = 1LL << 20;
+    for (;;) {
+        {
+            std::lock_guard<std::mutex> lk(g_pin_mu);
+            int have = 0;
+            for (auto &kv : g_pin_cache) have += kv.first >= chunk;
+            if (have >= count || g_pin_cache_bytes + (long long)sizeof(PzlHostHit) * chunk > kPinCacheLimit) return 0;
+        }
+        PzlHostHit *ptr = nullptr;
+        PZL_HIPCHK(pinned_alloc((void **)&ptr, sizeof(PzlHostHit) * (size_t)chunk));
+        pin_put(ptr, chunk);
+    }
+}
+
+namespace {
+
 void free_plan(Plan *p)
 {
     if (!p) return;
@@ -394,7 +433,7 @@ void free_plan(Plan *p)
 
 struct Timers {
     bool on = false;
-    bool active = true;  // record this batch (searches sample every kSampleEvery-th batch)
+    bool active = true;  // record this batch (long searches sample some)
     std::vector<hipEvent_t> pool;
     size_t used = 0;
     struct Rec {
@@ -554,6 +593,7 @@ int launch_corrs(Plan &p, int nb, int set, Timers *tm, bool seg_stream)
         PZL_HIPCHK(hipEventRecord(p.ev_side[set], ss));
         PZL_HIPCHK(hipStreamWaitEvent(p.st, p.ev_side[set], 0));
     }
+    if (!pzl_recorder) p.graph_ready = true;
     return 0;
 }
 
@@ -656,7 +696,11 @@ int build_batch_graph(Plan &p, int set, hipGraphExec_t *out)
 
 int launch_corr_graph(Plan &p, long long r0, int set, Timers *tm, bool seg_ahead)
 {
-    if (!p.gexec[set]) {
+    // (a set's first full batch is replayed too once the process has built what
+    // the kernels read once per device)
+    if (!p.gexec[set] && !(p.graph_ready && build_batch_graph(p, set, &p.gexec[set]) == 0)) {
+        (void)hipGetLastError();
+        pzl::g_err.clear();
         int rc = launch_corr_part(p, r0, p.B, set, tm, nullptr, seg_ahead);
         if (rc) return rc;
         if (build_batch_graph(p, set, &p.gexec[set])) {
@@ -715,6 +759,8 @@ int sync_all(Plan &p)
 // batches, applied in batch order (the scan order of the reference's
 // insertion); each sits in a pinned buffer of the plan's pool together with
 // the event of the copy that fills it, which the insertion thread waits for.
+constexpr long long kSmallChunk = 1LL << 16;  // records of a small pinned buffer
+
 struct SearchState {
     Plan *p = nullptr;
     CandList cl;
@@ -748,10 +794,12 @@ struct SearchState {
     // for the device and takes milliseconds, and a launching thread doing it
     // in the middle of a search leaves the GPU without work.  A free buffer,
     // else a new one while the pool stays within its limit, else wait for the
-    // insertion thread to release one.
-    int acquire()
+    // insertion thread to release one.  A batch of few hits asks for a small
+    // buffer (pinning 2 MiB takes a fraction of a millisecond, a whole chunk
+    // several), which most searches then need one or two of.
+    int acquire(long long records)
     {
-        const long long chunk = p->hit_chunk;
+        const long long chunk = std::min(p->hit_chunk, records <= kSmallChunk ? kSmallChunk : p->hit_chunk);
         const long long chunk_bytes = (long long)sizeof(PzlHostHit) * chunk;
         std::unique_lock<std::mutex> lk(mu);
         for (;;) {
@@ -904,7 +952,7 @@ int apply_slot(Plan &p, int slot, long long n, SearchState &ss)
     // applies the jobs first in, first out)
     for (long long off = 0; off < n; off += p.hit_chunk) {
         const long long m = std::min(p.hit_chunk, n - off);
-        const int buf = ss.acquire();
+        const int buf = ss.acquire(m);
         if (buf < 0)
             return fail(ss.err ? ss.err : PZL_ERR_HIP, "no pinned buffer for %lld hit records%s%s", m,
                         ss.err_msg.empty() ? "" : ": ", ss.err_msg.c_str());
@@ -926,9 +974,40 @@ int reset_slot(Plan &p, int slot, hipStream_t st)
     return 0;
 }
 
+// Search rsteps [r0, r0 + nb) again, nothing else in flight, in pieces of at
+// most 'step': a piece that overflows the slot is done one rstep at a time (one
+// rstep never exceeds a slot: hitcap >= cells per rstep x stages).
+int search_again(Plan &p, int slot, long long r0, int nb, int step, SearchState &ss, Timers *tm)
+{
+    for (int b = 0; b < nb; b += step) {
+        const int m = std::min(step, nb - b);
+        // the previous piece's sort (stream st2) reads and rewrites the slot's
+        // buffers: the harmonic sum refills them only after it
+        PZL_HIPCHK(hipStreamWaitEvent(p.sum_stream(), p.ev_free[slot], 0));
+        int rc = reset_slot(p, slot, p.sum_stream());
+        if (rc) return rc;
+        rc = launch_batch(p, r0 + b, m, 0, slot, nullptr, tm);
+        if (rc) return rc;
+        PZL_PINNED_CHECK(p.h_counts + 2 * slot, 2 * sizeof(unsigned long long));
+        PZL_HIPCHK(hipMemcpyAsync(p.h_counts + 2 * slot, p.d_counts + 2 * slot, 2 * sizeof(unsigned long long),
+                                  hipMemcpyDeviceToHost, p.sum_stream()));
+        rc = sync_all(p);
+        if (rc) return rc;
+        const unsigned long long n = p.h_counts[2 * slot];
+        if ((long long)n <= p.hitcap) {
+            rc = apply_slot(p, slot, (long long)n, ss);
+        } else if (m > 1) {
+            rc = search_again(p, slot, r0 + b, m, 1, ss, tm);
+        } else {
+            rc = fail(PZL_ERR_OVERFLOW, "hit buffer overflow: %llu hits in one rstep", n);
+        }
+        if (rc) return rc;
+    }
+    return 0;
+}
+
 // Wait for the batch in 'slot', order and apply its hits.  A batch that
-// overflowed the slot is searched again one rstep at a time (one rstep never
-// exceeds a slot: hitcap >= cells per rstep x stages).
+// overflowed the slot is searched again in the pieces the slot was sized for.
 int finalize(Plan &p, int slot, long long r0, int nb, SearchState &ss, Timers *tm)
 {
     const auto w0 = std::chrono::steady_clock::now();
@@ -936,30 +1015,10 @@ int finalize(Plan &p, int slot, long long r0, int nb, SearchState &ss, Timers *t
     ss.ms_wait_count += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - w0).count();
     const unsigned long long n = p.h_counts[2 * slot];
     if ((long long)n <= p.hitcap) return apply_slot(p, slot, (long long)n, ss);  // resets the slot
-    // overflow: let every batch in flight finish, then search this batch
-    // again one rstep at a time
-    int rc = sync_all(p);
+    // overflow: let every batch in flight finish, then search this batch again
+    const int rc = sync_all(p);
     if (rc) return rc;
-    for (int b = 0; b < nb; b++) {
-        // the previous rstep's sort (stream st2) reads and rewrites the slot's
-        // buffers: the harmonic sum refills them only after it
-        PZL_HIPCHK(hipStreamWaitEvent(p.sum_stream(), p.ev_free[slot], 0));
-        rc = reset_slot(p, slot, p.sum_stream());
-        if (rc) return rc;
-        rc = launch_batch(p, r0 + b, 1, 0, slot, nullptr, tm);
-        if (rc) return rc;
-        PZL_PINNED_CHECK(p.h_counts + 2 * slot, 2 * sizeof(unsigned long long));
-        PZL_HIPCHK(hipMemcpyAsync(p.h_counts + 2 * slot, p.d_counts + 2 * slot, 2 * sizeof(unsigned long long),
-                                  hipMemcpyDeviceToHost, p.sum_stream()));
-        rc = sync_all(p);
-        if (rc) return rc;
-        const unsigned long long n1 = p.h_counts[2 * slot];
-        if ((long long)n1 > p.hitcap)
-            return fail(PZL_ERR_OVERFLOW, "hit buffer overflow: %llu hits in one rstep", n1);
-        rc = apply_slot(p, slot, (long long)n1, ss);
-        if (rc) return rc;
-    }
-    return 0;
+    return search_again(p, slot, r0, nb, nb > p.sub_batch ? p.sub_batch : 1, ss, tm);
 }
 
 double plane_alg_bytes(const Plan &p)
@@ -1057,6 +1116,7 @@ int pzl_plan_create(const PzlConfig *cfg, int device, void **plan_out)
     for (int s = 0; s < p->g.numharmstages; s++) p->numindep_d[s] = (double)p->g.numindep[s];
     const PlanSizes sizes = plan_sizes(*cfg, p->g, p->harms);
     p->B = sizes.B;
+    p->sub_batch = sizes.sub;
     const int nh = (int)p->harms.size();
     const PzlHarm &F = p->harms[0];
     p->fnumz = F.numz;
@@ -1143,6 +1203,14 @@ int pzl_plan_create(const PzlConfig *cfg, int device, void **plan_out)
             for (int k : c.harms) c.nrows.push_back(p->sets[k].nrows);
             p->set_classes.push_back(c);
         }
+    }
+    // The harmonic sum's form: 4 r per thread, r chunks fastest, unless a batch has
+    // too few of its workgroups to fill the chip.  Measured on MI355X per search, at
+    // the batch sizes above: (200, 300, 8) 11.5 -> 11.1 ms, (50, 0, 8) 1.60 -> 1.51
+    // ms; 268 workgroups (67 rsteps of one z block) 0.255 -> 0.265 ms.
+    if ((long long)p->B * F.numw * ((F.numz + 31) / 32) * ((p->g.corr_uselen + 511) / 512) >= 512) {
+        p->sum_order = 1;
+        p->sum_rpt = 4;
     }
     p->hitcap = sizes.hitcap;
     const long long maxkey = std::max<long long>(p->g.nrsteps, 1) * p->g.numharmstages * F.numw * F.numz *
@@ -1383,9 +1451,10 @@ int pzl_search(void *plan, long long rstep_lo, long long rstep_hi, PzlCand *cand
     std::vector<Pending> pend;
     size_t head = 0;
     int i = 0;
-    // per-kernel events on every kSampleEvery-th batch only: the averages stay
+    // per-kernel events on every eighth batch of a long search only: the averages stay
     // representative and the event packets do not perturb the timed search
-    constexpr int kSampleEvery = 8;
+    const int sample_every =
+        (int)std::max<long long>(1, std::min<long long>(8, (rstep_hi - rstep_lo) / std::max(p->B, 1) / 8));
     long long sampled = 0;
     bool timed_out = false;
     for (long long r0 = rstep_lo; r0 < rstep_hi; r0 += p->B, i++) {
@@ -1395,7 +1464,7 @@ int pzl_search(void *plan, long long rstep_lo, long long rstep_hi, PzlCand *cand
         }
         const int nb = (int)std::min<long long>(p->B, rstep_hi - r0);
         const int slot = i % p->nslots;
-        tm.active = (i % kSampleEvery) == 0;
+        tm.active = (i % sample_every) == 0;
         sampled += tm.active;
         if (pend.size() - head == (size_t)p->nslots) {
             const Pending q = pend[head++];

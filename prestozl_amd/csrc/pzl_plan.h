@@ -44,6 +44,8 @@ int compute_geometry(const PzlConfig &c, PzlGeometry &g, std::vector<PzlHarm> *h
 bool compute_row_sets(const std::vector<PzlHarm> &harms, int corr_uselen, int (*has)(int n), std::vector<PzlHarm> *sets,
                       std::vector<int> *rows);
 
+int reserve_pinned_chunks(int count);  // pzl_engine.cpp
+
 struct Plan {
     PzlConfig cfg{};
     PzlGeometry g{};
@@ -65,7 +67,8 @@ struct Plan {
     int fnumw = 1, fnumz = 1, fzlo = 0, fwlo = 0;
     int max_fftlen = 0;
     int int_rlo = 1;  // every startr is an integer (integer r maps on the GPU)
-    int B = 8;
+    int B = 8;          // rsteps per launch
+    int sub_batch = 8;  // rsteps a hit slot is sized for (an overflowed batch is searched again by these)
     int device = 0;
     hipStream_t st = nullptr;   // segments and correlations
     hipStream_t st2 = nullptr;  // hit ordering
@@ -154,6 +157,7 @@ struct Plan {
     // graph replay of full batches (one executable graph per buffer set)
     bool use_graph = true;
     static constexpr int kMaxGraphFailures = 8;
+    bool graph_ready = false;  // a batch ran eagerly: the kernels' tables exist
     int graph_failures = 0;  // batch graphs the runtime refused (those batches ran eagerly)
     hipGraphExec_t gexec[kSets] = {};  // correlation part, per buffer set
     // pzl_plan_set_deadline: searches stop launching batches after this time

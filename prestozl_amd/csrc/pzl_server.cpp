@@ -202,6 +202,9 @@ struct Server {
             int rc = 0;
             if (!plan) {
                 rc = pzl_plan_create(&r->cfg, device, &plan);
+                // a request gives its candidates only: its hits (32 bytes each, up to
+                // millions) are not kept
+                if (rc == 0) rc = pzl_plan_set_keep_hits(plan, 0);
                 std::lock_guard<std::mutex> lk(mu);
                 if (rc == 0) {
                     PooledPlan p;
@@ -283,6 +286,10 @@ int pzl_server_create(int device, long long hbm_budget, int max_inflight, void *
             return fail(PZL_ERR_HIP, "hipMemGetInfo failed: %s", hipGetErrorString(e));
         }
         hbm_budget = (long long)(free_b * 0.8);
+    }
+    if (reserve_pinned_chunks(std::min(max_inflight, 8))) {
+        delete s;
+        return PZL_ERR_HIP;
     }
     s->budget = hbm_budget;
     s->max_inflight = max_inflight;
