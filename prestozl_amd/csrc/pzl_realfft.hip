@@ -67,11 +67,16 @@ __device__ __forceinline__ void rf_pass(float2 *buf, int L, int nseq, int sstrid
             const int s = dnbf.div(g), j = g - s * nbf, jm = j - dns.div(j) * Ns;
             const float2 *q = buf + s * sstride;
             v[b][0] = q[j];
+            if (Ns == 1) {  // the first pass: no twiddles
 #pragma unroll
-            for (int r = 1; r < R; r++) {
-                float2 t = tw[jm * r * step];
-                if (SIGN > 0) t.y = -t.y;
-                v[b][r] = cmul(q[j + r * nbf], t);
+                for (int r = 1; r < R; r++) v[b][r] = q[j + r * nbf];
+            } else {
+#pragma unroll
+                for (int r = 1; r < R; r++) {
+                    float2 t = tw[jm * r * step];
+                    if (SIGN > 0) t.y = -t.y;
+                    v[b][r] = cmul(q[j + r * nbf], t);
+                }
             }
         }
     }
@@ -138,42 +143,82 @@ __device__ inline long long rf_group(int b, int nb)
     return (nb % 8) ? b : (long long)(b % 8) * (nb / 8) + b / 8;
 }
 
+// The four-step kernels for FFT length L, a power of two compiled into the pass
+// sequence, or 0 for the run-time pass loop.
+//
+// The tile is C sequences of L float2 (C <= 16, per_block below): one radix-16
+// butterfly per thread, so NT = C L / 16 threads.
+// pad(): the compiled passes read and write LDS with one float2 of padding
+// after every 16.  The first radix-16 pass stores with a stride of 16 float2,
+// which without it puts a wave's 64 stores of 8 bytes on 2 of the 64 banks.
+// With 1024 threads for every L and no padding, 564 series of 2^18 samples (512
+// by 256) took 720 + 598 us in the two kernels, with both 625 + 323; one series
+// of 2^24 (4096 by 2048) 90 + 62 us, now 76 + 46.  Both kernels read and write
+// each value once: 1.18 GB, 0.2 ms each at the memory's rate; what is left is
+// the vector unit and, for L >= 4096, rows of 32 bytes.
+template <int L>
+struct RfTile {
+    static constexpr int cmax()
+    {
+        int c = 16;
+        while (c > 1 && c * (L + 1) > RF_MAXE) c >>= 1;
+        return c;
+    }
+    static constexpr int NT = L == 0 || cmax() * L / 16 > RF_NT ? RF_NT : cmax() * L / 16;
+    static constexpr int pad(int i) { return L == 0 ? i : i + (i >> 4); }
+};
+
+// float2 between the sequences of a tile.
+int rf_stride(int L)
+{
+    switch (L) {
+    case 256: case 512: case 1024: case 2048: case 4096: case 8192: return L + L / 16 + 1;
+    default: return L + 1;
+    }
+}
+
 // The same pass with L and Ns known at compile time (powers of two): the
-// butterfly indices are shifts and masks.  The sequence count stays a
-// run-time value.
+// butterfly indices are shifts and masks, and pad(o + r Ns) = pad(o) + a
+// constant.  The sequence count stays a run-time value.
 template <int SIGN, int R, int L, int Ns>
 __device__ __forceinline__ void rf_pass_ct(float2 *buf, int nseq, int sstride, const float2 *__restrict__ tw, int tid)
 {
-    constexpr int MAXB = (RF_MAXE / R + RF_NT - 1) / RF_NT;
+    using T = RfTile<L>;
+    constexpr int MAXB = (T::cmax() * L / R + T::NT - 1) / T::NT;
     constexpr int nbf = L / R, step = L / (Ns * R);
+    static_assert(nbf % 16 == 0 && (Ns % 16 == 0 || (Ns == 1 && R == 16)), "pad() must split");
     const int total = nbf * nseq;
     float2 v[MAXB][R];
 #pragma unroll
     for (int b = 0; b < MAXB; b++) {
-        const int g = tid + b * RF_NT;
+        const int g = tid + b * T::NT;
         if (g < total) {
             const int s = g / nbf, j = g % nbf, jm = j % Ns;
-            const float2 *q = buf + s * sstride;
-            v[b][0] = q[j];
+            const float2 *q = buf + s * sstride + T::pad(j);
+            v[b][0] = q[0];
+            if constexpr (Ns == 1) {  // the first pass: no twiddles
 #pragma unroll
-            for (int r = 1; r < R; r++) {
-                float2 t = tw[jm * r * step];
-                if (SIGN > 0) t.y = -t.y;
-                v[b][r] = cmul(q[j + r * nbf], t);
+                for (int r = 1; r < R; r++) v[b][r] = q[T::pad(r * nbf)];
+            } else {
+#pragma unroll
+                for (int r = 1; r < R; r++) {
+                    float2 t = tw[jm * r * step];
+                    if (SIGN > 0) t.y = -t.y;
+                    v[b][r] = cmul(q[T::pad(r * nbf)], t);
+                }
             }
         }
     }
     __syncthreads();
 #pragma unroll
     for (int b = 0; b < MAXB; b++) {
-        const int g = tid + b * RF_NT;
+        const int g = tid + b * T::NT;
         if (g < total) {
             const int s = g / nbf, j = g % nbf, jm = j % Ns, jq = j / Ns;
             dftR<R, SIGN>(v[b]);
-            float2 *q = buf + s * sstride;
-            const int o = jq * Ns * R + jm;
+            float2 *q = buf + s * sstride + T::pad(jq * Ns * R + jm);
 #pragma unroll
-            for (int r = 0; r < R; r++) q[o + r * Ns] = v[b][r];
+            for (int r = 0; r < R; r++) q[T::pad(r * Ns)] = v[b][r];
         }
     }
     __syncthreads();
@@ -190,8 +235,6 @@ __device__ __forceinline__ void rf_fft_ct(float2 *buf, int nseq, int sstride, co
     }
 }
 
-// FFT length L of the four-step kernels: 0 for the run-time pass loop, else a
-// power of two compiled into the pass sequence.
 template <int SIGN, int L>
 __device__ __forceinline__ void rf_fft_any(float2 *buf, int n, int nseq, int sstride, const float2 *__restrict__ tw,
                                            int tid)
@@ -205,27 +248,29 @@ __device__ inline float2 rf_scale(float2 v, double scale)
     return float2{(float)((double)v.x * scale), (float)((double)v.y * scale)};
 }
 
-// tw[j] = exp(-2 pi i j / L), j < L
-__global__ __launch_bounds__(256) void k_rf_twiddles(float2 *__restrict__ tw, int L)
-{
-    const int j = blockIdx.x * 256 + threadIdx.x;
-    if (j < L) {
-        double s, c;
-        sincospi(-2.0 * (double)j / (double)L, &s, &c);
-        tw[j] = float2{(float)c, (float)s};
-    }
-}
-
-// The four-step twiddles exp(-2 pi i p / M), p < M, as the product of
-// lo[p % RF_TB] = exp(-2 pi i (p % RF_TB) / M) and hi[p / RF_TB] =
-// exp(-2 pi i RF_TB (p / RF_TB) / M), both in double.
+// Every table of a transform in one launch: as three launches, 3 us more of a
+// 2^24-sample transform's 0.21 ms and of the 0.12 ms of three of 2112000.  Thread
+// j sets:
+//   tw1[j] = exp(-2 pi i j / M1), j < M1, and tw2 likewise;
+//   the four-step twiddles exp(-2 pi i p / M), p < M, as the product of
+//   lo[p % RF_TB] = exp(-2 pi i (p % RF_TB) / M) and hi[p / RF_TB] =
+//   exp(-2 pi i RF_TB (p / RF_TB) / M), both in double (nhi 0: none).
 #define RF_TB 4096
-__global__ __launch_bounds__(256) void k_rf_twiddles_step(double2 *__restrict__ lo, double2 *__restrict__ hi,
-                                                          long long M, int nhi)
+__global__ __launch_bounds__(256) void k_rf_twiddles(float2 *__restrict__ tw1, int M1, float2 *__restrict__ tw2, int M2,
+                                                     double2 *__restrict__ lo, double2 *__restrict__ hi,
+                                                     long long M, int nhi)
 {
     const int j = blockIdx.x * 256 + threadIdx.x;
     double s, c;
-    if (j < RF_TB) {
+    if (j < M1) {
+        sincospi(-2.0 * (double)j / (double)M1, &s, &c);
+        tw1[j] = float2{(float)c, (float)s};
+    }
+    if (j < M2) {
+        sincospi(-2.0 * (double)j / (double)M2, &s, &c);
+        tw2[j] = float2{(float)c, (float)s};
+    }
+    if (nhi > 0 && j < RF_TB) {
         sincospi(-2.0 * (double)j / (double)M, &s, &c);
         lo[j] = double2{c, s};
     }
@@ -250,92 +295,106 @@ __global__ __launch_bounds__(RF_NT) void k_rf_single(float2 *__restrict__ data, 
     for (int e = tid; e < M; e += RF_NT) data[e] = scale == 1.0 ? rbuf[e] : rf_scale(rbuf[e], scale);
 }
 
+// exp(SIGN 2 pi i p / M) from the two tables, p < M.
+template <int SIGN>
+__device__ __forceinline__ double2 rf_twiddle(unsigned p, const double2 *__restrict__ tlo,
+                                              const double2 *__restrict__ thi)
+{
+    const double2 a = tlo[p % RF_TB], h = thi[p / RF_TB];
+    return double2{a.x * h.x - a.y * h.y, (a.x * h.y + a.y * h.x) * (double)(-SIGN)};
+}
+
 // Columns j2b .. j2b + C - 1 of the [M1][M2] view of 'in': FFT of length M1
 // down each, times exp(SIGN 2 pi i k1 j2 / M), into 'out' at the same places.
+// C = 2^lc; places in the view are below 2^26.
 template <int SIGN, int L>
-__global__ __launch_bounds__(RF_NT) void k_rf_cols(const float2 *__restrict__ in, float2 *__restrict__ out, int M1,
-                                                   int M2, int C, const float2 *__restrict__ tw,
-                                                   const double2 *__restrict__ tlo, const double2 *__restrict__ thi)
+__global__ __launch_bounds__(RfTile<L>::NT) void k_rf_cols(const float2 *__restrict__ in, float2 *__restrict__ out,
+                                                           int M1, int M2, int lc, const float2 *__restrict__ tw,
+                                                           const double2 *__restrict__ tlo,
+                                                           const double2 *__restrict__ thi)
 {
     extern __shared__ float2 rbuf[];
-    const int tid = threadIdx.x, sstride = M1 + 1;
-    const long long j2b = rf_group(blockIdx.x, gridDim.x) * C;
-    const long long M = (long long)M1 * M2;
-    in += blockIdx.y * M;  // series of the batch (M float2 each)
-    out += blockIdx.y * M;
-    const int total = C * M1;
-    const RfDiv dc(C);
+    using T = RfTile<L>;
+    constexpr int NT = T::NT;
+    const int tid = threadIdx.x, C = 1 << lc, sstride = L ? T::pad(L) + 1 : M1 + 1;
+    const unsigned j2b = (unsigned)rf_group(blockIdx.x, gridDim.x) << lc;
+    in += blockIdx.y * ((long long)M1 * M2);  // series of the batch (M float2 each)
+    out += blockIdx.y * ((long long)M1 * M2);
+    const int total = M1 << lc;
     // RF_U loads in flight per thread before their LDS stores
-    for (int e0 = 0; e0 < total; e0 += RF_U * RF_NT) {
+    for (int e0 = 0; e0 < total; e0 += RF_U * NT) {
         float2 t[RF_U];
 #pragma unroll
         for (int u = 0; u < RF_U; u++) {
-            const int e = e0 + u * RF_NT + tid;
-            if (e < total) {
-                const int j1 = dc.div(e), c = e - j1 * C;
-                t[u] = in[(long long)j1 * M2 + j2b + c];
-            }
+            const int e = e0 + u * NT + tid;
+            if (e < total) t[u] = in[(unsigned)(e >> lc) * M2 + j2b + (e & (C - 1))];
         }
 #pragma unroll
         for (int u = 0; u < RF_U; u++) {
-            const int e = e0 + u * RF_NT + tid;
-            if (e < total) {
-                const int j1 = dc.div(e), c = e - j1 * C;
-                rbuf[c * sstride + j1] = t[u];
-            }
+            const int e = e0 + u * NT + tid;
+            if (e < total) rbuf[(e & (C - 1)) * sstride + T::pad(e >> lc)] = t[u];
         }
     }
     __syncthreads();
     rf_fft_any<SIGN, L>(rbuf, M1, C, sstride, tw, tid);
+    // A thread stays in its column, NT / C rows further each time: its twiddle is
+    // the last one times exp(SIGN 2 pi i (NT / C) j2 / M), in double (at most 16
+    // steps: 4e-15, far below the float it is rounded to).  Two gathers of 16
+    // bytes per element from tables that the L1 does not hold were half of this
+    // kernel's time (564 series of 2^18 samples, FFTs of 512: 625 us, now 475).
+    const unsigned c = tid & (C - 1), j2 = j2b + c, dk = NT >> lc;
+    const double2 w0 = rf_twiddle<SIGN>(tid < total ? (tid >> lc) * j2 : 0, tlo, thi);  // places below M1 M2 = M
+    const double2 dw = rf_twiddle<SIGN>(tid + NT < total ? dk * j2 : 0, tlo, thi);
+    double co = w0.x, sn = w0.y;
 #pragma unroll 4
-    for (int e = tid; e < total; e += RF_NT) {
-        const int k1 = dc.div(e), c = e - k1 * C;
-        const long long j2 = j2b + c, p = (long long)k1 * j2;  // < M1 M2 = M
-        const double2 a = tlo[p % RF_TB], h = thi[p / RF_TB];
-        const double co = a.x * h.x - a.y * h.y, sn = (a.x * h.y + a.y * h.x) * (double)(-SIGN);
-        out[(long long)k1 * M2 + j2] = cmul(rbuf[c * sstride + k1], float2{(float)co, (float)sn});
+    for (int e = tid; e < total; e += NT) {
+        const unsigned k1 = e >> lc;
+        out[k1 * M2 + j2] = cmul(rbuf[c * sstride + T::pad(k1)], float2{(float)co, (float)sn});
+        const double t = co * dw.x - sn * dw.y;
+        sn = co * dw.y + sn * dw.x;
+        co = t;
     }
 }
 
 // Rows k1b .. k1b + C2 - 1 of the [M1][M2] view of 'in': FFT of length M2
-// along each, element k2 of row k1 to out[k1 + M1 k2], times 'scale'.
+// along each, element k2 of row k1 to out[k1 + M1 k2], times 'scale'.  C2 = 2^lc.
 template <int SIGN, int L>
-__global__ __launch_bounds__(RF_NT) void k_rf_rows(const float2 *__restrict__ in, float2 *__restrict__ out, int M1,
-                                                   int M2, int C2, const float2 *__restrict__ tw, double scale)
+__global__ __launch_bounds__(RfTile<L>::NT) void k_rf_rows(const float2 *__restrict__ in, float2 *__restrict__ out,
+                                                           int M1, int M2, int lc, const float2 *__restrict__ tw,
+                                                           double scale)
 {
     extern __shared__ float2 rbuf[];
-    const int tid = threadIdx.x, sstride = M2 + 1;
-    const long long k1b = rf_group(blockIdx.x, gridDim.x) * C2;
-    in += blockIdx.y * (long long)M1 * M2;  // series of the batch
-    out += blockIdx.y * (long long)M1 * M2;
-    const int total = C2 * M2;
-    const RfDiv dm2(M2), dc2(C2);
-    for (int e0 = 0; e0 < total; e0 += RF_U * RF_NT) {
+    using T = RfTile<L>;
+    constexpr int NT = T::NT;
+    const int tid = threadIdx.x, C2 = 1 << lc, sstride = L ? T::pad(L) + 1 : M2 + 1;
+    const unsigned k1b = (unsigned)rf_group(blockIdx.x, gridDim.x) << lc;
+    in += blockIdx.y * ((long long)M1 * M2);  // series of the batch
+    out += blockIdx.y * ((long long)M1 * M2);
+    const int total = M2 << lc;
+    const RfDiv dm2(L ? L : M2);
+    for (int e0 = 0; e0 < total; e0 += RF_U * NT) {
         float2 t[RF_U];
 #pragma unroll
         for (int u = 0; u < RF_U; u++) {
-            const int e = e0 + u * RF_NT + tid;
-            if (e < total) {
-                const int c = dm2.div(e), j2 = e - c * M2;
-                t[u] = in[(k1b + c) * M2 + j2];
-            }
+            const int e = e0 + u * NT + tid;
+            if (e < total) t[u] = in[k1b * M2 + e];  // whole rows, one after the other
         }
 #pragma unroll
         for (int u = 0; u < RF_U; u++) {
-            const int e = e0 + u * RF_NT + tid;
+            const int e = e0 + u * NT + tid;
             if (e < total) {
-                const int c = dm2.div(e), j2 = e - c * M2;
-                rbuf[c * sstride + j2] = t[u];
+                const int c = L ? e / (L ? L : 1) : dm2.div(e), j2 = e - c * (L ? L : M2);
+                rbuf[c * sstride + T::pad(j2)] = t[u];
             }
         }
     }
     __syncthreads();
     rf_fft_any<SIGN, L>(rbuf, M2, C2, sstride, tw, tid);
 #pragma unroll 4
-    for (int e = tid; e < total; e += RF_NT) {
-        const int k2 = dc2.div(e), c = e - k2 * C2;
-        const float2 v = rbuf[c * sstride + k2];
-        out[(long long)k2 * M1 + k1b + c] = scale == 1.0 ? v : rf_scale(v, scale);
+    for (int e = tid; e < total; e += NT) {
+        const unsigned k2 = e >> lc, c = e & (C2 - 1);
+        const float2 v = rbuf[c * sstride + T::pad(k2)];
+        out[k2 * M1 + k1b + c] = scale == 1.0 ? v : rf_scale(v, scale);
     }
 }
 
@@ -466,12 +525,12 @@ template <int SIGN, typename... A>
 static hipError_t launch_cols(int L, dim3 grid, size_t lds, hipStream_t st, A... a)
 {
     switch (L) {
-    case 256: hipLaunchKernelGGL((k_rf_cols<SIGN, 256>), grid, dim3(RF_NT), lds, st, a...); break;
-    case 512: hipLaunchKernelGGL((k_rf_cols<SIGN, 512>), grid, dim3(RF_NT), lds, st, a...); break;
-    case 1024: hipLaunchKernelGGL((k_rf_cols<SIGN, 1024>), grid, dim3(RF_NT), lds, st, a...); break;
-    case 2048: hipLaunchKernelGGL((k_rf_cols<SIGN, 2048>), grid, dim3(RF_NT), lds, st, a...); break;
-    case 4096: hipLaunchKernelGGL((k_rf_cols<SIGN, 4096>), grid, dim3(RF_NT), lds, st, a...); break;
-    case 8192: hipLaunchKernelGGL((k_rf_cols<SIGN, 8192>), grid, dim3(RF_NT), lds, st, a...); break;
+    case 256: hipLaunchKernelGGL((k_rf_cols<SIGN, 256>), grid, dim3(RfTile<256>::NT), lds, st, a...); break;
+    case 512: hipLaunchKernelGGL((k_rf_cols<SIGN, 512>), grid, dim3(RfTile<512>::NT), lds, st, a...); break;
+    case 1024: hipLaunchKernelGGL((k_rf_cols<SIGN, 1024>), grid, dim3(RfTile<1024>::NT), lds, st, a...); break;
+    case 2048: hipLaunchKernelGGL((k_rf_cols<SIGN, 2048>), grid, dim3(RfTile<2048>::NT), lds, st, a...); break;
+    case 4096: hipLaunchKernelGGL((k_rf_cols<SIGN, 4096>), grid, dim3(RfTile<4096>::NT), lds, st, a...); break;
+    case 8192: hipLaunchKernelGGL((k_rf_cols<SIGN, 8192>), grid, dim3(RfTile<8192>::NT), lds, st, a...); break;
     default: hipLaunchKernelGGL((k_rf_cols<SIGN, 0>), grid, dim3(RF_NT), lds, st, a...); break;
     }
     return hipGetLastError();
@@ -481,12 +540,12 @@ template <int SIGN, typename... A>
 static hipError_t launch_rows(int L, dim3 grid, size_t lds, hipStream_t st, A... a)
 {
     switch (L) {
-    case 256: hipLaunchKernelGGL((k_rf_rows<SIGN, 256>), grid, dim3(RF_NT), lds, st, a...); break;
-    case 512: hipLaunchKernelGGL((k_rf_rows<SIGN, 512>), grid, dim3(RF_NT), lds, st, a...); break;
-    case 1024: hipLaunchKernelGGL((k_rf_rows<SIGN, 1024>), grid, dim3(RF_NT), lds, st, a...); break;
-    case 2048: hipLaunchKernelGGL((k_rf_rows<SIGN, 2048>), grid, dim3(RF_NT), lds, st, a...); break;
-    case 4096: hipLaunchKernelGGL((k_rf_rows<SIGN, 4096>), grid, dim3(RF_NT), lds, st, a...); break;
-    case 8192: hipLaunchKernelGGL((k_rf_rows<SIGN, 8192>), grid, dim3(RF_NT), lds, st, a...); break;
+    case 256: hipLaunchKernelGGL((k_rf_rows<SIGN, 256>), grid, dim3(RfTile<256>::NT), lds, st, a...); break;
+    case 512: hipLaunchKernelGGL((k_rf_rows<SIGN, 512>), grid, dim3(RfTile<512>::NT), lds, st, a...); break;
+    case 1024: hipLaunchKernelGGL((k_rf_rows<SIGN, 1024>), grid, dim3(RfTile<1024>::NT), lds, st, a...); break;
+    case 2048: hipLaunchKernelGGL((k_rf_rows<SIGN, 2048>), grid, dim3(RfTile<2048>::NT), lds, st, a...); break;
+    case 4096: hipLaunchKernelGGL((k_rf_rows<SIGN, 4096>), grid, dim3(RfTile<4096>::NT), lds, st, a...); break;
+    case 8192: hipLaunchKernelGGL((k_rf_rows<SIGN, 8192>), grid, dim3(RfTile<8192>::NT), lds, st, a...); break;
     default: hipLaunchKernelGGL((k_rf_rows<SIGN, 0>), grid, dim3(RF_NT), lds, st, a...); break;
     }
     return hipGetLastError();
@@ -528,13 +587,9 @@ static int realfft_enqueue(float *d_data, long long n, int nb, int isign, hipStr
     float2 *ws = buf, *tw1 = buf + (single ? 0 : M * nb), *tw2 = tw1 + M1;
     const long long toff = (tw2 + M2 - buf + 1) & ~1LL;  // 16-byte aligned (float2 units)
     double2 *tlo = (double2 *)(buf + toff), *thi = tlo + RF_TB;
-    hipLaunchKernelGGL(k_rf_twiddles, dim3((M1 + 255) / 256), dim3(256), 0, st, tw1, M1);
-    hipLaunchKernelGGL(k_rf_twiddles, dim3((M2 + 255) / 256), dim3(256), 0, st, tw2, M2);
-    if (!single) {
-        const long long nt = std::max<long long>(RF_TB, nhi);
-        hipLaunchKernelGGL(k_rf_twiddles_step, dim3((unsigned)((nt + 255) / 256)), dim3(256), 0, st, tlo, thi, M,
-                           (int)nhi);
-    }
+    const long long nt = std::max<long long>({(long long)M1, (long long)M2, nhi, single ? 0LL : (long long)RF_TB});
+    hipLaunchKernelGGL(k_rf_twiddles, dim3((unsigned)((nt + 255) / 256)), dim3(256), 0, st, tw1, M1, tw2, M2, tlo, thi, M,
+                       (int)nhi);
     PZL_HIPCHK(hipGetLastError());
     const int npairs = (int)((n >> 2) + 1);
     if (isign == 1) {
@@ -550,13 +605,14 @@ static int realfft_enqueue(float *d_data, long long n, int nb, int isign, hipStr
             hipLaunchKernelGGL(k_rf_single<1>, dim3(1, nb), dim3(RF_NT), lds, st, d, (int)M, tw1, scale);
     } else {
         const int C = per_block(M2, M1), C2 = per_block(M1, M2);
-        const size_t lds1 = sizeof(float2) * (size_t)C * (M1 + 1), lds2 = sizeof(float2) * (size_t)C2 * (M2 + 1);
+        const int lc = __builtin_ctz(C), lc2 = __builtin_ctz(C2);
+        const size_t lds1 = sizeof(float2) * (size_t)C * rf_stride(M1), lds2 = sizeof(float2) * (size_t)C2 * rf_stride(M2);
         if (isign == -1) {
-            PZL_HIPCHK(launch_cols<-1>(M1, dim3(M2 / C, nb), lds1, st, d, ws, M1, M2, C, tw1, tlo, thi));
-            PZL_HIPCHK(launch_rows<-1>(M2, dim3(M1 / C2, nb), lds2, st, ws, d, M1, M2, C2, tw2, scale));
+            PZL_HIPCHK(launch_cols<-1>(M1, dim3(M2 / C, nb), lds1, st, d, ws, M1, M2, lc, tw1, tlo, thi));
+            PZL_HIPCHK(launch_rows<-1>(M2, dim3(M1 / C2, nb), lds2, st, ws, d, M1, M2, lc2, tw2, scale));
         } else {
-            PZL_HIPCHK(launch_cols<1>(M1, dim3(M2 / C, nb), lds1, st, d, ws, M1, M2, C, tw1, tlo, thi));
-            PZL_HIPCHK(launch_rows<1>(M2, dim3(M1 / C2, nb), lds2, st, ws, d, M1, M2, C2, tw2, scale));
+            PZL_HIPCHK(launch_cols<1>(M1, dim3(M2 / C, nb), lds1, st, d, ws, M1, M2, lc, tw1, tlo, thi));
+            PZL_HIPCHK(launch_rows<1>(M2, dim3(M1 / C2, nb), lds2, st, ws, d, M1, M2, lc2, tw2, scale));
         }
     }
     PZL_HIPCHK(hipGetLastError());
