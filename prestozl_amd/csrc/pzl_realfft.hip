@@ -9,6 +9,7 @@
 //                 C adjacent columns per workgroup, times exp(SIGN 2 pi i k1 j2 / M)
 //     k_rf_rows   FFTs of length M2 along the rows, C2 rows per workgroup,
 //                 written transposed: X[k1 + M1 k2]
+//                 (k_rf_rows_split: with the forward packing step, 16-row tiles)
 //   k_rf_unpack_fwd / k_rf_pack_inv   the packing step of the forward and
 //                 inverse transform (one thread per pair of bins il, n/2 - il)
 //
@@ -356,6 +357,105 @@ __global__ __launch_bounds__(RfTile<L>::NT) void k_rf_cols(const float2 *__restr
     }
 }
 
+// The packing step of realfft's forward branch (fastffts.c:191-223) for the
+// pair a = bin il, b = bin n/2 - il (0 < il <= n/4), wr + i wi = exp(-2 pi i il / n).
+__device__ __forceinline__ void rf_split_pair(float2 a, float2 b, double wr, double wi, float2 *lo, float2 *hi)
+{
+    const double cc = -0.5;
+    const double h1r = 0.5 * ((double)a.x + b.x), h1i = 0.5 * ((double)a.y - b.y);
+    const double h2r = -cc * ((double)a.y + b.y), h2i = cc * ((double)a.x - b.x);
+    const double h2rwr = h2r * wr, h2rwi = h2r * wi, h2iwr = h2i * wr, h2iwi = h2i * wi;
+    *lo = float2{(float)(h1r + h2rwr - h2iwi), (float)(h1i + h2iwr + h2rwi)};
+    *hi = float2{(float)(h1r - h2rwr + h2iwi), (float)(-h1i + h2iwr + h2rwi)};
+}
+
+// Bin 0 of the packed spectrum: (DC, Nyquist).
+__device__ __forceinline__ float2 rf_split_zero(float2 z)
+{
+    const double t = z.x;
+    return float2{(float)(t + z.y), (float)(t - z.y)};
+}
+
+// The rows of the forward transform with the packing step in the same pass, for
+// 16 rows of a compiled length L = M2.  Bin k1 + M1 k2 pairs with bin
+// (M1 - k1) + M1 (M2 - 1 - k2), so a workgroup takes rows k1 = 8 g .. 8 g + 7
+// (slots 0 to 7) and M1 - k1 (slots 8 to 15; row 0, whose bins pair among
+// themselves, shares its slots with row M1/2, whose bins do too).
+// It saves the packing step's read and write of every bin: 564 series of 2^18
+// samples 326 + 176 us as two kernels, 358 as one.
+template <int L>
+__global__ __launch_bounds__(RfTile<L>::NT) void k_rf_rows_split(const float2 *__restrict__ in,
+                                                                 float2 *__restrict__ out, int M1,
+                                                                 const float2 *__restrict__ tw)
+{
+    extern __shared__ float2 rbuf[];
+    using T = RfTile<L>;
+    constexpr int NT = T::NT, sstride = T::pad(L) + 1;
+    static_assert(T::cmax() == 16 && NT % 8 == 0, "16 rows");
+    const int tid = threadIdx.x;
+    const unsigned k1b = 8u * (unsigned)rf_group(blockIdx.x, gridDim.x);
+    const long long M = (long long)M1 * L;
+    in += blockIdx.y * M;  // series of the batch
+    out += blockIdx.y * M;
+    for (int e0 = 0; e0 < 16 * L; e0 += RF_U * NT) {
+        float2 t[RF_U];
+#pragma unroll
+        for (int u = 0; u < RF_U; u++) {
+            const int e = e0 + u * NT + tid, s = e / L;
+            const unsigned k1 = k1b + (s & 7), row = s < 8 ? k1 : k1 == 0 ? M1 / 2 : M1 - k1;
+            t[u] = in[row * L + e % L];
+        }
+#pragma unroll
+        for (int u = 0; u < RF_U; u++) {
+            const int e = e0 + u * NT + tid;
+            rbuf[e / L * sstride + T::pad(e % L)] = t[u];
+        }
+    }
+    __syncthreads();
+    rf_fft_ct<-1, L>(rbuf, 16, sstride, tw, tid);
+    const unsigned c = tid & 7, k1 = k1b + c;
+    const float2 *qa = rbuf + c * sstride, *qb = qa + 8 * sstride;
+    if (k1 == 0) {
+        for (int k2 = tid >> 3; k2 < L; k2 += NT / 8) {
+            if (k2 < L / 2) {  // row M1/2
+                const unsigned il = M1 / 2 + M1 * k2;
+                double wi, wr;
+                sincospi(-(double)il / (double)M, &wi, &wr);
+                float2 lo, hi;
+                rf_split_pair(qb[T::pad(k2)], qb[T::pad(L - 1 - k2)], wr, wi, &lo, &hi);
+                out[il] = lo;
+                out[M1 / 2 + M1 * (L - 1 - k2)] = hi;
+            } else {  // row 0
+                const int q = k2 - L / 2, r = q ? q : L / 2;
+                if (q == 0) out[0] = rf_split_zero(qa[0]);
+                double wi, wr;
+                sincospi(-(double)(M1 * r) / (double)M, &wi, &wr);
+                float2 lo, hi;
+                rf_split_pair(qa[T::pad(r)], qa[T::pad(L - r)], wr, wi, &lo, &hi);
+                if (q) out[M1 * r] = lo;
+                out[M1 * (L - r)] = hi;
+            }
+        }
+        return;
+    }
+    // exp(-2 pi i il / n), il = k1 + M1 k2, stepped in double from row to row
+    double wr, wi, dr, di;
+    sincospi(-(double)(k1 + M1 * (tid >> 3)) / (double)M, &wi, &wr);
+    sincospi(-(double)(NT / 8) / (double)L, &di, &dr);
+#pragma unroll 2
+    for (int k2 = tid >> 3; k2 < L; k2 += NT / 8) {
+        const float2 a = qa[T::pad(k2)], b = qb[T::pad(L - 1 - k2)];
+        const bool up = k2 >= L / 2;  // the lower bin of the pair is b: exp(-2 pi i (n/2 - il) / n) = -conj
+        float2 lo, hi;
+        rf_split_pair(up ? b : a, up ? a : b, up ? -wr : wr, wi, &lo, &hi);
+        out[k1 + M1 * k2] = up ? hi : lo;
+        out[M1 - k1 + M1 * (L - 1 - k2)] = up ? lo : hi;
+        const double t = wr * dr - wi * di;
+        wi = wr * di + wi * dr;
+        wr = t;
+    }
+}
+
 // Rows k1b .. k1b + C2 - 1 of the [M1][M2] view of 'in': FFT of length M2
 // along each, element k2 of row k1 to out[k1 + M1 k2], times 'scale'.  C2 = 2^lc.
 template <int SIGN, int L>
@@ -398,10 +498,8 @@ __global__ __launch_bounds__(RfTile<L>::NT) void k_rf_rows(const float2 *__restr
     }
 }
 
-// The packing step of realfft's forward branch (fastffts.c:191-223) for the
-// pair il, ih = n/2 - il (il <= n/4), with w = exp(-2 pi i il / n); il = 0
-// sets bin 0 to (DC, Nyquist).  Where il = ih the second write is the one
-// that stays, as in the reference.
+// The packing step over a whole spectrum, one thread per pair.  Where il = ih
+// the second write is the one that stays, as in the reference.
 __global__ __launch_bounds__(256) void k_rf_unpack_fwd(float2 *__restrict__ d, long long n)
 {
     const long long il = (long long)blockIdx.x * 256 + threadIdx.x;
@@ -409,21 +507,14 @@ __global__ __launch_bounds__(256) void k_rf_unpack_fwd(float2 *__restrict__ d, l
     d += blockIdx.y * nby2;  // series of the batch
     if (il > (n >> 2)) return;
     if (il == 0) {
-        const float2 z = d[0];
-        const double t = z.x;
-        d[0] = float2{(float)(t + z.y), (float)(t - z.y)};
+        d[0] = rf_split_zero(d[0]);
         return;
     }
     const long long ih = nby2 - il;
-    const double cc = -0.5;
     double wi, wr;
     sincospi(-2.0 * (double)il / (double)n, &wi, &wr);
-    const float2 a = d[il], b = d[ih];
-    const double h1r = 0.5 * ((double)a.x + b.x), h1i = 0.5 * ((double)a.y - b.y);
-    const double h2r = -cc * ((double)a.y + b.y), h2i = cc * ((double)a.x - b.x);
-    const double h2rwr = h2r * wr, h2rwi = h2r * wi, h2iwr = h2i * wr, h2iwi = h2i * wi;
-    const float2 lo{(float)(h1r + h2rwr - h2iwi), (float)(h1i + h2iwr + h2rwi)};
-    const float2 hi{(float)(h1r - h2rwr + h2iwi), (float)(-h1i + h2iwr + h2rwi)};
+    float2 lo, hi;
+    rf_split_pair(d[il], d[ih], wr, wi, &lo, &hi);
     if (il != ih) d[il] = lo;
     d[ih] = hi;
 }
@@ -551,6 +642,23 @@ static hipError_t launch_rows(int L, dim3 grid, size_t lds, hipStream_t st, A...
     return hipGetLastError();
 }
 
+// The rows with the packing step (k_rf_rows_split), where its 16 rows make a
+// compiled tile; false (and nothing launched) for other lengths.  Longer rows
+// come 8 or 4 to a tile and would be written in pieces of 32 bytes or less.
+static bool launch_rows_split(int M1, int M2, int C2, int nb, size_t lds, hipStream_t st, const float2 *in, float2 *out,
+                              const float2 *tw)
+{
+    if (C2 != 16) return false;
+    const dim3 grid(M1 / 16, nb);
+    switch (M2) {
+    case 256: hipLaunchKernelGGL((k_rf_rows_split<256>), grid, dim3(RfTile<256>::NT), lds, st, in, out, M1, tw); break;
+    case 512: hipLaunchKernelGGL((k_rf_rows_split<512>), grid, dim3(RfTile<512>::NT), lds, st, in, out, M1, tw); break;
+    case 1024: hipLaunchKernelGGL((k_rf_rows_split<1024>), grid, dim3(RfTile<1024>::NT), lds, st, in, out, M1, tw); break;
+    default: return false;
+    }
+    return true;
+}
+
 // The workspace (float2 elements) of nb transforms of n floats: the series
 // workspace, the two FFT twiddle tables and the four-step tables (double2 = 2
 // float2).  Checks the arguments; fills M1, M2 and 'single'.
@@ -591,6 +699,7 @@ static int realfft_enqueue(float *d_data, long long n, int nb, int isign, hipStr
     hipLaunchKernelGGL(k_rf_twiddles, dim3((unsigned)((nt + 255) / 256)), dim3(256), 0, st, tw1, M1, tw2, M2, tlo, thi, M,
                        (int)nhi);
     PZL_HIPCHK(hipGetLastError());
+    bool split_done = false;
     const int npairs = (int)((n >> 2) + 1);
     if (isign == 1) {
         hipLaunchKernelGGL(k_rf_pack_inv, dim3((npairs + 255) / 256, nb), dim3(256), 0, st, d, n);
@@ -609,14 +718,16 @@ static int realfft_enqueue(float *d_data, long long n, int nb, int isign, hipStr
         const size_t lds1 = sizeof(float2) * (size_t)C * rf_stride(M1), lds2 = sizeof(float2) * (size_t)C2 * rf_stride(M2);
         if (isign == -1) {
             PZL_HIPCHK(launch_cols<-1>(M1, dim3(M2 / C, nb), lds1, st, d, ws, M1, M2, lc, tw1, tlo, thi));
-            PZL_HIPCHK(launch_rows<-1>(M2, dim3(M1 / C2, nb), lds2, st, ws, d, M1, M2, lc2, tw2, scale));
+            split_done = launch_rows_split(M1, M2, C2, nb, lds2, st, ws, d, tw2);
+            if (!split_done)
+                PZL_HIPCHK(launch_rows<-1>(M2, dim3(M1 / C2, nb), lds2, st, ws, d, M1, M2, lc2, tw2, scale));
         } else {
             PZL_HIPCHK(launch_cols<1>(M1, dim3(M2 / C, nb), lds1, st, d, ws, M1, M2, lc, tw1, tlo, thi));
             PZL_HIPCHK(launch_rows<1>(M2, dim3(M1 / C2, nb), lds2, st, ws, d, M1, M2, lc2, tw2, scale));
         }
     }
     PZL_HIPCHK(hipGetLastError());
-    if (isign == -1) {
+    if (isign == -1 && !split_done) {
         hipLaunchKernelGGL(k_rf_unpack_fwd, dim3((npairs + 255) / 256, nb), dim3(256), 0, st, d, n);
         PZL_HIPCHK(hipGetLastError());
     }

@@ -12,6 +12,7 @@ pytestmark = pytest.mark.gpu
     (256, 128),    # compiled columns, run-time rows
     (256, 243),    # an odd row count: tiles of one column
     (256, 256), (512, 256), (512, 512), (1024, 512), (1024, 1024), (2048, 1024), (2048, 2048), (4096, 2048),
+    (288, 256),    # run-time columns, compiled rows
     (1056, 1000),  # run-time passes, tiles of 8, a last partial round of threads
 ])
 def test_against_float64(M1, M2):
