@@ -151,15 +151,16 @@ int pzl_search(void *plan, long long rstep_lo, long long rstep_hi, PzlCand *cand
  * and not returned).  ms <= 0 clears the deadline. */
 int pzl_plan_set_deadline(void *plan, double ms);
 
-/* Autotuner: times every correlation-kernel variant (FFT radices, threads and
- * kernel rows per workgroup) of each FFT length of the plan on one batch of
- * its own data and keeps the fastest, for this plan and for later plans of the
- * same shape on the device.  report (optional) receives one line per variant.
+/* Autotuner: times the harmonic-sum forms on one batch of the plan's own data
+ * and the CU splits on a band of its search, and keeps the fastest, for this
+ * plan and for later plans of the same shape on the device.  The correlation is
+ * not timed: its rows-by-width launch (below) needs no choice.  report
+ * (optional) receives one line per form.
  * Replaces the reference's per-shape cuFFT plan choice (accel_kernels.cu:96-158). */
 int pzl_autotune(void *plan, int reps, char *report, int report_len);
 /* Graph replay: the correlations of every full batch of rsteps are launched
- * as one hipGraph (one per buffer set, built from the launches of the set's
- * first full batch); the batch's segments are launched before it (ahead on
+ * as one hipGraph (one per buffer set, built from the launches of the plan's
+ * full batches, also by a plan's first search); the batch's segments are launched before it (ahead on
  * their own stream, beside the previous batch's correlation, when
  * overlapped), and the harmonic sum stays a launch of its own, beside the
  * next batch.  On by
@@ -192,23 +193,27 @@ int pzl_plan_set_overlap(void *plan, int on);
  * Results do not depend on the batch size. */
 int pzl_tune_batchsize(const PzlConfig *cfg, int device, const float *host_fft, long long numbins,
                        const int *candidates, int ncand, long long band_rsteps, int *best, double *ms_per_rstep);
-/* The harmonic-sum form in use (chosen by pzl_autotune): workgroup order
+/* The harmonic-sum form in use (by a rule on the work in a batch, or chosen by
+ * pzl_autotune): workgroup order
  * (0: r chunk, z block, w fastest; 1: z block, w, r chunk fastest) and
  * consecutive fundamental r per thread (1, 2 or 4).  Results do not depend on
  * it. */
 int pzl_plan_sum_form(void *plan, int *order, int *rpt);
 int pzl_plan_set_sum_form(void *plan, int order, int rpt);
-/* Correlation launches per batch (chosen by pzl_autotune): one per FFT length
- * (group -1), or one grouped launch of correlation group 'group' for the
- * shorter lengths (all = 0; the longest keeps its own launch) or for every
- * length (all = 1: one correlation launch per batch).  A group holds one
- * kernel variant per length; it must hold every length it is given.  Results
- * do not depend on it beyond the variants' rounding. */
+/* Correlation launches per batch: one per FFT length (group -1), or one grouped
+ * launch of correlation group 'group' for the shorter lengths (all = 0; the
+ * longest keeps its own launch) or for every length (all = 1: one correlation
+ * launch per batch).  A group holds one kernel variant per length; it must hold
+ * every length it is given.  The default is the last group, whose name begins
+ * "rows by width": one launch in which each kernel row runs at the shortest
+ * transform that its own half-width allows instead of its harmonic's length.
+ * Results do not depend on the form beyond the transforms' rounding. */
 int pzl_plan_corr_group(void *plan, int *group, int *all);
 int pzl_plan_set_corr_group(void *plan, int group, int all);
 int pzl_corr_num_groups(void);
 const char *pzl_corr_group_name(int group);
-/* The variant in use for an FFT length of the plan; set one explicitly. */
+/* The variant in use for an FFT length of the plan when it has a launch of its
+ * own; setting one takes a plan from rows by width to one launch per length. */
 int pzl_plan_variant(void *plan, int fftlen, int *variant);
 int pzl_plan_set_variant(void *plan, int fftlen, int variant);
 

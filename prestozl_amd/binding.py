@@ -377,7 +377,7 @@ class Plan:
         check(lib().pzl_set_spectrum(self.h, _fptr(a), len(a) // 2))
 
     def autotune(self, reps=3):
-        """Time every correlation variant per FFT length on this plan's data and
+        """Time the harmonic-sum forms and the CU splits on this plan's data and
         keep the fastest; returns the report lines."""
         buf = C.create_string_buffer(1 << 16)
         check(lib().pzl_autotune(self.h, int(reps), buf, len(buf)))
@@ -435,7 +435,8 @@ class Plan:
         return _opt_result(arr, len(points))
 
     def fftlens(self):
-        """The FFT lengths of the plan's harmonics (one kernel variant each)."""
+        """The FFT lengths of the plan's harmonics (one kernel variant each, in
+        use when a length has a launch of its own)."""
         return sorted({h.fftlen for h in self.harms})
 
     def variant(self, fftlen):
@@ -448,7 +449,8 @@ class Plan:
 
     def corr_group(self):
         """(group, all): the correlation group of the shorter FFT lengths (all
-        False) or of every length (all True); group -1: one launch per length."""
+        False) or of every length (all True; the default, the last group: rows
+        by width); group -1: one launch per length."""
         g, a = C.c_int(0), C.c_int(0)
         check(lib().pzl_plan_corr_group(self.h, C.byref(g), C.byref(a)))
         return g.value, bool(a.value)

@@ -207,7 +207,7 @@ PlanSizes plan_sizes(const PzlConfig &cfg, const PzlGeometry &g, const std::vect
 }
 
 // The buffers a plan carves from its one device arena, in carving order
-// (pzl_plan_create assigns them in this order): harmonic tables, two sets of
+// (pzl_plan_create assigns them in this order): harmonic tables, three sets of
 // batch buffers (segments, r-index tables, harmonic r maps, planes), hit
 // slots and ordering buffers.  The sort scratch is the size the sort
 // reports for the slot capacity (a host computation, also before a plan exists).
@@ -635,8 +635,8 @@ int launch_sum_part(Plan &p, long long r0, int nb, int set, int slot, float *d_s
 
 int sync_all(Plan &p);
 
-// Drop the captured correlation graphs (they hold the variants chosen at
-// capture time): the next full batch of each set captures anew.
+// Drop the recorded correlation graphs (they hold the launch form of that
+// time): the next full batch of each set records anew.
 int drop_graphs(Plan &p)
 {
     int rc = sync_all(p);
@@ -1608,8 +1608,7 @@ int pzl_autotune(void *plan, int reps, char *report, int report_len)
     PZL_HIPCHK(hipSetDevice(p->device));
     if (reps < 1) reps = 1;
     {
-        // the variants may change below (drops the graphs), and every kernel is
-        // first timed on the whole chip
+        // every kernel is first timed on the whole chip, by launches of its own
         int grc = p->cu_split ? pzl_plan_set_cu_split(plan, 0, 0) : drop_graphs(*p);
         if (grc) return grc;
     }

@@ -1473,8 +1473,8 @@ struct CorrVariant {
 #define PZL_CVP(N, NT, G, PING, PADSH, ...)                                                                   \
     {N, launch_corr_t<N, NT, G, PING, 0, PADSH, __VA_ARGS__>,                                                 \
      #N ":" #NT "t:" #G "r:" #PING ":pad" #PADSH ":" #__VA_ARGS__}
-// Candidates per FFT length; the first of each length is the default, the
-// autotuner may pick another on the device.
+// Candidates per FFT length; the first of each length is the default of a plan
+// that launches each length by itself, pzl_plan_set_variant picks another.
 static const CorrVariant g_corr_variants[] = {
     PZL_CV(128, 128, 16, true, 16, 8),
     PZL_CV(128, 256, 16, true, 8, 4, 4),

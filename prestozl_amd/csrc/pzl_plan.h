@@ -28,7 +28,7 @@ struct SizeClass {
     std::vector<int> harms;
     std::vector<int> nrows;  // kernel rows of each harmonic (host copy for the launcher)
     int *d_harms = nullptr;
-    int variant = 0;         // correlation kernel variant (autotuned)
+    int variant = 0;         // correlation kernel variant, when the length has its own launch
 };
 
 // create_accelobs (accel_utils.c:1636-2037) + the harmonic shapes of
