@@ -22,6 +22,7 @@
 #include <deque>
 #include <thread>
 #include <cmath>
+#include <cstddef>
 #include <cstdio>
 #include <cstring>
 #include <map>
@@ -121,7 +122,7 @@ int acquire_bank(Plan *p, bool width, bool *built)
     evict_banks_locked(e.bytes);
     PZL_HIPCHK(hipMalloc(&e.ptr, e.bytes));
     hipError_t err = pzl_launch_bank_build(width ? p->d_sets : p->d_harms, (int)(width ? p->sets : p->harms).size(),
-                                           p->g.numharm_kernels, p->max_fftlen, e.ptr, p->st);
+                                           p->g.numharm_kernels, p->max_fftlen, e.ptr, 0, p->st);
     if (err == hipSuccess) err = hipStreamSynchronize(p->st);
     if (err != hipSuccess) {
         (void)hipFree(e.ptr);
@@ -2068,14 +2069,27 @@ int pzl_get_kernel(void *plan, int idx, int row, float *out)
     Plan *p = (Plan *)plan;
     if (!p || !out || idx < 0 || idx >= (int)p->harms.size() || row < 0 || row >= p->harms[idx].nrows)
         return fail(PZL_ERR_ARG, "bad kernel index");
-    const PzlHarm &H = p->harms[idx];
     PZL_HIPCHK(hipSetDevice(p->device));
-    const int brc = need_whole_bank(p);
-    if (brc) return brc;
-    PZL_HIPCHK(hipMemcpy(out, p->d_bank + H.bank_off + (long long)row * H.fftlen, sizeof(float2) * H.fftlen,
-                         hipMemcpyDeviceToHost));
-    // rows are held as K / fftlen: undo it
-    for (int k = 0; k < 2 * H.fftlen; k++) out[k] *= (float)H.fftlen;
+    // The row built by itself: a bank holds K / fftlen, which for most lengths
+    // does not scale back to the rounded K, and the searches' own bank has the
+    // row at another length.
+    struct One {
+        PzlHarm H;
+        int row;
+    } one{p->harms[idx], row};
+    const int n = one.H.fftlen;
+    char *d = nullptr;
+    const size_t head = (sizeof one + 255) / 256 * 256;
+    PZL_HIPCHK(hipMalloc(&d, head + sizeof(float2) * n));
+    one.H.nrows = 1;
+    one.H.bank_off = 0;
+    one.H.rowlist = (const int *)(d + offsetof(One, row));
+    hipError_t e = hipMemcpy(d, &one, sizeof one, hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = pzl_launch_bank_build((const PzlHarm *)d, 1, 1, n, (float2 *)(d + head), 1, p->st);
+    if (e == hipSuccess) e = hipStreamSynchronize(p->st);
+    if (e == hipSuccess) e = hipMemcpy(out, d + head, sizeof(float2) * n, hipMemcpyDeviceToHost);
+    (void)hipFree(d);
+    PZL_HIPCHK(e);
     return 0;
 }
 

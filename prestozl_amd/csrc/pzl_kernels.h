@@ -98,8 +98,10 @@ struct PzlSumArgs {
 #ifdef __cplusplus
 extern "C" {
 #endif
+// The kernel rows of nh harmonics: K / fftlen, as the correlations read them, or
+// (unit) K itself.
 hipError_t pzl_launch_bank_build(const PzlHarm *d_harms, int nh, int total_rows, int max_fftlen, float2 *d_bank,
-                                 hipStream_t st);
+                                 int unit, hipStream_t st);
 hipError_t pzl_launch_segments(const PzlBatchArgs *a, int max_fftlen, hipStream_t st);
 // Correlation of one FFT-length class with variant 'variant' (0 = default);
 // class_nrows: host copy of the kernel-row counts of the class's harmonics.

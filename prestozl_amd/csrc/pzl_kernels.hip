@@ -47,9 +47,10 @@ __device__ static int find_harm(const PzlHarm *harms, int nh, int row_global, in
     return -1;
 }
 
-// One workgroup per (harmonic, z, w) kernel.
+// One workgroup per (harmonic, z, w) kernel.  unit: as they are, without the
+// searches' scale.
 __global__ __launch_bounds__(BANK_NT) void k_bank_build(const PzlHarm *__restrict__ harms, int nh,
-                                                        float2 *__restrict__ bank)
+                                                        float2 *__restrict__ bank, int unit)
 {
     extern __shared__ double2 sbuf[];  // fftlen complex doubles
     const int tid = threadIdx.x;
@@ -83,7 +84,7 @@ __global__ __launch_bounds__(BANK_NT) void k_bank_build(const PzlHarm *__restric
     // The bank holds K / fftlen (scaled in double, rounded once): the
     // correlation's 1 / fftlen^2 power normalisation then comes out of the
     // product.
-    const double bscale = 1.0 / fftlen;
+    const double bscale = unit ? 1.0 : 1.0 / fftlen;
     float2 *out = bank + H.bank_off + (long long)row * fftlen;
     for (int k = tid; k < fftlen; k += BANK_NT)
         out[k] = float2{(float)(sbuf[k].x * bscale), (float)(sbuf[k].y * bscale)};
@@ -1217,10 +1218,10 @@ extern "C" hipError_t pzl_launch_hitprep(const long long *keys, const float *pow
 }
 
 extern "C" hipError_t pzl_launch_bank_build(const PzlHarm *d_harms, int nh, int total_rows, int max_fftlen,
-                                            float2 *d_bank, hipStream_t st)
+                                            float2 *d_bank, int unit, hipStream_t st)
 {
     const size_t smem = (size_t)max_fftlen * sizeof(double2);
-    hipLaunchKernelGGL(k_bank_build, dim3(total_rows), dim3(BANK_NT), smem, st, d_harms, nh, d_bank);
+    hipLaunchKernelGGL(k_bank_build, dim3(total_rows), dim3(BANK_NT), smem, st, d_harms, nh, d_bank, unit);
     return hipGetLastError();
 }
 

@@ -410,7 +410,7 @@ unsigned mix(unsigned long long x)
 
 extern "C" {
 
-hipError_t pzl_launch_bank_build(const PzlHarm *, int, int total_rows, int max_fftlen, float2 *d_bank,
+hipError_t pzl_launch_bank_build(const PzlHarm *, int, int total_rows, int max_fftlen, float2 *d_bank, int,
                                  hipStream_t st)
 {
     enqueue(st, [=] {
