@@ -46,7 +46,7 @@ typedef struct PzlConfig {
     double flo, fhi, rlo, rhi;
     double nph;          /* > 0: photon normalisation (-photon) */
     int batchsize;       /* rsteps per launch group (-batchsize), >= 1; above 1 a plan whose planes are
-                            small takes more (results do not depend on it) */
+                            small takes more (results do not depend on it; pzl_plan_create_launch) */
     long long maxhits;   /* hit-buffer capacity, 0 = default */
 } PzlConfig;
 
@@ -122,6 +122,12 @@ int pzl_plan_bank_built(void *plan);
 /* Geometry and the kernel bank on 'device'; the bank stays in HBM until
  * pzl_plan_destroy.  accel_utils.c:1636-2037 + create_subharminfos :236-282 */
 int pzl_plan_create(const PzlConfig *cfg, int device, void **plan);
+/* The same with exactly 'launch' rsteps per launch (at most the search's; 0: as
+ * pzl_plan_create chooses), so that a caller can bound a plan's memory;
+ * pzl_plan_launch: the plan's rsteps per launch and the size asked for (what its
+ * hit slots are sized for). */
+int pzl_plan_create_launch(const PzlConfig *cfg, int device, int launch, void **plan);
+int pzl_plan_launch(void *plan, int *launch, int *asked);
 void pzl_plan_destroy(void *plan);
 int pzl_plan_geometry(void *plan, PzlGeometry *g);
 int pzl_plan_harm(void *plan, int idx, PzlHarmInfo *h);
@@ -131,6 +137,8 @@ int pzl_plan_harm(void *plan, int idx, PzlHarmInfo *h);
  * with the sort scratch bounded before the plan exists; pzl_plan_geometry
  * reports it with the plan's actual sort scratch. */
 int pzl_geometry_from_config(const PzlConfig *cfg, PzlGeometry *g);
+/* ... of a plan made by pzl_plan_create_launch. */
+int pzl_geometry_launch(const PzlConfig *cfg, int launch, PzlGeometry *g);
 /* Device memory the plan holds: what it allocated (its spectrum once set
  * from the host included) plus its kernel bank.  accelsearch_maxsize.c:551-619 */
 int pzl_plan_device_bytes(void *plan, long long *held);

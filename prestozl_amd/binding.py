@@ -130,7 +130,10 @@ def lib():
                                              C.c_void_p, C.c_longlong]
         L.pzl_dedisperse.argtypes = [C.c_void_p, C.c_longlong, C.c_int, C.c_int, C.c_int, C.c_void_p, C.c_void_p]
         L.pzl_geometry_from_config.argtypes = [P(Config), P(Geometry)]
+        L.pzl_geometry_launch.argtypes = [P(Config), C.c_int, P(Geometry)]
         L.pzl_plan_create.argtypes = [P(Config), C.c_int, P(C.c_void_p)]
+        L.pzl_plan_create_launch.argtypes = [P(Config), C.c_int, C.c_int, P(C.c_void_p)]
+        L.pzl_plan_launch.argtypes = [C.c_void_p, P(C.c_int), P(C.c_int)]
         L.pzl_plan_destroy.argtypes = [C.c_void_p]
         L.pzl_plan_destroy.restype = None
         L.pzl_plan_geometry.argtypes = [C.c_void_p, P(Geometry)]
@@ -311,9 +314,10 @@ def bank_cache_clear():
     check(lib().pzl_bank_cache_clear())
 
 
-def geometry(cfg):
+def geometry(cfg, launch=0):
+    """The search's geometry, without a GPU; launch: as Plan's."""
     g = Geometry()
-    check(lib().pzl_geometry_from_config(C.byref(cfg), C.byref(g)))
+    check(lib().pzl_geometry_launch(C.byref(cfg), int(launch), C.byref(g)))
     return g
 
 
@@ -322,12 +326,14 @@ def _fptr(a):
 
 
 class Plan:
-    """A search plan: geometry + the kernel bank resident on one GPU."""
+    """A search plan: geometry + the kernel bank resident on one GPU.  launch:
+    exactly so many rsteps per launch (0: the plan's choice, at least the
+    configured batchsize)."""
 
-    def __init__(self, cfg, device=0):
+    def __init__(self, cfg, device=0, launch=0):
         self.cfg = cfg
         self.h = C.c_void_p()
-        check(lib().pzl_plan_create(C.byref(cfg), device, C.byref(self.h)))
+        check(lib().pzl_plan_create_launch(C.byref(cfg), device, int(launch), C.byref(self.h)))
         self.geom = Geometry()
         check(lib().pzl_plan_geometry(self.h, C.byref(self.geom)))
         self.harms = []
@@ -361,6 +367,12 @@ class Plan:
         v = C.c_longlong()
         check(lib().pzl_plan_device_bytes(self.h, C.byref(v)))
         return v.value
+
+    def launch(self):
+        """(rsteps per launch, the size asked for)."""
+        a, b = C.c_int(0), C.c_int(0)
+        check(lib().pzl_plan_launch(self.h, C.byref(a), C.byref(b)))
+        return a.value, b.value
 
     def geometry(self):
         """The plan's geometry; device_bytes carries its actual sort scratch."""

@@ -168,10 +168,12 @@ struct PlanSizes {
 int width_group() { return pzl_corr_num_groups() - 1; }
 int width_has(int n) { return pzl_corr_group_has(width_group(), n); }
 
-PlanSizes plan_sizes(const PzlConfig &cfg, const PzlGeometry &g, const std::vector<PzlHarm> &harms)
+// launch: rsteps per launch (0: by the rule below).
+PlanSizes plan_sizes(const PzlConfig &cfg, const PzlGeometry &g, const std::vector<PzlHarm> &harms, int launch)
 {
     PlanSizes z;
     z.sub = cfg.batchsize > 0 ? cfg.batchsize : 8;
+    if (launch > 0 && z.sub > launch) z.sub = launch;
     if (g.nrsteps > 0 && z.sub > g.nrsteps) z.sub = (int)g.nrsteps;
     if (z.sub < 1) z.sub = 1;
     // More rsteps per launch than asked for while a batch's planes are small:
@@ -181,8 +183,8 @@ PlanSizes plan_sizes(const PzlConfig &cfg, const PzlGeometry &g, const std::vect
     // row is read once per batch.  Measured on MI355X, per search, at 8 and at the
     // rule's count: 540 rsteps of 0.3 MB 4.3 -> 0.42 ms (512), 1117 of 1.3 MB 7.9 ->
     // 1.5 ms (512), 182 of 92 MB 12.9 -> 11.5 ms (32).
-    z.B = z.sub;
-    while (z.sub > 1 && z.B < kMaxBatch && z.B < g.nrsteps &&
+    z.B = launch > 0 ? (int)std::max<long long>(1, std::min<long long>(launch, g.nrsteps)) : z.sub;
+    while (launch <= 0 && z.sub > 1 && z.B < kMaxBatch && z.B < g.nrsteps &&
            (long long)z.B * g.plane_bytes_per_rstep < (z.B < 32 ? kBatchPlanesMost : kBatchPlanes))
         z.B = (int)std::min<long long>({2LL * z.B, kMaxBatch, g.nrsteps});
     const PzlHarm &F = harms[0];
@@ -1077,13 +1079,15 @@ int pzl_device_memory(int device, long long *free_bytes, long long *total_bytes)
     return 0;
 }
 
-int pzl_geometry_from_config(const PzlConfig *cfg, PzlGeometry *g)
+int pzl_geometry_from_config(const PzlConfig *cfg, PzlGeometry *g) { return pzl_geometry_launch(cfg, 0, g); }
+
+int pzl_geometry_launch(const PzlConfig *cfg, int launch, PzlGeometry *g)
 {
-    if (!cfg || !g) return fail(PZL_ERR_ARG, "null argument");
+    if (!cfg || !g || launch < 0) return fail(PZL_ERR_ARG, "bad arguments");
     std::vector<PzlHarm> harms;
     int rc = compute_geometry(*cfg, *g, &harms, nullptr);
     if (rc) return rc;
-    const PlanSizes z = plan_sizes(*cfg, *g, harms);
+    const PlanSizes z = plan_sizes(*cfg, *g, harms, launch);
     g->device_bytes = plan_device_bytes(*g, z, harms, -1);
     if (!z.sets.empty()) g->bank_bytes = z.wbank_bytes;
     return 0;
@@ -1091,7 +1095,12 @@ int pzl_geometry_from_config(const PzlConfig *cfg, PzlGeometry *g)
 
 int pzl_plan_create(const PzlConfig *cfg, int device, void **plan_out)
 {
-    if (!cfg || !plan_out) return fail(PZL_ERR_ARG, "null argument");
+    return pzl_plan_create_launch(cfg, device, 0, plan_out);
+}
+
+int pzl_plan_create_launch(const PzlConfig *cfg, int device, int launch, void **plan_out)
+{
+    if (!cfg || !plan_out || launch < 0) return fail(PZL_ERR_ARG, "bad arguments");
     *plan_out = nullptr;
     Plan *p = new Plan();
     p->cfg = *cfg;
@@ -1115,7 +1124,7 @@ int pzl_plan_create(const PzlConfig *cfg, int device, void **plan_out)
         p->max_fftlen = std::max(p->max_fftlen, H.fftlen);
     }
     for (int s = 0; s < p->g.numharmstages; s++) p->numindep_d[s] = (double)p->g.numindep[s];
-    const PlanSizes sizes = plan_sizes(*cfg, p->g, p->harms);
+    const PlanSizes sizes = plan_sizes(*cfg, p->g, p->harms, launch);
     p->B = sizes.B;
     p->sub_batch = sizes.sub;
     const int nh = (int)p->harms.size();
@@ -1367,6 +1376,15 @@ int pzl_plan_device_bytes(void *plan, long long *held)
     Plan *p = (Plan *)plan;
     if (!p || !held) return fail(PZL_ERR_ARG, "null argument");
     *held = p->dev_bytes + (p->d_bank ? p->bank_bytes : 0) + (p->d_wbank ? p->wbank_bytes : 0);
+    return 0;
+}
+
+int pzl_plan_launch(void *plan, int *launch, int *asked)
+{
+    Plan *p = (Plan *)plan;
+    if (!p) return fail(PZL_ERR_ARG, "null plan");
+    if (launch) *launch = p->B;
+    if (asked) *asked = p->sub_batch;
     return 0;
 }
 

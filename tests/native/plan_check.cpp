@@ -1,0 +1,145 @@
+// Checks of a plan's sizes and of what its searches launch, built with g++
+// against the HIP runtime stand-in (hipstub).  One check per run, named by the
+// first argument; exit status 0 when it holds.  Test infrastructure only.
+#include <hip/hip_runtime.h>
+
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <string>
+#include <vector>
+
+#include "pzl_accel.h"
+
+namespace {
+
+int bad = 0;
+
+#define EXPECT(cond, ...)                                     \
+    do {                                                      \
+        if (!(cond)) {                                        \
+            bad++;                                            \
+            fprintf(stderr, "line %d: %s: ", __LINE__, #cond); \
+            fprintf(stderr, __VA_ARGS__);                     \
+            fprintf(stderr, "\n");                            \
+        }                                                     \
+    } while (0)
+
+PzlConfig config(double N, int zmax, int wmax, int numharm, int batchsize)
+{
+    PzlConfig c;
+    memset(&c, 0, sizeof c);
+    c.N = N;
+    c.dt = 1e-4;
+    c.numbins = (long long)N / 2;
+    c.zmax = zmax;
+    c.wmax = wmax;
+    c.wmaxP = wmax > 0;
+    c.numharm = numharm;
+    c.sigma = 3.0f;
+    c.floP = 1;
+    c.flo = 1.0;
+    c.fhiP = 1;
+    c.fhi = 1e4;
+    c.batchsize = batchsize;
+    return c;
+}
+
+void ok(int rc)
+{
+    if (rc == 0) return;
+    fprintf(stderr, "call failed: %s\n", pzl_last_error());
+    exit(2);
+}
+
+struct Plan {
+    void *h = nullptr;
+    PzlConfig c;
+    Plan(const PzlConfig &cfg, int launch = 0) : c(cfg)
+    {
+        ok(pzl_plan_create_launch(&c, 0, launch, &h));
+        ok(pzl_set_spectrum_device(h, spectrum().data(), c.numbins));
+    }
+    ~Plan() { pzl_plan_destroy(h); }
+    static std::vector<float> &spectrum()
+    {
+        static std::vector<float> f(1 << 22, 1.0f);
+        return f;
+    }
+    int launch() const
+    {
+        int n = 0;
+        ok(pzl_plan_launch(h, &n, nullptr));
+        return n;
+    }
+    int asked() const
+    {
+        int n = 0;
+        ok(pzl_plan_launch(h, nullptr, &n));
+        return n;
+    }
+    std::vector<PzlCand> search(PzlStats *st = nullptr)
+    {
+        long long n = 0;
+        ok(pzl_search(h, 0, -1, nullptr, 0, &n, st));
+        return cands(n);
+    }
+    std::vector<PzlCand> cands(long long n)
+    {
+        std::vector<PzlCand> v((size_t)n);
+        ok(pzl_get_cands(h, v.data(), n, &n));
+        return v;
+    }
+};
+
+bool same(const std::vector<PzlCand> &a, const std::vector<PzlCand> &b)
+{
+    if (a.size() != b.size()) return false;
+    for (size_t i = 0; i < a.size(); i++)
+        if (a[i].power != b[i].power || a[i].sigma != b[i].sigma || a[i].numharm != b[i].numharm ||
+            a[i].r != b[i].r || a[i].z != b[i].z || a[i].w != b[i].w)
+            return false;
+    return true;
+}
+
+// A plan of a given launch size launches by it, holds what the model says, and
+// gives the same candidates as any other.
+void exact()
+{
+    const PzlConfig c = config(1 << 18, 8, 0, 2, 8);
+    std::vector<PzlCand> ref;
+    PzlGeometry g;
+    ok(pzl_geometry_from_config(&c, &g));
+    for (int b : {1, 3, 8, 20, 1 << 20}) {
+        const int want = (int)std::min<long long>(b, g.nrsteps);
+        Plan p(c, b);
+        EXPECT(p.launch() == want && p.asked() == std::min(want, 8), "%d: %d, %d", b, p.launch(), p.asked());
+        PzlStats st;
+        const auto v = p.search(&st);
+        EXPECT(st.corr_launches == (g.nrsteps + want - 1) / want, "%d: %lld launches", b, st.corr_launches);
+        if (ref.empty()) ref = v;
+        EXPECT(!v.empty() && same(v, ref), "%d: %zu candidates", b, v.size());
+        PzlGeometry gl;
+        ok(pzl_geometry_launch(&c, b, &gl));
+        long long held = 0;
+        ok(pzl_plan_device_bytes(p.h, &held));
+        EXPECT(held + (long long)sizeof(float2) * c.numbins == gl.device_bytes, "%d: %lld, model %lld", b, held,
+               gl.device_bytes);  // the spectrum is the caller's
+    }
+    Plan p(c);
+    EXPECT(p.launch() > 8 && p.asked() == 8 && same(p.search(), ref), "%d", p.launch());
+}
+
+}  // namespace
+
+int main(int argc, char **argv)
+{
+    const std::string name = argc > 1 ? argv[1] : "";
+    if (name == "exact") exact();
+    else {
+        fprintf(stderr, "no check '%s'\n", name.c_str());
+        return 2;
+    }
+    printf("%s: %s\n", name.c_str(), bad ? "FAILED" : "OK");
+    return bad ? 1 : 0;
+}
