@@ -45,8 +45,9 @@ typedef struct PzlConfig {
     int floP, fhiP, rloP, rhiP;
     double flo, fhi, rlo, rhi;
     double nph;          /* > 0: photon normalisation (-photon) */
-    int batchsize;       /* rsteps per launch group (-batchsize), >= 1; above 1 a plan whose planes are
-                            small takes more (results do not depend on it; pzl_plan_create_launch) */
+    int batchsize;       /* rsteps per launch group (-batchsize), >= 1; above 1 a plan doubles it while a
+                            group's planes stay within 512 MiB and 512 rsteps (from 8 on also within 3 GiB
+                            below 32 rsteps); results do not depend on it; pzl_plan_create_launch */
     long long maxhits;   /* hit-buffer capacity, 0 = default */
 } PzlConfig;
 

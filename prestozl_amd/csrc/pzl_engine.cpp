@@ -146,9 +146,47 @@ int need_whole_bank(Plan *p)
     return rc;
 }
 
-constexpr int kMaxBatch = 512;  // rsteps per launch the rule below goes up to
-// bytes of planes per batch it aims for; up to 32 rsteps
-constexpr long long kBatchPlanes = 512LL << 20, kBatchPlanesMost = 2LL << 30;
+// The most that the rule of launch_sizes goes up to: rsteps per launch and bytes
+// of planes per batch, and, for requests of at least the default batchsize, the
+// same of batches with large planes.
+constexpr int kDefaultBatch = 8, kMaxBatch = 512, kMaxBatchLarge = 32;
+constexpr long long kBatchPlanes = 512LL << 20, kBatchPlanesLarge = 3LL << 30;
+
+// Rsteps per launch of a request.
+struct LaunchSizes {
+    int asked;  // as configured
+    int small;  // raised while the planes are small
+    int large;  // ... and, of these, while they are large
+};
+
+// More rsteps per launch than asked for while a batch's planes stay small: a short
+// search then fills the chip and does not pay per batch for its launches, its
+// count's way to the host and its sort.  Up to 32 rsteps also while the planes are
+// large, as each kernel row is read once per batch; not where fewer than the
+// default of 8 are asked for, which bounds the plan's memory.  One rstep per launch
+// stays one.  Measured on MI355X, ms per search: 540 rsteps of 0.3 MiB: 8 per
+// launch 5.64, 270 0.54, 512 0.46; 1117 of 1.2 MiB: 8 8.9, 128 1.52, 256 1.46, 512
+// 1.46; 182 of 88 MiB: 8 12.7, 16 11.7, 32 11.1; 2920 of 157 MiB: 8 532, 16 462
+// (13 and 19: 483 and 487, so sizes are doubled and not filled up to the limit).
+LaunchSizes launch_sizes(const PzlConfig &cfg, const PzlGeometry &g)
+{
+    LaunchSizes s;
+    s.asked = cfg.batchsize > 0 ? cfg.batchsize : kDefaultBatch;
+    if (g.nrsteps > 0 && s.asked > g.nrsteps) s.asked = (int)g.nrsteps;
+    if (s.asked < 1) s.asked = 1;
+    auto raise = [&](int n, int most, long long planes) {
+        while (n < most && n < g.nrsteps) {
+            const int next = (int)std::min<long long>({2LL * n, kMaxBatch, g.nrsteps});
+            if (next * g.plane_bytes_per_rstep > planes) break;
+            n = next;
+        }
+        return n;
+    };
+    s.small = s.asked > 1 ? raise(s.asked, kMaxBatch, kBatchPlanes) : 1;
+    s.large = cfg.batchsize <= 0 || cfg.batchsize >= kDefaultBatch ? raise(s.small, kMaxBatchLarge, kBatchPlanesLarge)
+                                                                   : s.small;
+    return s;
+}
 
 // Batch size, hit-slot capacity and slot count of a plan (pzl_plan_create
 // uses them; the request loop uses them to size a request before admission).
@@ -168,25 +206,13 @@ struct PlanSizes {
 int width_group() { return pzl_corr_num_groups() - 1; }
 int width_has(int n) { return pzl_corr_group_has(width_group(), n); }
 
-// launch: rsteps per launch (0: by the rule below).
+// launch: rsteps per launch (0: by the rule above).
 PlanSizes plan_sizes(const PzlConfig &cfg, const PzlGeometry &g, const std::vector<PzlHarm> &harms, int launch)
 {
     PlanSizes z;
-    z.sub = cfg.batchsize > 0 ? cfg.batchsize : 8;
-    if (launch > 0 && z.sub > launch) z.sub = launch;
-    if (g.nrsteps > 0 && z.sub > g.nrsteps) z.sub = (int)g.nrsteps;
-    if (z.sub < 1) z.sub = 1;
-    // More rsteps per launch than asked for while a batch's planes are small:
-    // a short search then fills the chip and does not pay per batch for its
-    // launches, its count's way to the host and its sort.  (One rstep per launch
-    // stays one.)  Up to 32 rsteps also while the planes are large, as each kernel
-    // row is read once per batch.  Measured on MI355X, per search, at 8 and at the
-    // rule's count: 540 rsteps of 0.3 MB 4.3 -> 0.42 ms (512), 1117 of 1.3 MB 7.9 ->
-    // 1.5 ms (512), 182 of 92 MB 12.9 -> 11.5 ms (32).
-    z.B = launch > 0 ? (int)std::max<long long>(1, std::min<long long>(launch, g.nrsteps)) : z.sub;
-    while (launch <= 0 && z.sub > 1 && z.B < kMaxBatch && z.B < g.nrsteps &&
-           (long long)z.B * g.plane_bytes_per_rstep < (z.B < 32 ? kBatchPlanesMost : kBatchPlanes))
-        z.B = (int)std::min<long long>({2LL * z.B, kMaxBatch, g.nrsteps});
+    const LaunchSizes ls = launch_sizes(cfg, g);
+    z.B = launch > 0 ? (int)std::max<long long>(1, std::min<long long>(launch, g.nrsteps)) : ls.large;
+    z.sub = std::min(ls.asked, z.B);
     const PzlHarm &F = harms[0];
     // one rstep can never overflow a slot
     const long long per_rstep = (long long)g.corr_uselen * F.numz * F.numw * g.numharmstages;

@@ -3,6 +3,7 @@
 // first argument; exit status 0 when it holds.  Test infrastructure only.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -130,12 +131,57 @@ void exact()
     EXPECT(p.launch() > 8 && p.asked() == 8 && same(p.search(), ref), "%d", p.launch());
 }
 
+// The rule's launch sizes: within their limits on the bytes of planes, 1 as
+// asked, and fewer than the default of 8 raised only while the planes are small.
+void rule()
+{
+    struct Shape {
+        double N;
+        int zmax, wmax, numharm;
+        std::vector<std::pair<int, int>> want;  // asked, launched
+    };
+    const std::vector<Shape> shapes = {
+        {1 << 20, 20, 0, 4, {{8, 512}, {3, 512}, {700, 700}}},       // 0.3 MiB, 540 rsteps
+        {1 << 21, 50, 0, 8, {{0, 256}, {8, 256}, {4, 256}}},         // 1.2 MiB
+        {1 << 18, 200, 300, 8, {{8, 32}, {4, 4}, {2, 4}, {64, 64}}}, // 88 MiB
+        {1 << 22, 200, 300, 16, {{8, 16}, {16, 16}, {7, 7}, {2, 2}}}, // 157 MiB
+        {1 << 20, 200, 500, 16, {{8, 8}, {2, 2}}},                   // 612 MiB
+    };
+    for (const Shape &s : shapes) {
+        auto made = [&](int asked, long long *planes, long long *nr) {
+            const PzlConfig c = config(s.N, s.zmax, s.wmax, s.numharm, asked);
+            Plan p(c);
+            PzlGeometry g;
+            ok(pzl_plan_geometry(p.h, &g));
+            *planes = p.launch() * g.plane_bytes_per_rstep;
+            *nr = g.nrsteps;
+            return p.launch();
+        };
+        long long planes, nr;
+        for (auto w : s.want) {
+            const int n = made(w.first, &planes, &nr);
+            EXPECT(n == std::min<long long>(w.second, nr), "(%d, %d, %d) at %d: %d", s.zmax, s.wmax, s.numharm, w.first, n);
+        }
+        PzlGeometry g;
+        const PzlConfig c = config(s.N, s.zmax, s.wmax, s.numharm, 8);
+        ok(pzl_geometry_from_config(&c, &g));
+        for (int asked : {1, 2, 3, 5, 7, 8, 12, 24, 40, 100}) {
+            if (asked * g.plane_bytes_per_rstep > (5LL << 30)) break;  // what this machine's memory takes
+            const int n = made(asked, &planes, &nr);
+            const bool fits = planes <= (512LL << 20) || (asked >= 8 && planes <= (3LL << 30) && n < 64);
+            EXPECT(n == std::min<long long>(asked, nr) || (asked > 1 && n > asked && n <= 512 && fits),
+                   "(%d, %d, %d) at %d: %d, %lld bytes", s.zmax, s.wmax, s.numharm, asked, n, planes);
+        }
+    }
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
 {
     const std::string name = argc > 1 ? argv[1] : "";
     if (name == "exact") exact();
+    else if (name == "rule") rule();
     else {
         fprintf(stderr, "no check '%s'\n", name.c_str());
         return 2;
