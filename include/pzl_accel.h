@@ -121,7 +121,9 @@ int pzl_bank_cache_clear(void);
 int pzl_plan_bank_built(void *plan);
 
 /* Geometry and the kernel bank on 'device'; the bank stays in HBM until
- * pzl_plan_destroy.  accel_utils.c:1636-2037 + create_subharminfos :236-282 */
+ * pzl_plan_destroy.  accel_utils.c:1636-2037 + create_subharminfos :236-282.
+ * Rsteps per launch above the batchsize asked for are given up where the plan
+ * would take more than a quarter of the free device memory or cannot be made. */
 int pzl_plan_create(const PzlConfig *cfg, int device, void **plan);
 /* The same with exactly 'launch' rsteps per launch (at most the search's; 0: as
  * pzl_plan_create chooses), so that a caller can bound a plan's memory;

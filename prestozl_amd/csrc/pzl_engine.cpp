@@ -207,9 +207,8 @@ int width_group() { return pzl_corr_num_groups() - 1; }
 int width_has(int n) { return pzl_corr_group_has(width_group(), n); }
 
 // launch: rsteps per launch (0: by the rule above).
-PlanSizes plan_sizes(const PzlConfig &cfg, const PzlGeometry &g, const std::vector<PzlHarm> &harms, int launch)
+void size_launch(PlanSizes &z, const PzlConfig &cfg, const PzlGeometry &g, const std::vector<PzlHarm> &harms, int launch)
 {
-    PlanSizes z;
     const LaunchSizes ls = launch_sizes(cfg, g);
     z.B = launch > 0 ? (int)std::max<long long>(1, std::min<long long>(launch, g.nrsteps)) : ls.large;
     z.sub = std::min(ls.asked, z.B);
@@ -221,6 +220,12 @@ PlanSizes plan_sizes(const PzlConfig &cfg, const PzlGeometry &g, const std::vect
     z.hitcap = std::max<long long>(cap, per_rstep);
     const long long nbatches = (g.nrsteps + z.B - 1) / z.B;
     z.nslots = (int)std::max<long long>(1, std::min<long long>(Plan::kSlots, nbatches));
+}
+
+PlanSizes plan_sizes(const PzlConfig &cfg, const PzlGeometry &g, const std::vector<PzlHarm> &harms, int launch)
+{
+    PlanSizes z;
+    size_launch(z, cfg, g, harms, launch);
     z.seg_stride = 0;
     for (auto &H : harms) z.seg_stride += H.fftlen / 2;
     z.set_seg_stride = z.wbank_bytes = 0;
@@ -291,6 +296,24 @@ long long plan_device_bytes(const PzlGeometry &g, const PlanSizes &z, const std:
                             long long sort_temp)
 {
     return (z.sets.empty() ? g.bank_bytes : z.wbank_bytes) + (long long)sizeof(float2) * g.numbins + arena_bytes(plan_arena_items(g, z, harms, sort_temp));
+}
+
+// The largest launch size of the rule whose plan takes at most a quarter of the
+// device memory that is free now (the raise is for speed only, and what else the
+// process needs is not known here); the size asked for however much that takes.
+int fit_launch(PlanSizes &z, const PzlConfig &cfg, const PzlGeometry &g, const std::vector<PzlHarm> &harms)
+{
+    const LaunchSizes ls = launch_sizes(cfg, g);
+    if (ls.large > ls.asked) {
+        size_t free_b = 0, total_b = 0;
+        PZL_HIPCHK(hipMemGetInfo(&free_b, &total_b));
+        for (int n : {ls.large, ls.small}) {
+            size_launch(z, cfg, g, harms, n);
+            if (n > ls.asked && plan_device_bytes(g, z, harms, -1) <= (long long)(free_b / 4)) return 0;
+        }
+    }
+    size_launch(z, cfg, g, harms, ls.asked);
+    return 0;
 }
 
 // hipMalloc of a plan-owned buffer, counted in p->dev_bytes
@@ -1124,10 +1147,25 @@ int pzl_plan_create(const PzlConfig *cfg, int device, void **plan_out)
     return pzl_plan_create_launch(cfg, device, 0, plan_out);
 }
 
+static int make_plan(const PzlConfig *cfg, int device, int launch, void **plan_out, int *retry);
+
 int pzl_plan_create_launch(const PzlConfig *cfg, int device, int launch, void **plan_out)
 {
     if (!cfg || !plan_out || launch < 0) return fail(PZL_ERR_ARG, "bad arguments");
+    int retry = 0;  // a raised plan that could not be made: the size asked for
+    int rc = make_plan(cfg, device, launch, plan_out, &retry);
+    if (rc == PZL_ERR_HIP && retry) {
+        (void)hipGetLastError();
+        g_err.clear();
+        rc = make_plan(cfg, device, retry, plan_out, &retry);
+    }
+    return rc;
+}
+
+static int make_plan(const PzlConfig *cfg, int device, int launch, void **plan_out, int *retry)
+{
     *plan_out = nullptr;
+    *retry = 0;
     Plan *p = new Plan();
     p->cfg = *cfg;
     p->device = device;
@@ -1150,7 +1188,17 @@ int pzl_plan_create_launch(const PzlConfig *cfg, int device, int launch, void **
         p->max_fftlen = std::max(p->max_fftlen, H.fftlen);
     }
     for (int s = 0; s < p->g.numharmstages; s++) p->numindep_d[s] = (double)p->g.numindep[s];
-    const PlanSizes sizes = plan_sizes(*cfg, p->g, p->harms, launch);
+    PlanSizes sizes = plan_sizes(*cfg, p->g, p->harms, launch);
+    if (launch == 0) {
+        hipError_t e = hipSetDevice(device);
+        rc = e == hipSuccess ? fit_launch(sizes, *cfg, p->g, p->harms)
+                             : fail(PZL_ERR_HIP, "hipSetDevice(device) failed: %s", hipGetErrorString(e));
+        if (rc) {
+            delete p;
+            return rc;
+        }
+        if (sizes.B > sizes.sub) *retry = sizes.sub;
+    }
     p->B = sizes.B;
     p->sub_batch = sizes.sub;
     const int nh = (int)p->harms.size();

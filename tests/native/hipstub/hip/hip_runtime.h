@@ -118,3 +118,5 @@ template <typename T> inline hipError_t hipHostMalloc(T **p, size_t n, unsigned 
 
 // Stand-in bookkeeping the stress driver checks: bytes held by hipMalloc.
 long long hipstub_device_bytes();
+// Device memory that hipMemGetInfo counts from, and that hipMalloc gives out.
+void hipstub_set_memory(long long reported, long long available);

@@ -97,6 +97,7 @@ std::set<StubStream *> g_streams;
 std::mutex g_mem_mu;
 std::map<void *, size_t> g_dev;
 long long g_dev_bytes = 0;
+long long g_reported = 288ll << 30, g_available = 288ll << 30;
 
 // Run f on the stream, or now when the stream is the null stream; a stream
 // being captured records f into its graph instead.
@@ -166,7 +167,7 @@ hipError_t hipMemGetInfo(size_t *free_b, size_t *total_b)
 {
     std::lock_guard<std::mutex> lk(g_mem_mu);
     *total_b = 288ull << 30;
-    *free_b = *total_b - (size_t)g_dev_bytes;
+    *free_b = (size_t)std::max(0ll, g_reported - g_dev_bytes);
     return hipSuccess;
 }
 long long hipstub_device_bytes()
@@ -174,8 +175,18 @@ long long hipstub_device_bytes()
     std::lock_guard<std::mutex> lk(g_mem_mu);
     return g_dev_bytes;
 }
+void hipstub_set_memory(long long reported, long long available)
+{
+    std::lock_guard<std::mutex> lk(g_mem_mu);
+    g_reported = reported;
+    g_available = available;
+}
 hipError_t hipMalloc(void **p, size_t n)
 {
+    {
+        std::lock_guard<std::mutex> lk(g_mem_mu);
+        if (g_dev_bytes + (long long)n > g_available) return hipErrorOutOfMemory;
+    }
     *p = aligned_alloc(256, (n + 255) / 256 * 256);
     if (!*p) return hipErrorOutOfMemory;
     std::lock_guard<std::mutex> lk(g_mem_mu);

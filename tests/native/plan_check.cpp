@@ -175,6 +175,43 @@ void rule()
     }
 }
 
+// Where the device's memory is short a plan is made at the size asked for, by what
+// is reported free or after an allocation that failed.
+void memory()
+{
+    const PzlConfig c = config(1 << 21, 50, 0, 8, 8);
+    PzlGeometry full, least;
+    ok(pzl_geometry_from_config(&c, &full));
+    ok(pzl_geometry_launch(&c, 8, &least));
+    EXPECT(full.device_bytes > 3 * least.device_bytes, "%lld, %lld", full.device_bytes, least.device_bytes);
+    const long long all = 288LL << 30;
+    std::vector<PzlCand> ref;
+    const struct {
+        long long reported, available;
+        bool raised;
+    } cases[] = {{all, all, true},
+                 {4 * full.device_bytes, all, true},
+                 {4 * full.device_bytes - 1, all, false},
+                 {all, full.device_bytes / 2, false},
+                 {least.device_bytes, least.device_bytes, false}};
+    for (auto &k : cases) {
+        ok(pzl_bank_cache_clear());
+        hipstub_set_memory(k.reported, k.available);
+        Plan p(c);
+        EXPECT(p.asked() == 8 && (p.launch() > 8) == k.raised, "%lld, %lld: %d", k.reported, k.available, p.launch());
+        const auto v = p.search();
+        if (ref.empty()) ref = v;
+        EXPECT(!v.empty() && same(v, ref), "%zu candidates", v.size());
+        EXPECT(pzl_last_error()[0] == 0, "%s", pzl_last_error());
+    }
+    ok(pzl_bank_cache_clear());
+    hipstub_set_memory(all, least.device_bytes / 2);
+    void *h = nullptr;
+    EXPECT(pzl_plan_create(&c, 0, &h) == PZL_ERR_HIP && !h, "%p", h);
+    hipstub_set_memory(all, all);
+    EXPECT(hipstub_device_bytes() == 0, "%lld bytes held", hipstub_device_bytes());
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
@@ -182,6 +219,7 @@ int main(int argc, char **argv)
     const std::string name = argc > 1 ? argv[1] : "";
     if (name == "exact") exact();
     else if (name == "rule") rule();
+    else if (name == "memory") memory();
     else {
         fprintf(stderr, "no check '%s'\n", name.c_str());
         return 2;
