@@ -334,7 +334,10 @@ typedef struct PzlServerStats {
 
 /* A request is admitted by its footprint: the geometry's device_bytes plus
  * PZL_RUNTIME_BYTES_PER_SEARCH for the HIP runtime's own memory behind a
- * plan's streams (measured at most 27 MiB on MI355X).
+ * plan's streams (measured at most 27 MiB on MI355X).  Rsteps per launch above
+ * the request's batchsize are given up where the budget is short: up to 512 MiB
+ * of planes where the footprint exceeds the budget, more where it exceeds the
+ * budget over max_inflight.
  * hbm_budget <= 0: 80% of the device's free memory. */
 #define PZL_RUNTIME_BYTES_PER_SEARCH (32LL << 20)
 int pzl_server_create(int device, long long hbm_budget, int max_inflight, void **server);

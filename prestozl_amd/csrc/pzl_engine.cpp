@@ -152,13 +152,6 @@ int need_whole_bank(Plan *p)
 constexpr int kDefaultBatch = 8, kMaxBatch = 512, kMaxBatchLarge = 32;
 constexpr long long kBatchPlanes = 512LL << 20, kBatchPlanesLarge = 3LL << 30;
 
-// Rsteps per launch of a request.
-struct LaunchSizes {
-    int asked;  // as configured
-    int small;  // raised while the planes are small
-    int large;  // ... and, of these, while they are large
-};
-
 // More rsteps per launch than asked for while a batch's planes stay small: a short
 // search then fills the chip and does not pay per batch for its launches, its
 // count's way to the host and its sort.  Up to 32 rsteps also while the planes are
@@ -168,7 +161,7 @@ struct LaunchSizes {
 // launch 5.64, 270 0.54, 512 0.46; 1117 of 1.2 MiB: 8 8.9, 128 1.52, 256 1.46, 512
 // 1.46; 182 of 88 MiB: 8 12.7, 16 11.7, 32 11.1; 2920 of 157 MiB: 8 532, 16 462
 // (13 and 19: 483 and 487, so sizes are doubled and not filled up to the limit).
-LaunchSizes launch_sizes(const PzlConfig &cfg, const PzlGeometry &g)
+pzl::LaunchSizes launch_sizes(const PzlConfig &cfg, const PzlGeometry &g)
 {
     LaunchSizes s;
     s.asked = cfg.batchsize > 0 ? cfg.batchsize : kDefaultBatch;
@@ -1081,6 +1074,15 @@ double plane_alg_bytes(const Plan &p)
 }
 
 }  // namespace
+
+int pzl::launch_sizes_of(const PzlConfig &cfg, LaunchSizes *s)
+{
+    PzlGeometry g;
+    std::vector<PzlHarm> harms;
+    const int rc = compute_geometry(cfg, g, &harms, nullptr);
+    if (rc == 0) *s = launch_sizes(cfg, g);
+    return rc;
+}
 
 // ---------------------------------------------------------------------------
 // C ABI

@@ -46,6 +46,14 @@ bool compute_row_sets(const std::vector<PzlHarm> &harms, int corr_uselen, int (*
 
 int reserve_pinned_chunks(int count);  // pzl_engine.cpp
 
+// Rsteps per launch of a request (pzl_engine.cpp).
+struct LaunchSizes {
+    int asked;  // as configured
+    int small;  // raised while the planes are small
+    int large;  // ... and, of these, while they are large
+};
+int launch_sizes_of(const PzlConfig &cfg, LaunchSizes *s);
+
 struct Plan {
     PzlConfig cfg{};
     PzlGeometry g{};

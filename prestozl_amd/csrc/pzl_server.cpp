@@ -69,6 +69,7 @@ struct Request {
     bool on_device = false;      // fft is device memory of the server's device
     long long numbins = 0;
     long long footprint = 0;
+    int launch = 0, asked = 0;  // rsteps per launch of its plan; as configured
     double cells = 0;
     Clock::time_point t_submit, t_admit, t_end;
     bool has_deadline = false;
@@ -201,7 +202,9 @@ struct Server {
             }
             int rc = 0;
             if (!plan) {
-                rc = pzl_plan_create(&r->cfg, device, &plan);
+                rc = pzl_plan_create_launch(&r->cfg, device, r->launch, &plan);
+                if (rc == PZL_ERR_HIP && r->launch > r->asked)
+                    rc = pzl_plan_create_launch(&r->cfg, device, r->asked, &plan);
                 // a request gives its candidates only: its hits (32 bytes each, up to
                 // millions) are not kept
                 if (rc == 0) rc = pzl_plan_set_keep_hits(plan, 0);
@@ -303,9 +306,22 @@ static int submit(void *srv, const PzlConfig *cfg, const float *fft, bool on_dev
 {
     Server *s = (Server *)srv;
     if (!s || !cfg || !fft || numbins <= 0) return fail(PZL_ERR_ARG, "bad request");
-    PzlGeometry g;
-    int rc = pzl_geometry_from_config(cfg, &g);
+    LaunchSizes ls;
+    int rc = launch_sizes_of(*cfg, &ls);
     if (rc) return rc;
+    // Raised rsteps per launch as far as the budget allows: with large planes a
+    // request stays within its share, so that as many run at once as at the size
+    // asked for; with small ones (at most 1.5 GiB more) within the budget.
+    PzlGeometry g;
+    int launch = 0;
+    for (int n : {ls.large, ls.small, ls.asked}) {
+        if (n == launch) continue;
+        launch = n;
+        rc = pzl_geometry_launch(cfg, n, &g);
+        if (rc) return rc;
+        const long long need = g.device_bytes + PZL_RUNTIME_BYTES_PER_SEARCH;
+        if (need <= (n > ls.small ? s->budget / s->max_inflight : s->budget)) break;
+    }
     auto r = std::make_shared<Request>();
     r->cfg = *cfg;
     r->fft = fft;
@@ -315,6 +331,8 @@ static int submit(void *srv, const PzlConfig *cfg, const float *fft, bool on_dev
     // although requests of one shape share a cached bank), and the runtime's
     // memory behind the plan's streams
     r->footprint = g.device_bytes + PZL_RUNTIME_BYTES_PER_SEARCH;
+    r->launch = launch;
+    r->asked = ls.asked;
     r->t_submit = Clock::now();
     if (deadline_ms > 0) {
         r->has_deadline = true;

@@ -212,6 +212,57 @@ void memory()
     EXPECT(hipstub_device_bytes() == 0, "%lld bytes held", hipstub_device_bytes());
 }
 
+// A request's footprint: raised where the budget allows, else as asked, and
+// refused only where that does not fit.
+void server()
+{
+    const PzlConfig small = config(1 << 21, 50, 0, 8, 8), large = config(1 << 18, 200, 300, 8, 8);
+    struct Case {
+        const PzlConfig *c;
+        int launch, inflight;  // the budget: inflight such footprints
+        int want;              // rsteps per launch that the request gets, 0: refused
+        long long less;        // ... less this many bytes
+    };
+    const Case cases[] = {{&small, 0, 1, 256, 0}, {&small, 0, 1, 8, 1}, {&small, 8, 1, 8, 0},   {&small, 8, 1, 0, 1},
+                          {&small, 8, 2, 8, 0},   {&large, 0, 2, 32, 0}, {&large, 0, 2, 8, 1},  {&large, 8, 2, 8, 0},
+                          {&large, 8, 1, 8, 0},   {&large, 8, 1, 0, 1}};
+    for (const Case &k : cases) {
+        PzlGeometry g, want;
+        ok(pzl_geometry_launch(k.c, k.launch, &g));
+        const long long budget = k.inflight * (g.device_bytes + PZL_RUNTIME_BYTES_PER_SEARCH) - k.less;
+        void *srv = nullptr;
+        ok(pzl_server_create(0, budget, k.inflight, &srv));
+        long long id = 0, n = 0;
+        const int rc = pzl_server_submit_device(srv, k.c, Plan::spectrum().data(), k.c->numbins, &id);
+        EXPECT((rc != 0) == (k.want == 0), "budget %lld: %d", budget, rc);
+        if (rc == 0 && k.want) {
+            PzlRequestStats st;
+            std::vector<PzlCand> v(1 << 16);
+            ok(pzl_server_wait(srv, id, v.data(), (long long)v.size(), &n, &st));
+            v.resize((size_t)n);
+            ok(pzl_geometry_launch(k.c, k.want, &want));
+            EXPECT(st.footprint == want.device_bytes + PZL_RUNTIME_BYTES_PER_SEARCH, "budget %lld: %lld, not %lld", budget,
+                   st.footprint, want.device_bytes + PZL_RUNTIME_BYTES_PER_SEARCH);
+            Plan p(*k.c, 8);
+            EXPECT(n > 0 && same(v, p.search()), "%lld candidates", n);
+        }
+        pzl_server_destroy(srv);
+        ok(pzl_bank_cache_clear());
+    }
+    // memory that others took meanwhile: the plan is made as asked
+    PzlGeometry g;
+    ok(pzl_geometry_from_config(&small, &g));
+    hipstub_set_memory(288LL << 30, g.device_bytes / 2);
+    void *srv = nullptr;
+    ok(pzl_server_create(0, 8LL << 30, 1, &srv));
+    long long id = 0, n = 0;
+    ok(pzl_server_submit_device(srv, &small, Plan::spectrum().data(), small.numbins, &id));
+    PzlRequestStats st;
+    ok(pzl_server_wait(srv, id, nullptr, 0, &n, &st));
+    EXPECT(n > 0, "%lld candidates", n);
+    pzl_server_destroy(srv);
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
@@ -220,6 +271,7 @@ int main(int argc, char **argv)
     if (name == "exact") exact();
     else if (name == "rule") rule();
     else if (name == "memory") memory();
+    else if (name == "server") server();
     else {
         fprintf(stderr, "no check '%s'\n", name.c_str());
         return 2;
