@@ -152,12 +152,27 @@ int need_whole_bank(Plan *p)
 constexpr int kDefaultBatch = 8, kMaxBatch = 512, kMaxBatchLarge = 32;
 constexpr long long kBatchPlanes = 512LL << 20, kBatchPlanesLarge = 3LL << 30;
 
+// The most hits an rstep can have.
+long long rstep_hits(const PzlGeometry &g)
+{
+    return (long long)g.corr_uselen * g.numz * std::max(g.numw, 1) * g.numharmstages;
+}
+
+// Hits of a slot for batches of 'batch' rsteps.
+long long slot_hits(const PzlConfig &cfg, const PzlGeometry &g, int batch)
+{
+    const long long cap = cfg.maxhits > 0 ? cfg.maxhits : kDefaultHitCap;
+    // one rstep can never overflow a slot
+    return std::max(std::min(cap, rstep_hits(g) * batch), rstep_hits(g));
+}
+
 // More rsteps per launch than asked for while a batch's planes stay small: a short
 // search then fills the chip and does not pay per batch for its launches, its
 // count's way to the host and its sort.  Up to 32 rsteps also while the planes are
 // large, as each kernel row is read once per batch; not where fewer than the
 // default of 8 are asked for, which bounds the plan's memory.  One rstep per launch
-// stays one.  Measured on MI355X, ms per search: 540 rsteps of 0.3 MiB: 8 per
+// stays one.  A slot, sized for the rsteps asked for, holds a hit in one of 64 of a
+// launch's cells and stages at least.  Measured on MI355X, ms per search: 540 rsteps of 0.3 MiB: 8 per
 // launch 5.64, 270 0.54, 512 0.46; 1117 of 1.2 MiB: 8 8.9, 128 1.52, 256 1.46, 512
 // 1.46; 182 of 88 MiB: 8 12.7, 16 11.7, 32 11.1; 2920 of 157 MiB: 8 532, 16 462
 // (13 and 19: 483 and 487, so sizes are doubled and not filled up to the limit).
@@ -167,10 +182,11 @@ pzl::LaunchSizes launch_sizes(const PzlConfig &cfg, const PzlGeometry &g)
     s.asked = cfg.batchsize > 0 ? cfg.batchsize : kDefaultBatch;
     if (g.nrsteps > 0 && s.asked > g.nrsteps) s.asked = (int)g.nrsteps;
     if (s.asked < 1) s.asked = 1;
+    const long long slot = slot_hits(cfg, g, s.asked);
     auto raise = [&](int n, int most, long long planes) {
         while (n < most && n < g.nrsteps) {
             const int next = (int)std::min<long long>({2LL * n, kMaxBatch, g.nrsteps});
-            if (next * g.plane_bytes_per_rstep > planes) break;
+            if (next * g.plane_bytes_per_rstep > planes || next * rstep_hits(g) > 64 * slot) break;
             n = next;
         }
         return n;
@@ -200,25 +216,20 @@ int width_group() { return pzl_corr_num_groups() - 1; }
 int width_has(int n) { return pzl_corr_group_has(width_group(), n); }
 
 // launch: rsteps per launch (0: by the rule above).
-void size_launch(PlanSizes &z, const PzlConfig &cfg, const PzlGeometry &g, const std::vector<PzlHarm> &harms, int launch)
+void size_launch(PlanSizes &z, const PzlConfig &cfg, const PzlGeometry &g, int launch)
 {
     const LaunchSizes ls = launch_sizes(cfg, g);
     z.B = launch > 0 ? (int)std::max<long long>(1, std::min<long long>(launch, g.nrsteps)) : ls.large;
     z.sub = std::min(ls.asked, z.B);
-    const PzlHarm &F = harms[0];
-    // one rstep can never overflow a slot
-    const long long per_rstep = (long long)g.corr_uselen * F.numz * F.numw * g.numharmstages;
-    long long cap = cfg.maxhits > 0 ? cfg.maxhits : kDefaultHitCap;
-    cap = std::min<long long>(cap, per_rstep * z.sub);
-    z.hitcap = std::max<long long>(cap, per_rstep);
-    const long long nbatches = (g.nrsteps + z.B - 1) / z.B;
+    z.hitcap = slot_hits(cfg, g, z.sub);
+    const long long nbatches = (g.nrsteps + z.sub - 1) / z.sub;  // also where the search goes on at that size
     z.nslots = (int)std::max<long long>(1, std::min<long long>(Plan::kSlots, nbatches));
 }
 
 PlanSizes plan_sizes(const PzlConfig &cfg, const PzlGeometry &g, const std::vector<PzlHarm> &harms, int launch)
 {
     PlanSizes z;
-    size_launch(z, cfg, g, harms, launch);
+    size_launch(z, cfg, g, launch);
     z.seg_stride = 0;
     for (auto &H : harms) z.seg_stride += H.fftlen / 2;
     z.set_seg_stride = z.wbank_bytes = 0;
@@ -301,11 +312,11 @@ int fit_launch(PlanSizes &z, const PzlConfig &cfg, const PzlGeometry &g, const s
         size_t free_b = 0, total_b = 0;
         PZL_HIPCHK(hipMemGetInfo(&free_b, &total_b));
         for (int n : {ls.large, ls.small}) {
-            size_launch(z, cfg, g, harms, n);
+            size_launch(z, cfg, g, n);
             if (n > ls.asked && plan_device_bytes(g, z, harms, -1) <= (long long)(free_b / 4)) return 0;
         }
     }
-    size_launch(z, cfg, g, harms, ls.asked);
+    size_launch(z, cfg, g, ls.asked);
     return 0;
 }
 
@@ -1019,51 +1030,45 @@ int reset_slot(Plan &p, int slot, hipStream_t st)
     return 0;
 }
 
-// Search rsteps [r0, r0 + nb) again, nothing else in flight, in pieces of at
-// most 'step': a piece that overflows the slot is done one rstep at a time (one
-// rstep never exceeds a slot: hitcap >= cells per rstep x stages).
-int search_again(Plan &p, int slot, long long r0, int nb, int step, SearchState &ss, Timers *tm)
-{
-    for (int b = 0; b < nb; b += step) {
-        const int m = std::min(step, nb - b);
-        // the previous piece's sort (stream st2) reads and rewrites the slot's
-        // buffers: the harmonic sum refills them only after it
-        PZL_HIPCHK(hipStreamWaitEvent(p.sum_stream(), p.ev_free[slot], 0));
-        int rc = reset_slot(p, slot, p.sum_stream());
-        if (rc) return rc;
-        rc = launch_batch(p, r0 + b, m, 0, slot, nullptr, tm);
-        if (rc) return rc;
-        PZL_PINNED_CHECK(p.h_counts + 2 * slot, 2 * sizeof(unsigned long long));
-        PZL_HIPCHK(hipMemcpyAsync(p.h_counts + 2 * slot, p.d_counts + 2 * slot, 2 * sizeof(unsigned long long),
-                                  hipMemcpyDeviceToHost, p.sum_stream()));
-        rc = sync_all(p);
-        if (rc) return rc;
-        const unsigned long long n = p.h_counts[2 * slot];
-        if ((long long)n <= p.hitcap) {
-            rc = apply_slot(p, slot, (long long)n, ss);
-        } else if (m > 1) {
-            rc = search_again(p, slot, r0 + b, m, 1, ss, tm);
-        } else {
-            rc = fail(PZL_ERR_OVERFLOW, "hit buffer overflow: %llu hits in one rstep", n);
-        }
-        if (rc) return rc;
-    }
-    return 0;
-}
-
 // Wait for the batch in 'slot', order and apply its hits.  A batch that
-// overflowed the slot is searched again in the pieces the slot was sized for.
-int finalize(Plan &p, int slot, long long r0, int nb, SearchState &ss, Timers *tm)
+// overflowed the slot is searched again one rstep at a time (one rstep never
+// exceeds a slot: hitcap >= cells per rstep x stages); one of more rsteps than
+// the slot was sized for is left as it is, with *redo set.
+int finalize(Plan &p, int slot, long long r0, int nb, SearchState &ss, Timers *tm, bool *redo)
 {
     const auto w0 = std::chrono::steady_clock::now();
     PZL_HIPCHK(hipEventSynchronize(p.ev_count[slot]));
     ss.ms_wait_count += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - w0).count();
     const unsigned long long n = p.h_counts[2 * slot];
     if ((long long)n <= p.hitcap) return apply_slot(p, slot, (long long)n, ss);  // resets the slot
-    // overflow: let every batch in flight finish, then search this batch again
-    const int rc = sync_all(p);
+    if (nb > p.sub_batch) {
+        *redo = true;
+        return 0;
+    }
+    // overflow: let every batch in flight finish, then search this batch
+    // again one rstep at a time
+    int rc = sync_all(p);
     if (rc) return rc;
-    return search_again(p, slot, r0, nb, nb > p.sub_batch ? p.sub_batch : 1, ss, tm);
+    for (int b = 0; b < nb; b++) {
+        // the previous rstep's sort (stream st2) reads and rewrites the slot's
+        // buffers: the harmonic sum refills them only after it
+        PZL_HIPCHK(hipStreamWaitEvent(p.sum_stream(), p.ev_free[slot], 0));
+        rc = reset_slot(p, slot, p.sum_stream());
+        if (rc) return rc;
+        rc = launch_batch(p, r0 + b, 1, 0, slot, nullptr, tm);
+        if (rc) return rc;
+        PZL_PINNED_CHECK(p.h_counts + 2 * slot, 2 * sizeof(unsigned long long));
+        PZL_HIPCHK(hipMemcpyAsync(p.h_counts + 2 * slot, p.d_counts + 2 * slot, 2 * sizeof(unsigned long long),
+                                  hipMemcpyDeviceToHost, p.sum_stream()));
+        rc = sync_all(p);
+        if (rc) return rc;
+        const unsigned long long n1 = p.h_counts[2 * slot];
+        if ((long long)n1 > p.hitcap)
+            return fail(PZL_ERR_OVERFLOW, "hit buffer overflow: %llu hits in one rstep", n1);
+        rc = apply_slot(p, slot, (long long)n1, ss);
+        if (rc) return rc;
+    }
+    return 0;
 }
 
 double plane_alg_bytes(const Plan &p)
@@ -1552,48 +1557,70 @@ int pzl_search(void *plan, long long rstep_lo, long long rstep_hi, PzlCand *cand
         (int)std::max<long long>(1, std::min<long long>(8, (rstep_hi - rstep_lo) / std::max(p->B, 1) / 8));
     long long sampled = 0;
     bool timed_out = false;
-    for (long long r0 = rstep_lo; r0 < rstep_hi; r0 += p->B, i++) {
-        if (p->has_deadline && std::chrono::steady_clock::now() >= p->deadline) {
-            timed_out = true;  // launch nothing more; the batches in flight drain below
-            break;
-        }
-        const int nb = (int)std::min<long long>(p->B, rstep_hi - r0);
-        const int slot = i % p->nslots;
-        tm.active = (i % sample_every) == 0;
-        sampled += tm.active;
-        if (pend.size() - head == (size_t)p->nslots) {
-            const Pending q = pend[head++];
-            int rc = finalize(*p, q.slot, q.r0, q.nb, ss, &tm);
-            if (rc) return rc;
-        }
-        // the harmonic sum writes into the slot once the host has drained it
-        if (i >= p->nslots) PZL_HIPCHK(hipStreamWaitEvent(p->sum_stream(), p->ev_free[slot], 0));
-        // (segments ahead on their own stream read only what is constant during
-        // the search: the spectrum and the startr table)
-        int rc = launch_batch(*p, r0, nb, i % Plan::kSets, slot, nullptr, &tm, true, p->use_graph,
-                              p->overlap_sum && p->side_classes);
-        if (rc) return rc;
-        PZL_PINNED_CHECK(p->h_counts + 2 * slot, 2 * sizeof(unsigned long long));
-        PZL_HIPCHK(hipMemcpyAsync(p->h_counts + 2 * slot, p->d_counts + 2 * slot, 2 * sizeof(unsigned long long),
-                                  hipMemcpyDeviceToHost, p->sum_stream()));
-        PZL_HIPCHK(hipEventRecord(p->ev_count[slot], p->sum_stream()));
-        pend.push_back({slot, nb, r0});
-        // apply whatever the GPU has already finished
-        while (head + 1 < pend.size() && hipEventQuery(p->ev_count[pend[head].slot]) == hipSuccess) {
-            const Pending q = pend[head++];
-            rc = finalize(*p, q.slot, q.r0, q.nb, ss, &tm);
-            if (rc) return rc;
-        }
-    }
-    tm.active = true;
-    if (tm.on) {
-        ev_end = tm.get();
-        PZL_HIPCHK(hipEventRecord(ev_end, p->sum_stream()));  // the last harmonic sum follows the last correlation
-    }
-    while (head < pend.size()) {
+    int step = p->B;
+    long long r0 = rstep_lo;
+    // Apply the oldest batch in flight.  If it holds more hits than its slot and was
+    // raised above the size that the slot is for, it and the batches after it are
+    // dropped and the rest of the search goes on from it at that size: dense hits
+    // come in bands, and a slot for every raised batch would cost more memory than
+    // the raise is for.
+    auto apply_oldest = [&]() -> int {
         const Pending q = pend[head++];
-        int rc = finalize(*p, q.slot, q.r0, q.nb, ss, &tm);
-        if (rc) return rc;
+        bool redo = false;
+        int rc = finalize(*p, q.slot, q.r0, q.nb, ss, &tm, &redo);
+        if (rc || !redo) return rc;
+        rc = sync_all(*p);
+        for (head--; head < pend.size() && rc == 0; head++) rc = reset_slot(*p, pend[head].slot, p->sum_stream());
+        step = p->sub_batch;
+        r0 = q.r0;
+        return rc;
+    };
+    for (;;) {
+        while (r0 < rstep_hi) {
+            if (p->has_deadline && std::chrono::steady_clock::now() >= p->deadline) {
+                timed_out = true;  // launch nothing more; the batches in flight drain below
+                break;
+            }
+            if (pend.size() - head == (size_t)p->nslots) {
+                int rc = apply_oldest();
+                if (rc) return rc;
+                continue;
+            }
+            const int nb = (int)std::min<long long>(step, rstep_hi - r0);
+            const int slot = i % p->nslots;
+            tm.active = (i % sample_every) == 0;
+            sampled += tm.active;
+            // the harmonic sum writes into the slot once the host has drained it
+            if (i >= p->nslots) PZL_HIPCHK(hipStreamWaitEvent(p->sum_stream(), p->ev_free[slot], 0));
+            // (segments ahead on their own stream read only what is constant during
+            // the search: the spectrum and the startr table)
+            int rc = launch_batch(*p, r0, nb, i % Plan::kSets, slot, nullptr, &tm, true, p->use_graph,
+                                  p->overlap_sum && p->side_classes);
+            if (rc) return rc;
+            PZL_PINNED_CHECK(p->h_counts + 2 * slot, 2 * sizeof(unsigned long long));
+            PZL_HIPCHK(hipMemcpyAsync(p->h_counts + 2 * slot, p->d_counts + 2 * slot, 2 * sizeof(unsigned long long),
+                                      hipMemcpyDeviceToHost, p->sum_stream()));
+            PZL_HIPCHK(hipEventRecord(p->ev_count[slot], p->sum_stream()));
+            pend.push_back({slot, nb, r0});
+            r0 += nb;
+            i++;
+            // apply whatever the GPU has already finished
+            while (head + 1 < pend.size() && hipEventQuery(p->ev_count[pend[head].slot]) == hipSuccess) {
+                rc = apply_oldest();
+                if (rc) return rc;
+            }
+        }
+        tm.active = true;
+        if (tm.on) {
+            if (!ev_end) ev_end = tm.get();
+            PZL_HIPCHK(hipEventRecord(ev_end, p->sum_stream()));  // the last harmonic sum follows the last correlation
+        }
+        const long long launched = r0;
+        while (head < pend.size()) {
+            int rc = apply_oldest();
+            if (rc) return rc;
+        }
+        if (timed_out || r0 == launched) break;  // (else batches were dropped: on from there)
     }
     {
         int rc = sync_all(*p);
@@ -1605,7 +1632,7 @@ int pzl_search(void *plan, long long rstep_lo, long long rstep_hi, PzlCand *cand
         p->last_cands.clear();
         p->last_hits_complete = false;
         return fail(PZL_ERR_TIMEOUT, "search deadline passed after %d of %lld batches", i,
-                    (rstep_hi - rstep_lo + p->B - 1) / p->B);
+                    (rstep_hi - rstep_lo + step - 1) / step);
     }
     p->last_cands = ss.cl.items();
     const auto &items = p->last_cands;

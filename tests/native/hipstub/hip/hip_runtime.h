@@ -120,3 +120,7 @@ template <typename T> inline hipError_t hipHostMalloc(T **p, size_t n, unsigned 
 long long hipstub_device_bytes();
 // Device memory that hipMemGetInfo counts from, and that hipMalloc gives out.
 void hipstub_set_memory(long long reported, long long available);
+// From now on rsteps lo .. hi - 1 have a hit in every 'every'-th cell and stage.
+void hipstub_set_burst(long long lo, long long hi, long long every);
+// hipStreamSynchronize calls so far.
+long long hipstub_syncs();

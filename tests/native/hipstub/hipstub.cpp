@@ -170,6 +170,14 @@ hipError_t hipMemGetInfo(size_t *free_b, size_t *total_b)
     *free_b = (size_t)std::max(0ll, g_reported - g_dev_bytes);
     return hipSuccess;
 }
+static std::atomic<long long> g_burst[3], g_syncs;
+void hipstub_set_burst(long long lo, long long hi, long long every)
+{
+    g_burst[0] = lo;
+    g_burst[1] = hi;
+    g_burst[2] = every;
+}
+long long hipstub_syncs() { return g_syncs; }
 long long hipstub_device_bytes()
 {
     std::lock_guard<std::mutex> lk(g_mem_mu);
@@ -278,6 +286,7 @@ hipError_t hipStreamDestroy(hipStream_t st)
 }
 hipError_t hipStreamSynchronize(hipStream_t st)
 {
+    g_syncs++;
     if (st) st->drain();
     else drain_all();
     return hipSuccess;
@@ -517,6 +526,16 @@ hipError_t pzl_launch_harmsum(const PzlSumArgs *a, hipStream_t st)
             const long long rstep = r0 + b;
             const unsigned h = mix((unsigned long long)rstep + 12345);
             const int n = (h % 7 == 0) ? 0 : (int)(h % 37);
+            const long long cells = (long long)s.nstages * s.numw * s.numz * s.corr_uselen;
+            if (rstep >= g_burst[0] && rstep < g_burst[1]) {  // a hit in every g_burst[2]-th cell and stage
+                for (long long k = 0; k < cells; k += g_burst[2]) {
+                    const unsigned long long idx = __atomic_fetch_add(s.nhits, 1ull, __ATOMIC_RELAXED);
+                    if (idx >= s.maxhits) continue;
+                    s.hit_keys[idx] = rstep * cells + k;
+                    s.hit_pows[idx] = s.powcut[0] + (float)(mix((unsigned long long)k) % 1000) * 0.01f;
+                }
+                continue;
+            }
             for (int k = 0; k < n; k++) {
                 const unsigned g = mix(((unsigned long long)rstep << 20) + (unsigned)k);
                 const int stage = (int)(g % (unsigned)s.nstages);

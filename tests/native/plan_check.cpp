@@ -141,7 +141,7 @@ void rule()
         std::vector<std::pair<int, int>> want;  // asked, launched
     };
     const std::vector<Shape> shapes = {
-        {1 << 20, 20, 0, 4, {{8, 512}, {3, 512}, {700, 700}}},       // 0.3 MiB, 540 rsteps
+        {1 << 20, 20, 0, 4, {{8, 512}, {3, 192}, {700, 700}}},       // 0.3 MiB, 540 rsteps
         {1 << 21, 50, 0, 8, {{0, 256}, {8, 256}, {4, 256}}},         // 1.2 MiB
         {1 << 18, 200, 300, 8, {{8, 32}, {4, 4}, {2, 4}, {64, 64}}}, // 88 MiB
         {1 << 22, 200, 300, 16, {{8, 16}, {16, 16}, {7, 7}, {2, 2}}}, // 157 MiB
@@ -263,6 +263,54 @@ void server()
     pzl_server_destroy(srv);
 }
 
+// Batches that overflow their hit slot, anywhere in a search: the same hits and
+// candidates as with slots for every cell, and no more than the batches in flight
+// launched twice, the search going on at the size asked for.
+void overflow()
+{
+    const PzlConfig c = config(1 << 18, 8, 0, 2, 4);
+    PzlGeometry g;
+    ok(pzl_geometry_from_config(&c, &g));
+    const long long n = g.nrsteps;
+    const struct {
+        long long lo, hi, every;
+    } bursts[] = {{0, n, 8},           // a batch as asked fits, a raised one does not, throughout
+                  {0, n, 2},           // nor does one as asked: one rstep at a time
+                  {0, 3, 1},           // in the first batch
+                  {n - 9, n, 2},       // in the last
+                  {n / 2, n / 2 + 12, 3}, {-1, -1, 1}};
+    auto hits = [&](Plan &p) {
+        long long k = 0;
+        ok(pzl_get_hits(p.h, nullptr, nullptr, 0, &k));
+        std::vector<long long> keys((size_t)k);
+        std::vector<float> pows((size_t)k);
+        ok(pzl_get_hits(p.h, keys.data(), pows.data(), k, &k));
+        return std::make_pair(keys, pows);
+    };
+    for (auto &b : bursts) {
+        hipstub_set_burst(b.lo, b.hi, b.every);
+        Plan all(c, 1);  // a slot for every cell of a batch
+        PzlStats st;
+        const auto want = all.search();
+        const auto want_hits = hits(all);
+        PzlConfig cs = c;
+        cs.maxhits = 1;  // a slot for one rstep's
+        Plan rule(cs), p(cs, 16), asked(cs, 4);
+        EXPECT(rule.launch() == 64 && p.asked() == 4 && n > 7 * 16, "%d rsteps per launch of %lld", rule.launch(), n);
+        for (Plan *q : {&p, &asked, &rule, &p}) {
+            const long long s0 = hipstub_syncs();
+            const auto v = q->search(&st);
+            const long long syncs = hipstub_syncs() - s0;
+            EXPECT(!v.empty() && same(v, want), "burst %lld..%lld: %zu candidates, %zu", b.lo, b.hi, v.size(), want.size());
+            EXPECT(hits(*q) == want_hits, "burst %lld..%lld", b.lo, b.hi);
+            EXPECT(st.corr_launches <= 4 + (n + 3) / 4, "burst %lld..%lld: %lld launches", b.lo, b.hi, st.corr_launches);
+            // once for the batches dropped and once at the end, 5 streams each
+            if (b.every == 8) EXPECT(syncs <= 10, "%lld waits", syncs);
+        }
+    }
+    hipstub_set_burst(0, 0, 1);
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
@@ -272,6 +320,7 @@ int main(int argc, char **argv)
     else if (name == "rule") rule();
     else if (name == "memory") memory();
     else if (name == "server") server();
+    else if (name == "overflow") overflow();
     else {
         fprintf(stderr, "no check '%s'\n", name.c_str());
         return 2;
