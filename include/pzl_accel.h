@@ -159,7 +159,8 @@ int pzl_search(void *plan, long long rstep_lo, long long rstep_hi, PzlCand *cand
 /* A deadline for the plan's searches: once 'ms' milliseconds have passed
  * since this call, pzl_search launches no further batch, waits for the ones
  * in flight and returns PZL_ERR_TIMEOUT (its candidate list is then partial
- * and not returned).  ms <= 0 clears the deadline. */
+ * and not returned).  In the last 100 ms before it batches are of the batchsize
+ * asked for.  ms <= 0 clears the deadline. */
 int pzl_plan_set_deadline(void *plan, double ms);
 
 /* Autotuner: times the harmonic-sum forms on one batch of the plan's own data

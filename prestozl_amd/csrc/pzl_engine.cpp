@@ -1071,6 +1071,12 @@ int finalize(Plan &p, int slot, long long r0, int nb, SearchState &ss, Timers *t
     return 0;
 }
 
+// Time before a deadline from which on a search launches batches as asked for, so
+// that it stops as soon after it as without raised ones: a raised batch takes up to
+// 3 ms alone on MI355X (planes of 3 GiB) and 4 are in flight, 100 ms with 8 searches
+// sharing the GPU.
+constexpr std::chrono::milliseconds kDeadlineMargin(100);
+
 double plane_alg_bytes(const Plan &p)
 {
     double b = 0;
@@ -1577,9 +1583,13 @@ int pzl_search(void *plan, long long rstep_lo, long long rstep_hi, PzlCand *cand
     };
     for (;;) {
         while (r0 < rstep_hi) {
-            if (p->has_deadline && std::chrono::steady_clock::now() >= p->deadline) {
-                timed_out = true;  // launch nothing more; the batches in flight drain below
-                break;
+            if (p->has_deadline) {
+                const auto left = p->deadline - std::chrono::steady_clock::now();
+                if (left.count() <= 0) {
+                    timed_out = true;  // launch nothing more; the batches in flight drain below
+                    break;
+                }
+                if (left < kDeadlineMargin) step = p->sub_batch;
             }
             if (pend.size() - head == (size_t)p->nslots) {
                 int rc = apply_oldest();

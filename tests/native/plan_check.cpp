@@ -311,6 +311,38 @@ void overflow()
     hipstub_set_burst(0, 0, 1);
 }
 
+// Near a deadline batches are launched as asked for, and one that has passed stops
+// a search before its first batch; a far one and none change nothing.
+void deadline()
+{
+    const PzlConfig c = config(1 << 18, 8, 0, 2, 4);
+    Plan p(c);
+    PzlGeometry g;
+    ok(pzl_plan_geometry(p.h, &g));
+    EXPECT(p.launch() >= g.nrsteps, "%d", p.launch());
+    PzlStats st;
+    const auto want = p.search(&st);
+    EXPECT(!want.empty() && st.corr_launches == 1, "%lld launches", st.corr_launches);
+    ok(pzl_plan_set_deadline(p.h, 1e7));
+    EXPECT(same(p.search(&st), want) && st.corr_launches == 1, "%lld launches", st.corr_launches);
+    int in_time = 0;
+    for (int k = 0; k < 20; k++) {  // (a busy machine may miss some)
+        ok(pzl_plan_set_deadline(p.h, 99.0));
+        long long n = 0;
+        const int rc = pzl_search(p.h, 0, -1, nullptr, 0, &n, &st);
+        EXPECT(rc == 0 || rc == PZL_ERR_TIMEOUT, "%d", rc);
+        if (rc) continue;
+        in_time++;
+        EXPECT(same(p.cands(n), want) && st.corr_launches == (g.nrsteps + 3) / 4, "%lld launches", st.corr_launches);
+    }
+    EXPECT(in_time > 0, "no search in time");
+    ok(pzl_plan_set_deadline(p.h, 1e-6));
+    long long n = 0;
+    EXPECT(pzl_search(p.h, 0, -1, nullptr, 0, &n, nullptr) == PZL_ERR_TIMEOUT, "%lld candidates", n);
+    ok(pzl_plan_set_deadline(p.h, 0));
+    EXPECT(same(p.search(&st), want) && st.corr_launches == 1, "%lld launches", st.corr_launches);
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
@@ -321,6 +353,7 @@ int main(int argc, char **argv)
     else if (name == "memory") memory();
     else if (name == "server") server();
     else if (name == "overflow") overflow();
+    else if (name == "deadline") deadline();
     else {
         fprintf(stderr, "no check '%s'\n", name.c_str());
         return 2;
