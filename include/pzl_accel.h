@@ -200,8 +200,10 @@ int pzl_plan_cu_split(void *plan, int *sum_cus, int *sum_only_cus);
  * the search in one stream. */
 int pzl_plan_set_overlap(void *plan, int on);
 /* Rsteps per launch: for each candidate batch size, plan, autotune and time a
- * band of band_rsteps rsteps from the middle of the search on this spectrum;
- * *best gets the fastest, ms_per_rstep (optional, ncand entries) the times.
+ * band of band_rsteps rsteps (at least 4 batches) from the middle of the search
+ * on this spectrum; *best gets the fastest, ms_per_rstep (optional, ncand
+ * entries) the times.  Candidates that pzl_plan_create raises to the same rsteps
+ * per launch are timed once and share the time; the first of them counts.
  * Results do not depend on the batch size. */
 int pzl_tune_batchsize(const PzlConfig *cfg, int device, const float *host_fft, long long numbins,
                        const int *candidates, int ncand, long long band_rsteps, int *best, double *ms_per_rstep);

@@ -2035,16 +2035,26 @@ int pzl_tune_batchsize(const PzlConfig *cfg, int device, const float *host_fft, 
     if (!cfg || !host_fft || !candidates || ncand < 1 || !best) return fail(PZL_ERR_ARG, "bad arguments");
     double best_ms = 1e300;
     *best = candidates[0];
+    std::map<int, double> timed;  // rsteps per launch -> ms per rstep
     for (int k = 0; k < ncand; k++) {
         PzlConfig c = *cfg;
         c.batchsize = candidates[k];
+        LaunchSizes ls;
+        int rc = launch_sizes_of(c, &ls);
+        if (rc) return rc;
+        // candidates whose plans launch alike are one
+        if (timed.count(ls.large)) {
+            if (ms_per_rstep) ms_per_rstep[k] = timed[ls.large];
+            continue;
+        }
         void *plan = nullptr;
-        int rc = pzl_plan_create(&c, device, &plan);
+        rc = pzl_plan_create(&c, device, &plan);
         if (rc) return rc;
         Plan *p = (Plan *)plan;
         rc = pzl_set_spectrum(plan, host_fft, numbins);
         const long long nr = p->g.nrsteps;
-        const long long band = std::max<long long>(1, std::min<long long>(band_rsteps, nr));
+        // a few full batches at least, as a whole search has
+        const long long band = std::max<long long>(1, std::min(std::max<long long>(band_rsteps, 4LL * p->B), nr));
         const long long lo = std::max<long long>(0, std::min<long long>(nr / 2, nr - band));
         if (rc == 0) rc = pzl_autotune(plan, 2, nullptr, 0);
         if (rc == 0) rc = pzl_search(plan, lo, lo + band, nullptr, 0, nullptr, nullptr);  // warm
@@ -2057,6 +2067,7 @@ int pzl_tune_batchsize(const PzlConfig *cfg, int device, const float *host_fft, 
         pzl_plan_destroy(plan);
         if (rc) return rc;
         if (ms_per_rstep) ms_per_rstep[k] = ms;
+        timed[ls.large] = ms;
         if (ms < best_ms) {
             best_ms = ms;
             *best = candidates[k];

@@ -343,6 +343,32 @@ void deadline()
     EXPECT(same(p.search(&st), want) && st.corr_launches == 1, "%lld launches", st.corr_launches);
 }
 
+// The batch-size tuner times each launch size once.
+void tuner()
+{
+    const PzlConfig c = config(1 << 19, 20, 0, 4, 8);
+    const int cand[] = {8, 2, 16, 1, 64, 8};
+    double ms[6] = {};
+    int best = 0;
+    ok(pzl_tune_batchsize(&c, 0, Plan::spectrum().data(), c.numbins, cand, 6, 16, &best, ms));
+    std::vector<int> launch;
+    for (int b : cand) {
+        PzlConfig k = c;
+        k.batchsize = b;
+        launch.push_back(Plan(k).launch());
+    }
+    EXPECT(launch[0] == launch[2] && launch[0] == launch[4] && launch[1] < launch[0], "%d, %d", launch[0], launch[1]);
+    for (int i = 0; i < 6; i++) {
+        EXPECT(ms[i] > 0, "%d: %g", cand[i], ms[i]);
+        for (int j = 0; j < i; j++)
+            EXPECT((ms[i] == ms[j]) == (launch[i] == launch[j]), "%d: %g ms, %d: %g", cand[i], ms[i], cand[j], ms[j]);
+    }
+    int first = 0;
+    for (int i = 1; i < 6; i++)
+        if (ms[i] < ms[first]) first = i;
+    EXPECT(best == cand[first], "%d, not %d", best, cand[first]);
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
@@ -354,6 +380,7 @@ int main(int argc, char **argv)
     else if (name == "server") server();
     else if (name == "overflow") overflow();
     else if (name == "deadline") deadline();
+    else if (name == "tuner") tuner();
     else {
         fprintf(stderr, "no check '%s'\n", name.c_str());
         return 2;
