@@ -423,29 +423,6 @@ void pin_put(PzlHostHit *ptr, long long cap)
     pinned_free(ptr);
 }
 
-}  // namespace
-
-// At least 'count' whole chunks of hit records in the process-wide cache, as far
-// as its limit allows: the searches of a request loop then find theirs instead of
-// pinning 32 MiB (5 to 10 ms) while others run.
-int pzl::reserve_pinned_chunks(int count)
-{
-    constexpr long long chunk = 1LL << 20;
-    for (;;) {
-        {
-            std::lock_guard<std::mutex> lk(g_pin_mu);
-            int have = 0;
-            for (auto &kv : g_pin_cache) have += kv.first >= chunk;
-            if (have >= count || g_pin_cache_bytes + (long long)sizeof(PzlHostHit) * chunk > kPinCacheLimit) return 0;
-        }
-        PzlHostHit *ptr = nullptr;
-        PZL_HIPCHK(pinned_alloc((void **)&ptr, sizeof(PzlHostHit) * (size_t)chunk));
-        pin_put(ptr, chunk);
-    }
-}
-
-namespace {
-
 void free_plan(Plan *p)
 {
     if (!p) return;

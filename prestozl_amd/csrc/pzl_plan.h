@@ -44,8 +44,6 @@ int compute_geometry(const PzlConfig &c, PzlGeometry &g, std::vector<PzlHarm> *h
 bool compute_row_sets(const std::vector<PzlHarm> &harms, int corr_uselen, int (*has)(int n), std::vector<PzlHarm> *sets,
                       std::vector<int> *rows);
 
-int reserve_pinned_chunks(int count);  // pzl_engine.cpp
-
 // Rsteps per launch of a request (pzl_engine.cpp).
 struct LaunchSizes {
     int asked;  // as configured

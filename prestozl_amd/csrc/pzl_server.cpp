@@ -290,10 +290,6 @@ int pzl_server_create(int device, long long hbm_budget, int max_inflight, void *
         }
         hbm_budget = (long long)(free_b * 0.8);
     }
-    if (reserve_pinned_chunks(std::min(max_inflight, 8))) {
-        delete s;
-        return PZL_ERR_HIP;
-    }
     s->budget = hbm_budget;
     s->max_inflight = max_inflight;
     for (int i = 0; i < max_inflight; i++) s->workers.emplace_back([s] { s->worker(); });

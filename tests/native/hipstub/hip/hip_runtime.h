@@ -120,6 +120,8 @@ template <typename T> inline hipError_t hipHostMalloc(T **p, size_t n, unsigned 
 long long hipstub_device_bytes();
 // Device memory that hipMemGetInfo counts from, and that hipMalloc gives out.
 void hipstub_set_memory(long long reported, long long available);
+// Bytes that hipHostMalloc gives out from the start of the process on.
+void hipstub_set_pinnable(long long bytes);
 // From now on rsteps lo .. hi - 1 have a hit in every 'every'-th cell and stage.
 void hipstub_set_burst(long long lo, long long hi, long long every);
 // hipStreamSynchronize calls so far.

@@ -219,8 +219,15 @@ hipError_t hipFree(void *p)
     free(p);
     return hipSuccess;
 }
+static std::atomic<long long> g_pinned{0}, g_pinnable{1ll << 40};
+void hipstub_set_pinnable(long long bytes) { g_pinnable = bytes; }
 hipError_t hipHostMalloc(void **p, size_t n, unsigned)
 {
+    if ((g_pinned += (long long)n) > g_pinnable) {
+        g_pinned -= (long long)n;
+        *p = nullptr;
+        return hipErrorOutOfMemory;
+    }
     *p = malloc(n);
     return *p ? hipSuccess : hipErrorOutOfMemory;
 }

@@ -369,6 +369,23 @@ void tuner()
     EXPECT(best == cand[first], "%d, not %d", best, cand[first]);
 }
 
+// A server pins nothing before its requests need it.
+void pinned()
+{
+    hipstub_set_pinnable(0);
+    void *srv = nullptr;
+    EXPECT(pzl_server_create(0, 8LL << 30, 8, &srv) == 0, "%s", pzl_last_error());
+    if (!srv) return;
+    hipstub_set_pinnable(8 << 20);  // a small buffer and the counts, not a whole chunk of 32 MiB
+    const PzlConfig c = config(1 << 18, 8, 0, 2, 4);
+    long long id = 0, n = 0;
+    PzlRequestStats st;
+    ok(pzl_server_submit_device(srv, &c, Plan::spectrum().data(), c.numbins, &id));
+    ok(pzl_server_wait(srv, id, nullptr, 0, &n, &st));
+    EXPECT(n > 0, "%lld candidates", n);
+    pzl_server_destroy(srv);
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
@@ -381,6 +398,7 @@ int main(int argc, char **argv)
     else if (name == "overflow") overflow();
     else if (name == "deadline") deadline();
     else if (name == "tuner") tuner();
+    else if (name == "pinned") pinned();
     else {
         fprintf(stderr, "no check '%s'\n", name.c_str());
         return 2;
