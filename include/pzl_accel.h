@@ -100,7 +100,7 @@ typedef struct PzlStats {
                                      conj(kernel), 3 per stored power */
     double ms_corr_group;         /* summed duration of the grouped correlation launches (the
                                      class_ms of the lengths they hold are then 0) */
-    long long group_launches;
+    long long group_launches; /* ... and how many they were */
     double ms_wait_count;  /* launching thread waiting for the oldest batch in flight (its hit count) */
     double ms_wait_pool;   /* launching thread waiting for a pinned hit-record buffer (the insertion
                               thread behind) */
@@ -219,8 +219,9 @@ int pzl_plan_set_sum_form(void *plan, int order, int rpt);
  * longest keeps its own launch) or for every length (all = 1: one correlation
  * launch per batch).  A group holds one kernel variant per length; it must hold
  * every length it is given.  The default is the last group, whose name begins
- * "rows by width": one launch in which each kernel row runs at the shortest
- * transform that its own half-width allows instead of its harmonic's length.
+ * "rows by width": each kernel row at the shortest transform that its own
+ * half-width allows instead of its harmonic's length, in one launch, and a second
+ * one for the rows of more than 2048 points where the search has any.
  * Results do not depend on the form beyond the transforms' rounding. */
 int pzl_plan_corr_group(void *plan, int *group, int *all);
 int pzl_plan_set_corr_group(void *plan, int group, int all);

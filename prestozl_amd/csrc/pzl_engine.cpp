@@ -1665,8 +1665,9 @@ int pzl_search(void *plan, long long rstep_lo, long long rstep_hi, PzlCand *cand
         const bool width = by_width(*p);
         for (auto &H : width ? p->sets : p->harms) seg_bytes += H.fftlen / 2 * 8.0;
         const double planes = plane_alg_bytes(*p);
-        stats->bytes_alg = stats->nrsteps * (planes + seg_bytes) + (double)p->g.bank_bytes;
-        stats->bytes_alg_corr = stats->nrsteps * (planes / 2 + seg_bytes) + (double)p->g.bank_bytes;
+        const double bank = (double)(width ? p->wbank_bytes : p->bank_bytes);
+        stats->bytes_alg = stats->nrsteps * (planes + seg_bytes) + bank;
+        stats->bytes_alg_corr = stats->nrsteps * (planes / 2 + seg_bytes) + bank;
         // sampled batches -> estimates for the whole search (launch counts exact)
         const double scale = sampled > 0 ? (double)i / (double)sampled : 0.0;
         stats->ms_segments *= scale;
@@ -1677,8 +1678,15 @@ int pzl_search(void *plan, long long rstep_lo, long long rstep_hi, PzlCand *cand
         for (auto &kv : per_class) kv.second *= scale;
         for (auto &kv : per_class_n) kv.second = i;
         const bool grouped = width || (p->side_group >= 0 && p->classes.size() > 1);
-        stats->group_launches = grouped ? i : 0;
-        stats->corr_launches = (long long)i * (grouped ? (p->group_all ? 1LL : 2LL) : (long long)p->classes.size());
+        long long per_batch = 1;  // grouped launches
+        if (width) {
+            std::vector<int> lens;
+            for (auto &c : p->set_classes) lens.push_back(c.fftlen);
+            per_batch = pzl_corr_group_launches(p->side_group, (int)lens.size(), lens.data());
+        }
+        stats->group_launches = grouped ? i * per_batch : 0;
+        stats->corr_launches =
+            (long long)i * (grouped ? (p->group_all ? per_batch : 2LL) : (long long)p->classes.size());
         stats->graph_launches = (long long)std::llround(stats->graph_launches * scale);
         for (auto &kv : per_class) stats->ms_corr_max_class = std::max(stats->ms_corr_max_class, kv.second);
         stats->nclass = 0;

@@ -114,6 +114,8 @@ const char *pzl_corr_variant_name(int n, int v);
 // error.  The last group holds closely spaced lengths, for classes of row sets.
 hipError_t pzl_launch_corr_group(int group, int ncls, const int *fftlens, const PzlCorrArgs *const *args,
                                  const int *const *class_nrows, hipStream_t st);
+// How many kernels that launch is (the last group's lengths above 2048 have their own).
+int pzl_corr_group_launches(int group, int ncls, const int *fftlens);
 int pzl_corr_num_groups(void);
 const char *pzl_corr_group_name(int group);
 int pzl_corr_group_has(int group, int n);

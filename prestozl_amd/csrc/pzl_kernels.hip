@@ -1419,6 +1419,13 @@ static hipError_t width_group_launch(int ncls, const int *fftlens, const PzlCorr
     return hipSuccess;
 }
 
+static int width_group_launches(int ncls, const int *fftlens)
+{
+    int n = 0;
+    for (int c = 0; c < ncls; c++) n += CorrGroupWidthLong::has(fftlens[c]) != 0;
+    return (n > 0) + (n < ncls);
+}
+
 struct CorrGroupEntry {
     const char *name;
     hipError_t (*launch)(int, const int *, const PzlCorrArgs *const *, const int *const *, hipStream_t);
@@ -1436,6 +1443,11 @@ static const CorrGroupEntry g_corr_groups[] = {
 static const int g_ncorr_groups = (int)(sizeof(g_corr_groups) / sizeof(g_corr_groups[0]));
 
 extern "C" int pzl_corr_num_groups(void) { return g_ncorr_groups; }
+
+extern "C" int pzl_corr_group_launches(int group, int ncls, const int *fftlens)
+{
+    return group == g_ncorr_groups - 1 ? width_group_launches(ncls, fftlens) : 1;
+}
 
 extern "C" const char *pzl_corr_group_name(int group)
 {

@@ -85,3 +85,26 @@ def test_not_finite_values_spread_as_far(bad):
                 assert np.max(np.abs(x[ok] - y[ok]) / np.maximum(y[ok], 1.0)) < TOL
     assert seen == {True, False}
     plan.close()
+
+
+@pytest.mark.parametrize("wmax,per_batch", [(300, 1), (500, 2)])
+def test_statistics_of_the_launch_form(wmax, per_batch):
+    """A search's statistics count the launches of the form in use (rows of more
+    than 2048 points have a launch of their own) and the bank it reads."""
+    N = 1 << 18
+    plan = _plan(N, _spectrum(N, wmax), 200, wmax, 16)
+    batches = -(-plan.geom.nrsteps // plan.launch()[0])
+    st = plan.search()[1]
+    assert (st["corr_launches"], st["group_launches"]) == (per_batch * batches, per_batch * batches)
+    bank = plan.geom.bank_bytes  # the rows' by width
+    plan.set_corr_group(-1)
+    whole = plan.search()[1]
+    assert (whole["corr_launches"], whole["group_launches"]) == (len(plan.fftlens()) * batches, 0)
+    whole_bank = sum(8 * h.numw * h.numz * h.fftlen for h in plan.harms)
+    assert whole_bank > bank
+    # beside the banks the two forms differ by the segments, which both figures hold alike
+    assert st["bytes_alg"] - st["bytes_alg_corr"] == whole["bytes_alg"] - whole["bytes_alg_corr"]
+    segments = plan.geom.nrsteps * sum(4 * h.fftlen for h in plan.harms)
+    planes = st["bytes_alg"] - st["bytes_alg_corr"]
+    assert whole["bytes_alg_corr"] == pytest.approx(planes + segments + whole_bank, rel=1e-12)
+    plan.close()
