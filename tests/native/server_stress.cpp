@@ -6,7 +6,8 @@
 // that pass in the queue and while running, and repeated rounds so that
 // pinned hit buffers move through the process-wide cache between plans.
 // Before that, one plan per shape searches again under CU splits, hit-record
-// chunk sizes and graph settings changed between its searches.
+// chunk sizes and graph settings changed between its searches.  Every search is
+// of many batches: requests of one rstep per launch, and plans of 4 made so.
 // Exit status 0 when every check holds.  Test infrastructure only.
 #include <hip/hip_runtime.h>
 
@@ -17,7 +18,7 @@
 
 #include "pzl_accel.h"
 
-static PzlConfig config(double N, double dt, int zmax, int wmax, int numharm)
+static PzlConfig config(double N, double dt, int zmax, int wmax, int numharm, int batchsize)
 {
     PzlConfig c;
     memset(&c, 0, sizeof c);
@@ -33,7 +34,7 @@ static PzlConfig config(double N, double dt, int zmax, int wmax, int numharm)
     c.flo = 1.0;
     c.fhiP = 1;
     c.fhi = 1e4;
-    c.batchsize = 4;
+    c.batchsize = batchsize;
     return c;
 }
 
@@ -55,8 +56,14 @@ static std::vector<PzlCand> alone(const PzlConfig &c, const float *fft)
         exit(2);
     }
     long long n = 0;
-    if (pzl_set_spectrum(plan, fft, c.numbins) || pzl_search(plan, 0, -1, nullptr, 0, &n, nullptr)) {
+    PzlStats st;
+    if (pzl_set_spectrum(plan, fft, c.numbins) || pzl_search(plan, 0, -1, nullptr, 0, &n, &st)) {
         fprintf(stderr, "search: %s\n", pzl_last_error());
+        exit(2);
+    }
+    int launch = 0;
+    if (pzl_plan_launch(plan, &launch, nullptr) || (c.batchsize == 1 && st.corr_launches < 32)) {
+        fprintf(stderr, "%lld batches of %d\n", st.corr_launches, launch);
         exit(2);
     }
     std::vector<PzlCand> v((size_t)n);
@@ -69,8 +76,9 @@ int main(int argc, char **argv)
 {
     setvbuf(stdout, nullptr, _IOLBF, 0);
     const int rounds = argc > 1 ? atoi(argv[1]) : 3;
-    std::vector<PzlConfig> shapes = {config(1 << 17, 1e-3, 8, 0, 2), config(1 << 17, 1e-3, 10, 20, 4),
-                                     config(1 << 16, 2e-3, 4, 0, 8), config(1 << 18, 5e-4, 6, 20, 2)};
+    // (the third is raised to the whole search)
+    std::vector<PzlConfig> shapes = {config(1 << 17, 1e-3, 8, 0, 2, 1), config(1 << 17, 1e-3, 10, 20, 4, 1),
+                                     config(1 << 16, 2e-3, 4, 0, 8, 4), config(1 << 18, 5e-4, 6, 20, 2, 1)};
     std::vector<std::vector<float>> spectra;
     std::vector<std::vector<PzlCand>> ref;
     std::vector<void *> dev;
@@ -101,7 +109,10 @@ int main(int argc, char **argv)
     const Opt opts[] = {{96, 0, 16, 1}, {64, 64, 1 << 20, 1}, {96, 0, 64, 0}, {0, 0, 16, 1}, {96, 0, 1 << 20, 1}};
     for (size_t s = 0; s < shapes.size(); s++) {
         void *plan = nullptr;
-        if (pzl_plan_create(&shapes[s], 0, &plan) || pzl_set_spectrum(plan, spectra[s].data(), shapes[s].numbins)) {
+        PzlConfig c4 = shapes[s];
+        c4.batchsize = 4;
+        if (pzl_plan_create_launch(&c4, 0, 4, &plan) ||
+            pzl_set_spectrum(plan, spectra[s].data(), shapes[s].numbins)) {
             fprintf(stderr, "plan: %s\n", pzl_last_error());
             return 2;
         }

@@ -21,10 +21,12 @@ TOL_POW = 1e-5
 TOL_KERN = 2e-6
 
 
-def _plan(cfg_kwargs, fft):
+def _plan(cfg_kwargs, fft, launch=0):
+    """launch: exactly so many rsteps per launch (0: the plan's choice, which for
+    short searches is most of the search)."""
     from prestozl_amd import binding as B
     cfg = B.make_config(**cfg_kwargs)
-    plan = B.Plan(cfg)
+    plan = B.Plan(cfg, launch=launch)
     plan.set_spectrum(fft)
     return plan
 
@@ -199,10 +201,16 @@ def _compare_hits(plan, hits_gpu, pows_gpu, ohits, powcut):
     return near, worst, len(set(g) & set(o))
 
 
-def test_search_config1(config1_data):
-    """Full config-1 search (N=2^20, zmax 20, wmax 0, numharm 4, sigma 2)."""
+KSLOTS = 4  # batches in flight
+
+
+@pytest.mark.parametrize("launch", [0, 8])
+def test_search_config1(config1_data, launch):
+    """Full config-1 search (N=2^20, zmax 20, wmax 0, numharm 4, sigma 2), in the
+    plan's launches (two) and in launches of 8 rsteps."""
     fft, kw = _c1(config1_data)
-    plan = _plan(kw, fft)
+    plan = _plan(kw, fft, launch)
+    assert launch == 0 or plan.geom.nrsteps > 2 * KSLOTS * launch
     obs, ctx32 = _oracle(kw, O.FP32)
     cg, st = plan.search()
     hg, pg = plan.hits()
@@ -302,16 +310,24 @@ def test_search_config3_band():
 
 
 def test_batch_size_invariance(config1_data):
-    """Candidate list is independent of rsteps per launch (determinism)."""
+    """Candidates and hits are independent of rsteps per launch (determinism):
+    1, 3, 8, 11 (batches and a rest) and 60 of them, and the plan's choice, which
+    is none of these."""
     fft, kw = _c1(config1_data)
     res = []
-    for bs in (1, 3, 8):
-        kw["batchsize"] = bs
-        plan = _plan(kw, fft)
-        c, _ = plan.search(0, 60)
-        res.append(c)
+    for bs in (1, 3, 8, 11, 60, 0):
+        kw["batchsize"] = bs or 8
+        plan = _plan(kw, fft, bs)
+        assert plan.launch()[0] == bs or (bs == 0 and plan.launch()[0] > 60)
+        c, st = plan.search(0, 60)
+        assert st["corr_launches"] == (-(-60 // bs) if bs else 1)
+        res.append((c, plan.hits()))
         plan.close()
-    assert res[0] == res[1] == res[2]
+    c0, h0 = res[0]
+    assert len(c0) > 0
+    for c, h in res[1:]:
+        assert c == c0
+        assert all(np.array_equal(a, b) for a, b in zip(h, h0))
 
 
 @pytest.mark.parametrize("which", ["c1", "c2", "h32"])
@@ -383,29 +399,35 @@ def test_fractional_rlo_every_sum_form(config1_data):
     plan.close()
 
 
-def test_hit_overflow_rerun_identical(config1_data):
+@pytest.mark.parametrize("launch", [8, 40, 0])
+def test_hit_overflow_rerun_identical(config1_data, launch):
     """A batch whose hits overflow the hit slot is searched again one rstep at
-    a time (the slot always holds one rstep's cells x stages): candidates and
-    hits equal those of a plan whose slots hold whole batches.  Strong bins in
-    one band of the spectrum (every third bin, well above the noise median)
-    make nearly every cell there a hit."""
+    a time (the slot always holds one rstep's cells x stages), one raised above
+    the size asked for at that size: candidates and hits equal those of a plan
+    whose slots hold whole batches.  Strong bins in one band of the spectrum (every
+    third bin, well above the noise median) make nearly every cell there a hit.
+    In batches of 8 the band starts in the third of 12, with others in flight."""
     fft, kw = _c1(config1_data)
     fft = fft.copy()
     lo_bin, hi_bin = 12000, 19000
     fft[lo_bin:hi_bin:3] *= 40.0
-    lo, hi = 8, 24  # two batches of 8 rsteps over the band
-    p1 = _plan(kw, fft)
+    lo, hi = 0, 96
+    p1 = _plan(kw, fft, 8)
+    p1.set_keep_hits(1 << 24)
     c1, _ = p1.search(lo, hi)
     h1, w1 = p1.hits()
     kw2 = dict(kw, maxhits=1)  # slot = one rstep's cells x stages
-    p2 = _plan(kw2, fft)
+    p2 = _plan(kw2, fft, launch)
+    p2.set_keep_hits(1 << 24)
     c2, _ = p2.search(lo, hi)
     h2, w2 = p2.hits()
     g = p1.geom
     per_rstep = g.corr_uselen * p1.harms[0].numz * max(p1.harms[0].numw, 1) * g.numharmstages
     per_batch = np.bincount((h1[:, 0] - lo) // kw["batchsize"])
     print("hits %d, per batch %s, slot of the small plan %d" % (len(h1), per_batch.tolist(), per_rstep))
-    assert per_batch.max() > per_rstep  # the small plan's slot did overflow
+    assert per_batch.max() > per_rstep  # the small plan's slot did overflow ...
+    over = np.flatnonzero(per_batch > per_rstep)
+    assert 0 < over[0] and over[-1] < 96 // 8 - 1  # ... between batches that fitted
     assert c1 == c2
     i1, i2 = np.lexsort(h1.T[::-1]), np.lexsort(h2.T[::-1])
     assert np.array_equal(h1[i1], h2[i2]) and np.array_equal(w1[i1], w2[i2])
@@ -564,8 +586,9 @@ def test_graph_replay_identical(config1_data, which):
     """Batches replayed from captured graphs give the eager path's hits and
     candidates exactly."""
     fft, kw = _c1(config1_data) if which == "c1" else _c2_small()
-    plan = _plan(kw, fft)
+    plan = _plan(kw, fft, kw["batchsize"])
     lo, hi = (0, -1) if which == "c1" else (40, 80)  # more batches than hit slots: replays happen
+    assert (hi if hi > 0 else plan.geom.nrsteps) - lo > 2 * KSLOTS * plan.launch()[0]
     plan.set_graph(False)
     c_eager, _ = plan.search(lo, hi, stats=False)
     h_eager = plan.hits()
@@ -575,7 +598,7 @@ def test_graph_replay_identical(config1_data, which):
     c_again, _ = plan.search(lo, hi, stats=False)  # replay of the already captured graphs
     plan.close()
     print("graph launches %d, eager candidates %d" % (st["graph_launches"], len(c_eager)))
-    assert st["graph_launches"] > 0
+    assert st["graph_launches"] > KSLOTS
     assert c_graph == c_eager and c_again == c_eager
     assert np.array_equal(h_graph[1], h_eager[1])
     assert all(np.array_equal(a, b) for a, b in zip(h_graph[0], h_eager[0]))
@@ -587,8 +610,9 @@ def test_cu_split_identical(config1_data, which):
     every CU, or kept off the sums' own) give the whole chip's hits and
     candidates exactly, eager and replayed; invalid counts are refused."""
     fft, kw = _c1(config1_data) if which == "c1" else _c2_small()
-    plan = _plan(kw, fft)
+    plan = _plan(kw, fft, kw["batchsize"])
     lo, hi = (0, -1) if which == "c1" else (40, 80)
+    assert (hi if hi > 0 else plan.geom.nrsteps) - lo > 2 * KSLOTS * plan.launch()[0]
     assert plan.cu_split() == (0, 0)
     c0, _ = plan.search(lo, hi, stats=False)
     h0 = plan.hits()
@@ -617,7 +641,7 @@ def test_hit_chunks_identical(config1_data):
     jobs) give the default chunk's hits and candidates exactly; invalid sizes
     are refused."""
     fft, kw = _c1(config1_data)
-    plan = _plan(kw, fft)
+    plan = _plan(kw, fft, 8)
     c0, _ = plan.search(stats=False)
     h0 = plan.hits()
     assert len(h0[1]) > 1000

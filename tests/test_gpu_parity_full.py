@@ -26,9 +26,9 @@ pytestmark = pytest.mark.gpu
 NTHREADS = 16
 
 
-def _plan(kw, fft):
+def _plan(kw, fft, launch=0):
     from prestozl_amd import binding as B
-    plan = B.Plan(B.make_config(**kw))
+    plan = B.Plan(B.make_config(**kw), launch=launch)
     plan.set_spectrum(fft)
     plan.set_keep_hits(1 << 24)
     return plan
@@ -64,19 +64,21 @@ def config2_full():
 
 @pytest.mark.parametrize("inj", [0, 1, 2])
 def test_config2_full_length_bands(config2_full, inj):
-    """N = 2^24, sigma 5, batchsize 8: 8 rsteps centred on injection 'inj',
-    with every FFT length in one grouped launch (the lean group: the form the
-    autotuner keeps at this shape) for two of the bands and one launch per
-    length for the third."""
+    """N = 2^24, sigma 5, 8 rsteps per launch: 8 rsteps centred on injection
+    'inj', by width (the default form) in every band, then with every FFT length
+    of whole rows in one grouped launch (the lean group) for two of the bands and
+    one launch per length for the third."""
     from prestozl_amd import binding as B
     fft, kw, sigs = config2_full
-    plan = _plan(kw, fft)
-    if inj != 1:
-        lean = [g for g, name in enumerate(B.corr_groups()) if "lean" in name][0]
-        plan.set_corr_group(lean, True)
+    plan = _plan(kw, fft, 8)
+    groups = B.corr_groups()
+    assert plan.corr_group() == (len(groups) - 1, True) and groups[-1].startswith("rows by width")
+    lean = [g for g, name in enumerate(groups) if "lean" in name][0]
     obs, ctx = _oracle(kw)
     k = injection_rstep(obs, kw["N"], kw["dt"], sigs[inj])
     _check("config2 injection %d" % inj, plan, ctx, obs, fft, k - 4, k + 4, kw["sigma"])
+    plan.set_corr_group(*((lean, True) if inj != 1 else (-1, False)))
+    _check("config2 injection %d, whole rows" % inj, plan, ctx, obs, fft, k - 4, k + 4, kw["sigma"])
     ctx.close()
     plan.close()
 
