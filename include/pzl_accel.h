@@ -164,9 +164,8 @@ int pzl_search(void *plan, long long rstep_lo, long long rstep_hi, PzlCand *cand
 int pzl_plan_set_deadline(void *plan, double ms);
 
 /* Autotuner: times the harmonic-sum forms on one batch of the plan's own data
- * and the CU splits on a band of its search, and keeps the fastest, for this
- * plan and for later plans of the same shape on the device.  The correlation is
- * not timed: its rows-by-width launch (below) needs no choice.  report
+ * and the CU splits on a band of its search, and keeps the fastest for this
+ * plan.  The correlation is not timed: its rows-by-width launch (below) needs no choice.  report
  * (optional) receives one line per form.
  * Replaces the reference's per-shape cuFFT plan choice (accel_kernels.cu:96-158). */
 int pzl_autotune(void *plan, int reps, char *report, int report_len);

@@ -687,8 +687,9 @@ int drop_graphs(Plan &p)
 // batch's rsteps) is built once and replayed for every later full batch in
 // that set, after the batch's segments, which are launched as they are (ahead
 // on their own stream when overlapped, beside the previous batch's
-// correlation); the first batch of each set runs eagerly (it also builds what
-// the kernels read once per device).  The graph is built from the
+// correlation); the plan's first batch runs eagerly (it also builds what the
+// kernels read once per device), as does one for which that is missing after
+// the launch form changed.  The graph is built from the
 // recorded launches with hipGraphAddKernelNode, in launch order, each node
 // depending on the one before: no stream is captured, so HIP calls made
 // meanwhile by other threads are unaffected.  A graph the runtime refuses is

@@ -718,8 +718,8 @@ template <int N_, int NT_, int G_, bool PING, int SH, int PADSH, int... Rs> stru
         corr_units<N, NT, G, PING, SH, PADSH, Rs...>(a, u, a.total_items, sm);
     }
     // The variant's twiddles ([TWN][NT], see k_corr_twiddles), built on the
-    // current device on first use (never inside a stream capture: the first
-    // batch of every plan runs eagerly) and kept until the process ends.
+    // current device on first use (not while a batch is recorded for a graph:
+    // that is refused, and the batch launched) and kept until the process ends.
     static hipError_t table(hipStream_t st, const float2 **out)
     {
         static std::mutex mu;

@@ -170,10 +170,10 @@ struct Plan {
     bool has_deadline = false;
     std::chrono::steady_clock::time_point deadline{};
     hipStream_t sum_stream() const { return overlap_sum ? st3 : st; }
-    int side_group = -1;     // >= 0: the shorter FFT lengths in one grouped launch (autotuned) ...
+    int side_group = -1;     // >= 0: the shorter FFT lengths in one grouped launch ...
     bool group_all = false;  // ... and the longest length in it too: one correlation launch per batch
-    int sum_order = 0;  // harmonic-sum workgroup order (autotuned)
-    int sum_rpt = 1;    // harmonic-sum fundamental r per thread (autotuned)
+    int sum_order = 0;  // harmonic-sum workgroup order (by the work in a batch, or autotuned)
+    int sum_rpt = 1;    // harmonic-sum fundamental r per thread (likewise)
     // results of the last search
     std::vector<PzlHostHit> last_hits;
     std::vector<PzlCand> last_cands;

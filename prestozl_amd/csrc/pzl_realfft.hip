@@ -154,7 +154,8 @@ __device__ inline long long rf_group(int b, int nb)
 // which without it puts a wave's 64 stores of 8 bytes on 2 of the 64 banks.
 // With 1024 threads for every L and no padding, 564 series of 2^18 samples (512
 // by 256) took 720 + 598 us in the two kernels, with both 625 + 323; one series
-// of 2^24 (4096 by 2048) 90 + 62 us, now 76 + 46.  Both kernels read and write
+// of 2^24 (4096 by 2048) 90 + 62 us, with both 76 + 46 (63 + 45 with the column
+// kernel's twiddles stepped, too).  Both kernels read and write
 // each value once: 1.18 GB, 0.2 ms each at the memory's rate; what is left is
 // the vector unit and, for L >= 4096, rows of 32 bytes.
 template <int L>
@@ -341,8 +342,8 @@ __global__ __launch_bounds__(RfTile<L>::NT) void k_rf_cols(const float2 *__restr
     // A thread stays in its column, NT / C rows further each time: its twiddle is
     // the last one times exp(SIGN 2 pi i (NT / C) j2 / M), in double (at most 16
     // steps: 4e-15, far below the float it is rounded to).  Two gathers of 16
-    // bytes per element from tables that the L1 does not hold were half of this
-    // kernel's time (564 series of 2^18 samples, FFTs of 512: 625 us, now 475).
+    // bytes per element from tables that the L1 does not hold were a quarter of
+    // this kernel's time (564 series of 2^18 samples, FFTs of 512: 625 us, now 475).
     const unsigned c = tid & (C - 1), j2 = j2b + c, dk = NT >> lc;
     const double2 w0 = rf_twiddle<SIGN>(tid < total ? (tid >> lc) * j2 : 0, tlo, thi);  // places below M1 M2 = M
     const double2 dw = rf_twiddle<SIGN>(tid + NT < total ? dk * j2 : 0, tlo, thi);
