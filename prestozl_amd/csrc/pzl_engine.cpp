@@ -178,7 +178,7 @@ long long slot_hits(const PzlConfig &cfg, const PzlGeometry &g, int batch)
 // (13 and 19: 483 and 487, so sizes are doubled and not filled up to the limit).
 pzl::LaunchSizes launch_sizes(const PzlConfig &cfg, const PzlGeometry &g)
 {
-    LaunchSizes s;
+    LaunchSizes s{};
     s.asked = cfg.batchsize > 0 ? cfg.batchsize : kDefaultBatch;
     if (g.nrsteps > 0 && s.asked > g.nrsteps) s.asked = (int)g.nrsteps;
     if (s.asked < 1) s.asked = 1;
@@ -1069,8 +1069,15 @@ int pzl::launch_sizes_of(const PzlConfig &cfg, LaunchSizes *s)
     PzlGeometry g;
     std::vector<PzlHarm> harms;
     const int rc = compute_geometry(cfg, g, &harms, nullptr);
-    if (rc == 0) *s = launch_sizes(cfg, g);
-    return rc;
+    if (rc) return rc;
+    *s = launch_sizes(cfg, g);
+    PlanSizes z = plan_sizes(cfg, g, harms, s->asked);
+    s->asked_bytes = plan_device_bytes(g, z, harms, -1);
+    size_launch(z, cfg, g, s->small);
+    s->small_bytes = plan_device_bytes(g, z, harms, -1);
+    size_launch(z, cfg, g, s->large);
+    s->large_bytes = plan_device_bytes(g, z, harms, -1);
+    return 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -2025,9 +2032,11 @@ int pzl_tune_batchsize(const PzlConfig *cfg, int device, const float *host_fft, 
     for (int k = 0; k < ncand; k++) {
         PzlConfig c = *cfg;
         c.batchsize = candidates[k];
-        LaunchSizes ls;
-        int rc = launch_sizes_of(c, &ls);
+        PzlGeometry g;
+        std::vector<PzlHarm> harms;
+        int rc = compute_geometry(c, g, &harms, nullptr);
         if (rc) return rc;
+        const LaunchSizes ls = launch_sizes(c, g);
         // candidates whose plans launch alike are one
         if (timed.count(ls.large)) {
             if (ms_per_rstep) ms_per_rstep[k] = timed[ls.large];

@@ -183,40 +183,68 @@ bool compute_row_sets(const std::vector<PzlHarm> &harms, int corr_uselen, int (*
     sets->clear();
     rows->clear();
     long long bank_off = 0, seg_off = 0;
+    // the half-widths of the whole (z, w) grid, of which every harmonic has a part
+    // (a harmonic of 5000 rows has a few dozen different ones), and every held length
+    int zmax = 0, wmax = 0, longest = 0;
     for (const PzlHarm &H : harms) {
         if (!has(H.fftlen)) return false;
-        std::vector<int> lens;  // held lengths up to the harmonic's own
-        for (int n = 2; n <= H.fftlen; n += 2)
-            if (has(n)) lens.push_back(n);
+        zmax = std::max(zmax, H.zmax);
+        wmax = std::max(wmax, H.wmax);
+        longest = std::max(longest, H.fftlen);
+    }
+    const int gz = zmax / PZL_DZ * 2 + 1, gw = wmax / PZL_DW * 2 + 1;
+    std::vector<int> grid((size_t)gz * gw), held;
+    for (int k = 0; k < gw; k++)
+        for (int i = 0; i < gz; i++)
+            grid[(size_t)k * gz + i] = pzl_w_resp_halfwidth(-zmax + i * PZL_DZ, -wmax + k * PZL_DW);
+    for (int n = 2; n <= longest; n += 2)
+        if (has(n)) held.push_back(n);
+    std::vector<int> len_of;  // index in lens of each half-width's shortest length
+    std::vector<int> row_len, count, widest;
+    for (const PzlHarm &H : harms) {
+        // held lengths up to the harmonic's own
+        const std::vector<int> lens(held.begin(), std::upper_bound(held.begin(), held.end(), H.fftlen));
         // the widest window any start gives this harmonic (pzl_harm_r): its ends
         // round to half bins and then outwards to whole ones
         const double span = (corr_uselen / 2 - PZL_DR) * H.hf + 0.5;
         const int window = H.stage == 0 ? corr_uselen : std::max(H.max_numrs, 2 * ((int)floor(span + 1.0) + 1));
-        std::vector<std::vector<int>> by_len(lens.size());  // rows of each length
-        std::vector<int> widest(lens.size(), 0);
-        for (int row = 0; row < H.nrows; row++) {
-            const double z = -H.zmax + (row % H.numz) * PZL_DZ, w = -H.wmax + (row / H.numz) * PZL_DW;
-            const int khw = pzl_w_resp_halfwidth(z, w);
-            size_t k = lens.size() - 1;
-            if (khw <= H.halfwidth)
-                k = std::min<size_t>(k, std::lower_bound(lens.begin(), lens.end(), window + 4 * khw) - lens.begin());
-            by_len[k].push_back(row);
-            widest[k] = std::max(widest[k], khw);
+        const int last = (int)lens.size() - 1;
+        len_of.resize(H.halfwidth + 1);
+        for (int khw = 0, k = 0; khw <= H.halfwidth; khw++) {
+            while (k < last && lens[k] < window + 4 * khw) k++;
+            len_of[khw] = k;
         }
-        for (size_t k = lens.size(); k-- > 0;) {
-            if (by_len[k].empty()) continue;
+        row_len.resize(H.nrows);  // index in lens of each row, rows and widest row of each length
+        count.assign(lens.size(), 0);
+        widest.assign(lens.size(), 0);
+        int row = 0;
+        for (int wi = 0; wi < H.numw; wi++) {
+            const int *khws = &grid[(size_t)(wi + (wmax - H.wmax) / PZL_DW) * gz + (zmax - H.zmax) / PZL_DZ];
+            for (int zi = 0; zi < H.numz; zi++, row++) {
+                const int khw = khws[zi], k = khw <= H.halfwidth ? len_of[khw] : last;
+                row_len[row] = k;
+                count[k]++;
+                widest[k] = std::max(widest[k], khw);
+            }
+        }
+        int at = (int)rows->size();
+        rows->resize(rows->size() + H.nrows);
+        for (int k = last; k >= 0; k--) {
+            if (count[k] == 0) continue;
             PzlHarm S = H;
             S.fftlen = lens[k];
             // the full length keeps the harmonic's own segment, whatever its rows reach
             S.halfwidth = lens[k] == H.fftlen ? H.halfwidth : widest[k];
-            S.nrows = (int)by_len[k].size();
+            S.nrows = count[k];
             S.bank_off = bank_off;
             S.seg_off = seg_off;
             bank_off += (long long)S.nrows * S.fftlen;
             seg_off += S.fftlen / 2;
-            rows->insert(rows->end(), by_len[k].begin(), by_len[k].end());
             sets->push_back(S);
+            count[k] = at;  // where the length's rows go
+            at += S.nrows;
         }
+        for (row = 0; row < H.nrows; row++) (*rows)[count[row_len[row]]++] = row;
     }
     return true;
 }

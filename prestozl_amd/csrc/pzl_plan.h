@@ -49,6 +49,7 @@ struct LaunchSizes {
     int asked;  // as configured
     int small;  // raised while the planes are small
     int large;  // ... and, of these, while they are large
+    long long asked_bytes, small_bytes, large_bytes;  // device_bytes of their plans (launch_sizes_of)
 };
 int launch_sizes_of(const PzlConfig &cfg, LaunchSizes *s);
 

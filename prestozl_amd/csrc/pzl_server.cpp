@@ -308,15 +308,14 @@ static int submit(void *srv, const PzlConfig *cfg, const float *fft, bool on_dev
     // Raised rsteps per launch as far as the budget allows: with large planes a
     // request stays within its share, so that as many run at once as at the size
     // asked for; with small ones (at most 1.5 GiB more) within the budget.
-    PzlGeometry g;
-    int launch = 0;
-    for (int n : {ls.large, ls.small, ls.asked}) {
-        if (n == launch) continue;
-        launch = n;
-        rc = pzl_geometry_launch(cfg, n, &g);
-        if (rc) return rc;
-        const long long need = g.device_bytes + PZL_RUNTIME_BYTES_PER_SEARCH;
-        if (need <= (n > ls.small ? s->budget / s->max_inflight : s->budget)) break;
+    int launch = ls.asked;
+    long long need = ls.asked_bytes + PZL_RUNTIME_BYTES_PER_SEARCH;
+    if (ls.large > ls.small && ls.large_bytes + PZL_RUNTIME_BYTES_PER_SEARCH <= s->budget / s->max_inflight) {
+        launch = ls.large;
+        need = ls.large_bytes + PZL_RUNTIME_BYTES_PER_SEARCH;
+    } else if (ls.small_bytes + PZL_RUNTIME_BYTES_PER_SEARCH <= s->budget) {
+        launch = ls.small;
+        need = ls.small_bytes + PZL_RUNTIME_BYTES_PER_SEARCH;
     }
     auto r = std::make_shared<Request>();
     r->cfg = *cfg;
@@ -326,7 +325,7 @@ static int submit(void *srv, const PzlConfig *cfg, const float *fft, bool on_dev
     // plan buffers, resident spectrum and kernel bank (counted per request,
     // although requests of one shape share a cached bank), and the runtime's
     // memory behind the plan's streams
-    r->footprint = g.device_bytes + PZL_RUNTIME_BYTES_PER_SEARCH;
+    r->footprint = need;
     r->launch = launch;
     r->asked = ls.asked;
     r->t_submit = Clock::now();

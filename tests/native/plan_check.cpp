@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -11,6 +12,9 @@
 #include <vector>
 
 #include "pzl_accel.h"
+#include "pzl_geom.h"
+#include "pzl_math.h"
+#include "pzl_plan.h"
 
 namespace {
 
@@ -386,6 +390,69 @@ void pinned()
     pzl_server_destroy(srv);
 }
 
+// Rows by width: every row at the shortest length that holds its window and its own
+// width, row by row.
+void row_sets()
+{
+    static const int menu[] = {128,  192,  256,  320,  384,  512,  640,  768,  1024,
+                               1152, 1280, 1536, 1792, 2048, 2560, 3072, 3584, 4096};
+    auto menu_has = [](int n) { return (int)std::binary_search(std::begin(menu), std::end(menu), n); };
+    auto even_has = [](int n) { return (int)(n >= 8 && n <= 4096 && n % 2 == 0); };
+    auto powers_has = [](int n) { return (int)(n >= 64 && n <= 4096 && (n & (n - 1)) == 0); };
+    using Has = int (*)(int);
+    const struct {
+        int zmax, wmax, numharm;
+    } shapes[] = {{0, 0, 1}, {0, 0, 32}, {4, 0, 32}, {2, 20, 4}, {51, 0, 8}, {0, 300, 16}, {20, 500, 8},
+                  {200, 300, 16}, {200, 500, 32}, {37, 133, 16}, {600, 0, 4}};
+    for (auto &sh : shapes)
+        for (Has has : {Has(menu_has), Has(even_has), Has(powers_has)}) {
+            const PzlConfig c = config(1 << 17, sh.zmax, sh.wmax, sh.numharm, 8);
+            PzlGeometry g;
+            std::vector<PzlHarm> harms, sets;
+            std::vector<int> rows;
+            ok(pzl::compute_geometry(c, g, &harms, nullptr));
+            bool held = true;
+            for (auto &H : harms) held = held && has(H.fftlen);
+            EXPECT(pzl::compute_row_sets(harms, g.corr_uselen, has, &sets, &rows) == held, "(%d, %d)", sh.zmax, sh.wmax);
+            if (!held) continue;
+            size_t k = 0, at = 0;
+            long long bank = 0, seg = 0;
+            for (auto &H : harms) {
+                std::vector<int> len(H.nrows), khw(H.nrows);
+                for (int r = 0; r < H.nrows; r++) {
+                    khw[r] = pzl_w_resp_halfwidth(-H.zmax + 2 * (r % H.numz), -H.wmax + 20 * (r / H.numz));
+                    const double span = (g.corr_uselen / 2 - 0.5) * H.hf + 0.5;
+                    const int window =
+                        H.stage == 0 ? g.corr_uselen : std::max(H.max_numrs, 2 * ((int)floor(span + 1.0) + 1));
+                    len[r] = H.fftlen;
+                    for (int n = H.fftlen; n >= 2 && khw[r] <= H.halfwidth; n--)
+                        if (has(n) && n >= window + 4 * khw[r]) len[r] = n;
+                }
+                for (int n = H.fftlen; n >= 2; n--) {
+                    std::vector<int> want;
+                    int widest = 0;
+                    for (int r = 0; r < H.nrows; r++)
+                        if (len[r] == n) {
+                            want.push_back(r);
+                            widest = std::max(widest, khw[r]);
+                        }
+                    if (want.empty()) continue;
+                    EXPECT(k < sets.size(), "(%d, %d)", sh.zmax, sh.wmax);
+                    if (k >= sets.size()) return;
+                    const PzlHarm &S = sets[k++];
+                    EXPECT(S.fftlen == n && S.nrows == (int)want.size() && S.bank_off == bank && S.seg_off == seg &&
+                               S.halfwidth == (n == H.fftlen ? H.halfwidth : widest) && S.parent == H.parent &&
+                               std::equal(want.begin(), want.end(), rows.begin() + (long)at),
+                           "(%d, %d) harmonic %d/%d, %d points", sh.zmax, sh.wmax, H.harmnum, H.numharm, n);
+                    at += want.size();
+                    bank += (long long)want.size() * n;
+                    seg += n / 2;
+                }
+            }
+            EXPECT(k == sets.size() && at == rows.size(), "(%d, %d)", sh.zmax, sh.wmax);
+        }
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
@@ -399,6 +466,7 @@ int main(int argc, char **argv)
     else if (name == "deadline") deadline();
     else if (name == "tuner") tuner();
     else if (name == "pinned") pinned();
+    else if (name == "row_sets") row_sets();
     else {
         fprintf(stderr, "no check '%s'\n", name.c_str());
         return 2;

@@ -24,7 +24,8 @@ def exe(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("check", ["exact", "rule", "memory", "server", "overflow", "deadline", "tuner", "pinned"])
+@pytest.mark.parametrize("check", ["exact", "rule", "memory", "server", "overflow", "deadline", "tuner", "pinned",
+                                   "row_sets"])
 def test_plan(exe, check):
     r = subprocess.run([exe, check], capture_output=True, text=True, timeout=300)
     print(r.stdout[-3000:], r.stderr[-3000:])
