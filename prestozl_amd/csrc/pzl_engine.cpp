@@ -172,10 +172,12 @@ long long slot_hits(const PzlConfig &cfg, const PzlGeometry &g, int batch)
 // large, as each kernel row is read once per batch; not where fewer than the
 // default of 8 are asked for, which bounds the plan's memory.  One rstep per launch
 // stays one.  A slot, sized for the rsteps asked for, holds a hit in one of 64 of a
-// launch's cells and stages at least.  Measured on MI355X, ms per search: 540 rsteps of 0.3 MiB: 8 per
-// launch 5.64, 270 0.54, 512 0.46; 1117 of 1.2 MiB: 8 8.9, 128 1.52, 256 1.46, 512
-// 1.46; 182 of 88 MiB: 8 12.7, 16 11.7, 32 11.1; 2920 of 157 MiB: 8 532, 16 462
-// (13 and 19: 483 and 487, so sizes are doubled and not filled up to the limit).
+// launch's cells and stages at least.  Measured on MI355X, ms per search:
+//   540 rsteps of 0.3 MiB: 8 per launch 5.64, 270 0.54, 512 0.46;
+//   1117 of 1.2 MiB: 8 8.9, 128 1.52, 256 1.46, 512 1.46;
+//   182 of 88 MiB: 8 12.7, 16 11.7, 32 11.1;
+//   2920 of 157 MiB, with many hits: 8 532, 16 462 (13 and 19: 483 and 487, so
+//   sizes are doubled and not filled up to the limit).
 pzl::LaunchSizes launch_sizes(const PzlConfig &cfg, const PzlGeometry &g)
 {
     LaunchSizes s{};

@@ -424,11 +424,12 @@ void row_sets()
                     const double span = (g.corr_uselen / 2 - 0.5) * H.hf + 0.5;
                     const int window =
                         H.stage == 0 ? g.corr_uselen : std::max(H.max_numrs, 2 * ((int)floor(span + 1.0) + 1));
-                    len[r] = H.fftlen;
-                    for (int n = H.fftlen; n >= 2 && khw[r] <= H.halfwidth; n--)
-                        if (has(n) && n >= window + 4 * khw[r]) len[r] = n;
+                    len[r] = window + 4 * khw[r];
+                    while (len[r] < H.fftlen && !has(len[r])) len[r]++;
+                    if (len[r] > H.fftlen || khw[r] > H.halfwidth) len[r] = H.fftlen;
                 }
                 for (int n = H.fftlen; n >= 2; n--) {
+                    if (std::find(len.begin(), len.end(), n) == len.end()) continue;
                     std::vector<int> want;
                     int widest = 0;
                     for (int r = 0; r < H.nrows; r++)
@@ -436,7 +437,6 @@ void row_sets()
                             want.push_back(r);
                             widest = std::max(widest, khw[r]);
                         }
-                    if (want.empty()) continue;
                     EXPECT(k < sets.size(), "(%d, %d)", sh.zmax, sh.wmax);
                     if (k >= sets.size()) return;
                     const PzlHarm &S = sets[k++];
