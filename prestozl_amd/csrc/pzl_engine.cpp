@@ -122,7 +122,7 @@ int acquire_bank(Plan *p, bool width, bool *built)
     evict_banks_locked(e.bytes);
     PZL_HIPCHK(hipMalloc(&e.ptr, e.bytes));
     hipError_t err = pzl_launch_bank_build(width ? p->d_sets : p->d_harms, (int)(width ? p->sets : p->harms).size(),
-                                           p->g.numharm_kernels, p->max_fftlen, e.ptr, 0, p->st);
+                                           p->g.numharm_kernels, p->max_fftlen, e.ptr, p->st);
     if (err == hipSuccess) err = hipStreamSynchronize(p->st);
     if (err != hipSuccess) {
         (void)hipFree(e.ptr);
@@ -1690,9 +1690,9 @@ int pzl_search(void *plan, long long rstep_lo, long long rstep_hi, PzlCand *cand
         const bool grouped = width || (p->side_group >= 0 && p->classes.size() > 1);
         long long per_batch = 1;  // grouped launches
         if (width) {
-            std::vector<int> lens;
-            for (auto &c : p->set_classes) lens.push_back(c.fftlen);
-            per_batch = pzl_corr_group_launches(p->side_group, (int)lens.size(), lens.data());
+            long long nlong = 0;
+            for (auto &c : p->set_classes) nlong += c.fftlen > PZL_CORR_LONG;
+            per_batch = (nlong > 0) + (nlong < (long long)p->set_classes.size());
         }
         stats->group_launches = grouped ? i * per_batch : 0;
         stats->corr_launches =
@@ -2222,9 +2222,10 @@ int pzl_get_kernel(void *plan, int idx, int row, float *out)
     PZL_HIPCHK(hipMalloc(&d, head + sizeof(float2) * n));
     one.H.nrows = 1;
     one.H.bank_off = 0;
+    one.H.unit = 1;
     one.H.rowlist = (const int *)(d + offsetof(One, row));
     hipError_t e = hipMemcpy(d, &one, sizeof one, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = pzl_launch_bank_build((const PzlHarm *)d, 1, 1, n, (float2 *)(d + head), 1, p->st);
+    if (e == hipSuccess) e = pzl_launch_bank_build((const PzlHarm *)d, 1, 1, n, (float2 *)(d + head), p->st);
     if (e == hipSuccess) e = hipStreamSynchronize(p->st);
     if (e == hipSuccess) e = hipMemcpy(out, d + head, sizeof(float2) * n, hipMemcpyDeviceToHost);
     (void)hipFree(d);

@@ -81,4 +81,5 @@ struct PzlHarm {
     int parent;                   // the harmonic's index (its own index where this is no row set)
     int ref_fftlen, ref_halfwidth;  // the harmonic's fftlen and halfwidth: its median window
     const int *rowlist;           // device: row of the harmonic of each row of the set; null: all, in order
+    int unit;                     // 1: kernel rows built as they are, without a bank's 1 / fftlen
 };

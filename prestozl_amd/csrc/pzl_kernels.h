@@ -98,10 +98,8 @@ struct PzlSumArgs {
 #ifdef __cplusplus
 extern "C" {
 #endif
-// The kernel rows of nh harmonics: K / fftlen, as the correlations read them, or
-// (unit) K itself.
 hipError_t pzl_launch_bank_build(const PzlHarm *d_harms, int nh, int total_rows, int max_fftlen, float2 *d_bank,
-                                 int unit, hipStream_t st);
+                                 hipStream_t st);
 hipError_t pzl_launch_segments(const PzlBatchArgs *a, int max_fftlen, hipStream_t st);
 // Correlation of one FFT-length class with variant 'variant' (0 = default);
 // class_nrows: host copy of the kernel-row counts of the class's harmonics.
@@ -111,11 +109,11 @@ const char *pzl_corr_variant_name(int n, int v);
 // Correlation of several FFT-length classes in one launch of group 'group':
 // class c has length fftlens[c], arguments *args[c] and host row counts
 // class_nrows[c]; a length the group does not hold, or one given twice, is an
-// error.  The last group holds closely spaced lengths, for classes of row sets.
+// error.  The last group holds closely spaced lengths, for classes of row sets; its
+// lengths above PZL_CORR_LONG have a launch of their own.
+#define PZL_CORR_LONG 2048
 hipError_t pzl_launch_corr_group(int group, int ncls, const int *fftlens, const PzlCorrArgs *const *args,
                                  const int *const *class_nrows, hipStream_t st);
-// How many kernels that launch is (the last group's lengths above 2048 have their own).
-int pzl_corr_group_launches(int group, int ncls, const int *fftlens);
 int pzl_corr_num_groups(void);
 const char *pzl_corr_group_name(int group);
 int pzl_corr_group_has(int group, int n);

@@ -47,10 +47,9 @@ __device__ static int find_harm(const PzlHarm *harms, int nh, int row_global, in
     return -1;
 }
 
-// One workgroup per (harmonic, z, w) kernel.  unit: as they are, without the
-// searches' scale.
+// One workgroup per (harmonic, z, w) kernel.
 __global__ __launch_bounds__(BANK_NT) void k_bank_build(const PzlHarm *__restrict__ harms, int nh,
-                                                        float2 *__restrict__ bank, int unit)
+                                                        float2 *__restrict__ bank)
 {
     extern __shared__ double2 sbuf[];  // fftlen complex doubles
     const int tid = threadIdx.x;
@@ -84,7 +83,7 @@ __global__ __launch_bounds__(BANK_NT) void k_bank_build(const PzlHarm *__restric
     // The bank holds K / fftlen (scaled in double, rounded once): the
     // correlation's 1 / fftlen^2 power normalisation then comes out of the
     // product.
-    const double bscale = unit ? 1.0 : 1.0 / fftlen;
+    const double bscale = H.unit ? 1.0 : 1.0 / fftlen;
     float2 *out = bank + H.bank_off + (long long)row * fftlen;
     for (int k = tid; k < fftlen; k += BANK_NT)
         out[k] = float2{(float)(sbuf[k].x * bscale), (float)(sbuf[k].y * bscale)};
@@ -1218,10 +1217,10 @@ extern "C" hipError_t pzl_launch_hitprep(const long long *keys, const float *pow
 }
 
 extern "C" hipError_t pzl_launch_bank_build(const PzlHarm *d_harms, int nh, int total_rows, int max_fftlen,
-                                            float2 *d_bank, int unit, hipStream_t st)
+                                            float2 *d_bank, hipStream_t st)
 {
     const size_t smem = (size_t)max_fftlen * sizeof(double2);
-    hipLaunchKernelGGL(k_bank_build, dim3(total_rows), dim3(BANK_NT), smem, st, d_harms, nh, d_bank, unit);
+    hipLaunchKernelGGL(k_bank_build, dim3(total_rows), dim3(BANK_NT), smem, st, d_harms, nh, d_bank);
     return hipGetLastError();
 }
 
@@ -1395,6 +1394,10 @@ using CorrGroupWidthLong =
     CorrGroup<512, 4, CorrV<4096, 512, 1, true, 0, 5, 8, 8, 8, 8>, CorrV<3584, 512, 1, true, 0, 5, 8, 8, 8, 7>,
               CorrV<3072, 512, 1, true, 0, 5, 8, 8, 6, 8>, CorrV<2560, 512, 1, true, 0, 5, 8, 8, 5, 8>>;
 
+static_assert(CorrGroupWidth::lens[0] <= PZL_CORR_LONG &&
+                  CorrGroupWidthLong::lens[CorrGroupWidthLong::M - 1] > PZL_CORR_LONG,
+              "longest first, apart at PZL_CORR_LONG");
+
 static int width_group_has(int n) { return CorrGroupWidth::has(n) || CorrGroupWidthLong::has(n); }
 
 static hipError_t width_group_launch(int ncls, const int *fftlens, const PzlCorrArgs *const *args,
@@ -1405,7 +1408,7 @@ static hipError_t width_group_launch(int ncls, const int *fftlens, const PzlCorr
         std::vector<const PzlCorrArgs *> a;
         std::vector<const int *> rows;
         for (int c = 0; c < ncls; c++)
-            if ((CorrGroupWidthLong::has(fftlens[c]) != 0) == (pass == 0)) {
+            if ((fftlens[c] > PZL_CORR_LONG) == (pass == 0)) {
                 lens.push_back(fftlens[c]);
                 a.push_back(args[c]);
                 rows.push_back(class_nrows[c]);
@@ -1417,13 +1420,6 @@ static hipError_t width_group_launch(int ncls, const int *fftlens, const PzlCorr
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
-}
-
-static int width_group_launches(int ncls, const int *fftlens)
-{
-    int n = 0;
-    for (int c = 0; c < ncls; c++) n += CorrGroupWidthLong::has(fftlens[c]) != 0;
-    return (n > 0) + (n < ncls);
 }
 
 struct CorrGroupEntry {
@@ -1444,10 +1440,6 @@ static const int g_ncorr_groups = (int)(sizeof(g_corr_groups) / sizeof(g_corr_gr
 
 extern "C" int pzl_corr_num_groups(void) { return g_ncorr_groups; }
 
-extern "C" int pzl_corr_group_launches(int group, int ncls, const int *fftlens)
-{
-    return group == g_ncorr_groups - 1 ? width_group_launches(ncls, fftlens) : 1;
-}
 
 extern "C" const char *pzl_corr_group_name(int group)
 {
